@@ -831,8 +831,8 @@ __global__ void k_lateral_bc(Dims d, AsmDev in, LatDev L, double* __restrict__ b
 }
 
 // basal_sliding_bc_3d, local option: diagonal of the basal level
-// (:8921-8953), owned rows.
-__global__ void k_basal_local(Dims d, AsmDev in, double* __restrict__ A) {
+// (:8921-8953), owned rows; the added term per vertex also to bd, when given.
+__global__ void k_basal_local(Dims d, AsmDev in, double* __restrict__ A, double* __restrict__ bd) {
     const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
     if (t >= (long long)d.nxo * d.nyo) return;
     const int io = (int)(t % d.nxo), jo = (int)(t / d.nxo);
@@ -844,6 +844,7 @@ __global__ void k_basal_local(Dims d, AsmDev in, double* __restrict__ A) {
     const double add = in.dx * in.dy / 1.0e9 * in.beta[p] / cos(in.theta[p]);
     a[(0 * 27 + 13) * WAVE] = a[(0 * 27 + 13) * WAVE] + add;
     a[(3 * 27 + 13) * WAVE] = a[(3 * 27 + 13) * WAVE] + add;
+    if (bd) bd[p] = add;
 }
 
 // dirichlet_boundary_conditions_3d restated per owned row P: the row of a

@@ -19,6 +19,7 @@
 #include "assembly.hip"
 #include "assembly2d.hip"
 #include "spmv_sym.hip"
+#include "spmv_elem.hip"
 #include "ensemble.hip"
 #include "noalloc.hip"
 #include "reprosum.hip"
@@ -78,6 +79,9 @@ struct cismgpu_system {
     double* efvs = nullptr;
     double* Atmp = nullptr;      // second matrix buffer for the symmetry fix (only when a pair differs)
     double* elemq = nullptr;     // element-once assembly: inverse Jacobian and f per element and point
+    double* elem_bd = nullptr;   // basal friction term of the diagonal per vertex (element-form product)
+    bool elem_ok = false;        // A64 equals the element form of asm_in, elemq and elem_bd
+    bool elem_use = false;       // the running FP64 solve takes its products in element form
     bool raw_ready = false;      // stage holds the raw Auu/Avv of the current matrix
     bool saved_raw_ready = false;
     bool sym_exact = false;      // the assembled FP64 matrix is known to be exactly symmetric
@@ -165,6 +169,8 @@ Dims make_dims(const cismgpu_grid* g) {
 }
 
 inline int spmv_blocks(const Dims& d) { return (d.nxp / WAVE) * ((d.nyo + 3) / 4); }
+// workgroups, and so partial sums, of the FP64 solve's products
+inline int spmv64_parts(const cismgpu_system* S) { return S->elem_use ? elem_blocks(S->d) : spmv_blocks(S->d); }
 inline int col_blocks(const Dims& d) { return (int)nblocks((long long)d.nvx * d.nvy, 256); }
 
 template <typename TV>
@@ -217,7 +223,10 @@ void spmv(cismgpu_system* S, const TA* A, const TV* xu, const TV* xv, TV* yu, TV
     if (S->two_d)   // one level: only the kA = 0 plane of the rows is read
         k_spmv_plane<TA, TV, MODE><<<spmv_blocks(S->d), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part);
     else if constexpr (std::is_same<TA, double>::value) {
-        if (S->a64_sym && (const double*)A == S->A64)   // FP64 half (symmetric) storage
+        if (S->elem_use && MODE != 0)   // an assembled system in element form
+            k_spmv_elem<MODE == 0 ? 1 : MODE><<<elem_blocks(S->d), WAVE * EL_J, 0, S->s>>>(
+                S->d, S->asm_in, S->elemq, S->elem_bd, xu, xv, yu, yv, bu, bv, part);
+        else if (S->a64_sym && (const double*)A == S->A64)   // FP64 half (symmetric) storage
             k_spmv_sym64<MODE><<<spmv_blocks(S->d), 256, 0, S->s>>>(S->d, S->A64h, xu, xv, yu, yv, bu, bv, part);
         else
             k_spmv<TA, TV, MODE><<<spmv_blocks(S->d), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part);
@@ -510,7 +519,7 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
     TV *xu = v[0], *xv = v[1], *ru = v[2], *rv = v[3], *du = v[4], *dv = v[5], *qu = v[6], *qv = v[7];
     TV *zu = v[8], *zv = v[9], *Azu = v[10], *Azv = v[11];
     const TV* M = std::is_same<TV, double>::value ? (const TV*)S->M64 : (const TV*)S->M32;
-    const int nsp = spmv_blocks(d), ncb = col_blocks(d);
+    const int nsp = std::is_same<TV, double>::value ? spmv64_parts(S) : spmv_blocks(d), ncb = col_blocks(d);
     const long long nv = d.vlen * sizeof(TV);
     // reprosum: the global sums of the FP64 solve are exact integer-vector
     // sums (the fused compensated partials are then not used)
@@ -611,7 +620,7 @@ int std_solve(cismgpu_system* S, int precond, int ncheck, double tol, int maxite
     const Dims& d = S->d;
     double *xu = S->V(0), *xv = S->V(1), *bu = S->V(2), *bv = S->V(3), *ru = S->V(4), *rv = S->V(5);
     double *du = S->V(6), *dv = S->V(7), *qu = S->V(8), *qv = S->V(9), *zu = S->V(10), *zv = S->V(11);
-    const int nsp = spmv_blocks(d), ncb = col_blocks(d);
+    const int nsp = spmv64_parts(S), ncb = col_blocks(d);
     const long long nv = d.vlen * sizeof(double);
     int st = reset_scal(S);
     if (st) return st;
@@ -875,7 +884,7 @@ static int32_t system_create(const cismgpu_grid* grid, bool two_d, cismgpu_syste
     if ((e = hipStreamCreateWithFlags(&S->s, hipStreamNonBlocking)) != hipSuccess) return fail(e, "stream");
     const long long n2 = (long long)d.nvx * d.nvy;
     const long long na = d.nrows * NCOEF;
-    const int nparts = std::max(spmv_blocks(d), std::max(col_blocks(d), dot_blocks<double>(d))) + 8;
+    const int nparts = std::max(std::max(spmv_blocks(d), elem_blocks(d)), std::max(col_blocks(d), dot_blocks<double>(d))) + 8;
     if ((e = hipMalloc(&S->active, n2)) != hipSuccess) return fail(e, "active");
     if ((e = hipMalloc(&S->A64, na * sizeof(double))) != hipSuccess) return fail(e, "A64");
     if ((e = hipMalloc(&S->M64, 8 * d.vlen * sizeof(double))) != hipSuccess) return fail(e, "M64");
@@ -922,7 +931,7 @@ int32_t cismgpu_system_destroy(cismgpu_system* S) {
     for (void* p : {(void*)S->active, (void*)S->A64, (void*)S->A32, (void*)S->A16, (void*)S->stage, (void*)S->M64,
                     (void*)S->M32, (void*)S->v64, (void*)S->v32, (void*)S->partA, (void*)S->partB, (void*)S->scal,
                     (void*)S->tri.a, (void*)S->tri.a32, S->asm_buf, (void*)S->efvs, (void*)S->Atmp, (void*)S->saved, (void*)S->work, (void*)S->load3, (void*)S->A64h, (void*)S->diva_buf, (void*)S->efva2, (void*)S->rs_part, (void*)S->rs_bad,
-                    (void*)S->rs_out, (void*)S->elemq, S->cb_buf})
+                    (void*)S->rs_out, (void*)S->elemq, (void*)S->elem_bd, S->cb_buf})
         if (p) hipFree(p);
     if (S->scal_h) hipHostFree(S->scal_h);
     for (auto& x : S->ev) hipEventDestroy(x);
@@ -977,6 +986,7 @@ static int set_matrix_impl(cismgpu_system* S, const int32_t* active_vertex, int 
     S->raw_ready = true;
     S->sym_exact = false;
     S->edge_zero = false;
+    S->elem_ok = false;
     S->m32_ready = S->a32_ready = S->a16_ready = S->a64h_ready = false;
     S->a32_sym = S->a64_sym = false;
     S->tri.mode = 0;
@@ -1096,17 +1106,24 @@ int32_t cismgpu_system_solve(cismgpu_system* S, const cismgpu_solve_opts* o, cis
     // new matrix and cached until the next: the line-solve factors, the
     // exact-symmetry checks and the half-storage / low-precision copies
     {
-        const bool fresh = ((o->precond == 3 || o->precond == 4) && S->tri.mode != o->precond) || !S->a64h_ready ||
+        // FP64 products of an assembled system in element form
+        // (CISMGPU_SPMV_FULL=1 keeps the full rows)
+        const char* full = getenv("CISMGPU_SPMV_FULL");
+        S->elem_use = S->elem_ok && o->precision == CISMGPU_FP64 && !(full && full[0] == '1');
+        const bool fresh = ((o->precond == 3 || o->precond == 4) && S->tri.mode != o->precond) ||
+                           (!S->elem_use && !S->a64h_ready) ||
                            (o->precision == CISMGPU_MIXED_FP32 && !S->a32_ready) ||
                            (o->precision == CISMGPU_MIXED_BF16 && !S->a16_ready) ||
                            (o->precision != CISMGPU_FP64 && !S->m32_ready);
         const auto t0 = std::chrono::steady_clock::now();
         if ((o->precond == 3 || o->precond == 4) && S->tri.mode != o->precond) {
             st = setup_tri(S, o->precond);
+            if (st) { S->elem_use = false; return st; }
+        }
+        if (!S->elem_use) {
+            st = ensure_half64(S);
             if (st) return st;
         }
-        st = ensure_half64(S);
-        if (st) return st;
         if (o->precision != CISMGPU_FP64) {
             st = ensure_lowp(S, o->precision);
             if (st) return st;
@@ -1138,7 +1155,8 @@ int32_t cismgpu_system_solve(cismgpu_system* S, const cismgpu_solve_opts* o, cis
         }
         info->err = err;
         info->niters = nit;
-        info->spmv_kind = S->a64_sym ? 4 : 0;
+        info->spmv_kind = (S->elem_use || S->a64_sym) ? 4 : 0;
+        S->elem_use = false;
     } else {
         st = mixed_solve(S, o, info);
     }
@@ -1538,6 +1556,7 @@ extern "C" int32_t cismgpu_system_assemble_3d(cismgpu_system* S, const cismgpu_a
     hipEvent_t e0, e1, e2;
     hipEventCreate(&e0); hipEventCreate(&e1); hipEventCreate(&e2);
     { const int st_ = reset_scal(S); if (st_) return st_; }
+    S->elem_ok = false;
     const double* uv = S->V(0);
     const double* vv = S->V(1);
     // element-once assembly (CISMGPU_ASSEMBLY=gather: the per-row gather
@@ -1545,10 +1564,10 @@ extern "C" int32_t cismgpu_system_assemble_3d(cismgpu_system* S, const cismgpu_a
     const char* aenv = getenv("CISMGPU_ASSEMBLY");
     const bool gather = aenv && !strcmp(aenv, "gather");
     if (!gather && !S->elemq) CG_CHECK(hipMalloc(&S->elemq, (size_t)8 * EQ * nfl * sizeof(double)));
-    // counters: nnz, pairs left asymmetric by the fix, differing pairs
+    // counters: nnz, pairs left asymmetric by the fix, differing pairs, vertices off a rectilinear grid
     unsigned long long* cnt = nullptr;
-    CG_CHECK(hipMalloc(&cnt, 3 * sizeof(unsigned long long)));
-    CG_CHECK(hipMemsetAsync(cnt, 0, 3 * sizeof(unsigned long long), S->s));
+    CG_CHECK(hipMalloc(&cnt, 4 * sizeof(unsigned long long)));
+    CG_CHECK(hipMemsetAsync(cnt, 0, 4 * sizeof(unsigned long long), S->s));
     // The element-once rows are symmetric by construction between owned
     // nodes; with no pass after them that changes couplings inside the
     // owned region (Dirichlet rows and columns, standard basal quadrature)
@@ -1556,8 +1575,16 @@ extern "C" int32_t cismgpu_system_assemble_3d(cismgpu_system* S, const cismgpu_a
     // the other rows are counted as they are written (CISMGPU_SYMCHECK=full:
     // every row checked and counted).
     const char* senv = getenv("CISMGPU_SYMCHECK");
-    const bool rim_only = !gather && !(senv && !strcmp(senv, "full")) && !in->umask_dirichlet &&
-                          !in->vmask_dirichlet && !(has_beta(in) && a.beta_std);
+    const bool plain = !gather && !in->umask_dirichlet && !in->vmask_dirichlet && !(has_beta(in) && a.beta_std);
+    const bool rim_only = plain && !(senv && !strcmp(senv, "full"));
+    // The element form of the FP64 product holds for these rows as they are
+    // summed here, and stays equal to them when the symmetry check finds
+    // nothing to change (spmv_elem.hip).
+    const bool elem_form = plain && !S->repro;
+    if (elem_form) {
+        if (!S->elem_bd) CG_CHECK(hipMalloc(&S->elem_bd, n2 * sizeof(double)));
+        CG_CHECK(hipMemsetAsync(S->elem_bd, 0, n2 * sizeof(double), S->s));
+    }
     hipEventRecord(e0, S->s);
     if (gather) {
         k_assemble<<<nblocks(d.nrows, 64), 64, 0, S->s>>>(d, a, uv, vv, S->A64, S->scal + S_NAN);
@@ -1573,8 +1600,9 @@ extern "C" int32_t cismgpu_system_assemble_3d(cismgpu_system* S, const cismgpu_a
             k_basal_std<<<nblocks((long long)d.nxo * d.nyo, 128), 128, 0, S->s>>>(d, a, d.nz - 1, 1, a.beta, a.beta, S->A64,
                                                                                S->scal + S_NAN);
         else
-            k_basal_local<<<nblocks((long long)d.nxo * d.nyo, 256), 256, 0, S->s>>>(d, a, S->A64);
+            k_basal_local<<<nblocks((long long)d.nxo * d.nyo, 256), 256, 0, S->s>>>(d, a, S->A64, S->elem_bd);
     }
+    if (elem_form) k_rectilinear<<<nblocks(n2, 256), 256, 0, S->s>>>(d, a.xV, a.yV, cnt + 3);
     if (a.taud_std)
         k_load_gravity_std<<<nblocks(n2, 64), 64, 0, S->s>>>(d, a, S->V(2), S->V(3), S->scal + S_NAN);
     else
@@ -1619,7 +1647,7 @@ extern "C" int32_t cismgpu_system_assemble_3d(cismgpu_system* S, const cismgpu_a
     // the raw Auu/Avv of the line-solve preconditioners are built when first needed
     S->raw_ready = false;
     hipEventRecord(e2, S->s);
-    unsigned long long hc[2] = {0, 0};
+    unsigned long long hc[4] = {0, 0, 0, 0};
     CG_CHECK(hipMemcpyAsync(hc, cnt, sizeof(hc), hipMemcpyDeviceToHost, S->s));
     CG_CHECK(sync_scal(S) ? hipErrorUnknown : hipSuccess);
     hipFree(cnt);
@@ -1633,6 +1661,7 @@ extern "C" int32_t cismgpu_system_assemble_3d(cismgpu_system* S, const cismgpu_a
         info->assemble_ms = ms1;
         info->total_ms = ms2;
     }
+    S->elem_ok = elem_form && S->sym_exact && hc[3] == 0 && S->scal_h[S_NAN] == 0.0;
     S->have_matrix = true;
     S->m32_ready = S->a32_ready = S->a16_ready = S->a64h_ready = false;
     S->a32_sym = S->a64_sym = false;
@@ -1988,6 +2017,7 @@ extern "C" int32_t cismgpu_system_restore_assembly(cismgpu_system* S) {
     S->raw_ready = S->saved_raw_ready;
     S->sym_exact = false;
     S->edge_zero = false;
+    S->elem_ok = false;
     S->m32_ready = S->a32_ready = S->a16_ready = S->a64h_ready = false;
     S->a32_sym = S->a64_sym = false;
     S->tri.mode = 0;

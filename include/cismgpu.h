@@ -165,7 +165,8 @@ typedef struct cismgpu_solve_info {
     double  solve_ms;        /* device time of the solve (HIP events on the system stream) */
     double  spmv_ms;         /* summed duration of the timed SpMV launches */
     int32_t spmv_count;      /* number of timed SpMV launches */
-    int32_t spmv_kind;       /* storage of the dominant SpMV: 0 fp64, 1 fp32, 2 bf16, 3 fp32 half (symmetric), 4 fp64 half */
+    int32_t spmv_kind;       /* storage of the dominant SpMV: 0 fp64, 1 fp32, 2 bf16, 3 fp32 half (symmetric), 4 fp64
+                                symmetric (half storage, or the element form of an assembled system) */
     double  setup_ms;        /* host wall time of the per-assembly set-up this call did before solve_ms began
                                 (symmetry checks, half-storage and low-precision copies, line-solve
                                 factors); 0 when a previous solve of the same matrix did it */

@@ -1,0 +1,65 @@
+"""FP64 solves of an assembled system take their products in element form; the
+rows (CISMGPU_SPMV_FULL=1) are the reference.  Sides around the 63 x 7 vertex
+tile, two to seventeen levels, periodic and ice-free rims, floating ice.
+
+Bar: the iterates after 7 Chronopoulos-Gear (6 standard) iterations.  Each
+product of either form sums a few hundred terms, so it is off by some 1e-14 of
+sum |A| |x| at most, and the iterates add a handful of such errors: 1e-12."""
+import os
+
+import numpy as np
+import pytest
+
+from cism_amd import pcg, synthetic
+from cism_amd.velo import BPSolver
+
+pytestmark = pytest.mark.gpu
+
+PROBLEMS = {
+    "stream62": lambda: synthetic.ice_stream(62, nz=3, seed=1),
+    "stream63": lambda: synthetic.ice_stream(63, nz=11, seed=2),
+    "stream64": lambda: synthetic.ice_stream(64, nz=2, seed=3),
+    "stream128": lambda: synthetic.ice_stream(128, nz=5, seed=4),
+    "stream20": lambda: synthetic.ice_stream(20, nz=17, seed=5),
+    "ismip_c": lambda: synthetic.ismip_hom("c", n=40, nz=6),
+    "yield_stream": lambda: synthetic.yield_stress_stream("raymond"),
+    "marine": lambda: synthetic.marine_sheet(70, nz=7, seed=6),
+}
+
+
+def _iterate(prob, full, algo, bend=False):
+    os.environ["CISMGPU_SPMV_FULL"] = "1" if full else "0"
+    try:
+        s = BPSolver(prob)
+        if bend:                       # one vertex off the rectilinear grid: the rows are the only form
+            s.xV[s.grid.nvx // 2, s.grid.nvy // 2] += 1.0
+        s.assemble(prob.uvel, prob.vvel)
+        s.sys.zero_x()
+        r = s.sys.solve(algo=algo, precond=2, tolerance=0.0, maxiters=7 if algo == pcg.ALGO_CHRONGEAR else 6,
+                        raise_on_error=False)
+        x = np.stack(s.sys.get_x())
+        s.sys.close()
+        return r, x
+    finally:
+        os.environ.pop("CISMGPU_SPMV_FULL", None)
+
+
+@pytest.mark.parametrize("algo", [pcg.ALGO_CHRONGEAR, pcg.ALGO_STANDARD])
+@pytest.mark.parametrize("name", list(PROBLEMS))
+def test_element_form_matches_rows(require_gpu, name, algo):
+    prob = PROBLEMS[name]()
+    r1, x1 = _iterate(prob, True, algo)
+    r0, x0 = _iterate(prob, False, algo)
+    assert r1["spmv_kind"] == 0
+    rel = np.linalg.norm(x0 - x1) / np.linalg.norm(x1)
+    print(name, algo, f"rel {rel:.2e}, err {r0['err']:.6e} / {r1['err']:.6e}, same bits {np.array_equal(x0, x1)}")
+    assert np.linalg.norm(x1) > 0 and rel < 1e-12
+    assert r0["err"] == pytest.approx(r1["err"], rel=1e-10)
+
+
+def test_bent_grid_keeps_the_rows(require_gpu):
+    prob = PROBLEMS["stream63"]()
+    (_, x1), (_, x0) = _iterate(prob, True, pcg.ALGO_CHRONGEAR, True), _iterate(prob, False, pcg.ALGO_CHRONGEAR, True)
+    assert np.array_equal(x0, x1)
+    assert not np.array_equal(_iterate(prob, False, pcg.ALGO_CHRONGEAR)[1],
+                              _iterate(prob, True, pcg.ALGO_CHRONGEAR)[1])
