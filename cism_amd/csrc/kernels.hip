@@ -24,7 +24,10 @@ __device__ __forceinline__ int xcd_remap(int lin, int nblk) {
 }
 
 // ---------------------------------------------------------------------------
-// SpMV: one thread per owned vertex column (io, jo); loop over levels.
+// SpMV: one thread per owned vertex column (io, jo); loop over the kper levels
+// of its share (blockIdx.y).  On small grids a workgroup that walks all the
+// levels leaves most CUs idle and pays a memory latency per level, so the
+// columns are split (level_split, libcismgpu.hip).
 // MODE 0: y = A x
 // MODE 1: y = A x, partial (y, x) over owned            (delta, eta2)
 // MODE 2: r = b - A x, partial (r, r) over owned        (convergence check)
@@ -36,7 +39,7 @@ __global__ __launch_bounds__(256) void k_spmv(Dims d, const TA* __restrict__ A,
                                               const TV* __restrict__ xu, const TV* __restrict__ xv,
                                               TV* __restrict__ yu, TV* __restrict__ yv,
                                               const TV* __restrict__ bu, const TV* __restrict__ bv,
-                                              double* __restrict__ partials) {
+                                              double* __restrict__ partials, int kper) {
     const int nbx = d.nxp / WAVE;
     const int nblk = nbx * ((d.nyo + 3) / 4);
     const int lin = xcd_remap(blockIdx.x, nblk);
@@ -44,13 +47,14 @@ __global__ __launch_bounds__(256) void k_spmv(Dims d, const TA* __restrict__ A,
     const int lane = threadIdx.x % WAVE;
     const int io = bx * WAVE + lane;
     const int jo = by * 4 + threadIdx.x / WAVE;
+    const int k0 = blockIdx.y * kper, k1 = min(d.nz, k0 + kper);
     const bool live = (io < d.nxo) && (jo < d.nyo);
     dd acc = {0.0, 0.0};
     if (live) {
         const int i = d.ilo + io, j = d.jlo + jo;
         const long long pl = d.plane;
         const int px = d.px;
-        for (int k = 0; k < d.nz; ++k) {
+        for (int k = k0; k < k1; ++k) {
             const long long r = ((long long)k * d.nyo + jo) * d.nxp + io;
             const TA* a = A + ((r / WAVE) * NCOEF) * WAVE + (r % WAVE);
             const long long c0 = vidx(d, k, i, j);
@@ -87,8 +91,8 @@ __global__ __launch_bounds__(256) void k_spmv(Dims d, const TA* __restrict__ A,
         dd v[1] = {acc};
         block_reduce_dd<1, 256>(v);
         if (threadIdx.x == 0) {
-            partials[2 * lin + 0] = v[0].hi;
-            partials[2 * lin + 1] = v[0].lo;
+            partials[2 * (blockIdx.y * nblk + lin) + 0] = v[0].hi;
+            partials[2 * (blockIdx.y * nblk + lin) + 1] = v[0].lo;
         }
     }
 }
@@ -119,9 +123,11 @@ template <typename TA, int MODE>
 __global__ __launch_bounds__(256) void k_spmv_q(Dims d, const TA* __restrict__ A, const float* __restrict__ xu,
                                                 const float* __restrict__ xv, float* __restrict__ yu,
                                                 float* __restrict__ yv, const float* __restrict__ bu,
-                                                const float* __restrict__ bv, double* __restrict__ partials) {
+                                                const float* __restrict__ bv, double* __restrict__ partials,
+                                                int kper) {
     const int nbx = d.nxp / WAVE;
     const int bx = blockIdx.x % nbx, by = blockIdx.x / nbx;
+    const int k0 = blockIdx.y * kper, k1 = min(d.nz, k0 + kper);
     const int lane = threadIdx.x % WAVE;
     const int io = bx * WAVE + lane;
     const int jo = by * 4 + threadIdx.x / WAVE;
@@ -136,11 +142,11 @@ __global__ __launch_bounds__(256) void k_spmv_q(Dims d, const TA* __restrict__ A
         for (int l = 0; l < 2; ++l)
 #pragma unroll
             for (int h = 0; h < 9; ++h) {
-                const long long n = cb + l * pl + (h / 3 - 1) * px + (h % 3 - 1);
+                const long long n = cb + (k0 + l) * pl + (h / 3 - 1) * px + (h % 3 - 1);
                 wu[l][h] = xu[n];
                 wv[l][h] = xv[n];
             }
-        for (int k = 0; k < d.nz; ++k) {
+        for (int k = k0; k < k1; ++k) {
             const long long cup = cb + (long long)(k + 2) * pl;
 #pragma unroll
             for (int h = 0; h < 9; ++h) {
@@ -183,8 +189,9 @@ __global__ __launch_bounds__(256) void k_spmv_q(Dims d, const TA* __restrict__ A
         dd v[1] = {{acc, 0.0}};
         block_reduce_dd<1, 256>(v);
         if (threadIdx.x == 0) {
-            partials[2 * blockIdx.x + 0] = v[0].hi;
-            partials[2 * blockIdx.x + 1] = v[0].lo;
+            const int lin = blockIdx.y * gridDim.x + blockIdx.x;
+            partials[2 * lin + 0] = v[0].hi;
+            partials[2 * lin + 1] = v[0].lo;
         }
     }
 }
@@ -952,21 +959,21 @@ __global__ void k_ir_update(Dims d, double* __restrict__ xu, double* __restrict_
 // ---------------------------------------------------------------------------
 #define INST_SPMV(TA, TV)                                                                                   \
     template __global__ void k_spmv<TA, TV, 0>(Dims, const TA*, const TV*, const TV*, TV*, TV*, const TV*,   \
-                                               const TV*, double*);                                        \
+                                               const TV*, double*, int);                                   \
     template __global__ void k_spmv<TA, TV, 1>(Dims, const TA*, const TV*, const TV*, TV*, TV*, const TV*,   \
-                                               const TV*, double*);                                        \
+                                               const TV*, double*, int);                                   \
     template __global__ void k_spmv<TA, TV, 2>(Dims, const TA*, const TV*, const TV*, TV*, TV*, const TV*,   \
-                                               const TV*, double*);
+                                               const TV*, double*, int);
 INST_SPMV(double, double)
 INST_SPMV(float, float)
 INST_SPMV(__hip_bfloat16, float)
 #define INST_SPMV_Q(TA)                                                                                      \
     template __global__ void k_spmv_q<TA, 0>(Dims, const TA*, const float*, const float*, float*, float*,     \
-                                             const float*, const float*, double*);                          \
+                                             const float*, const float*, double*, int);                     \
     template __global__ void k_spmv_q<TA, 1>(Dims, const TA*, const float*, const float*, float*, float*,     \
-                                             const float*, const float*, double*);                          \
+                                             const float*, const float*, double*, int);                     \
     template __global__ void k_spmv_q<TA, 2>(Dims, const TA*, const float*, const float*, float*, float*,     \
-                                             const float*, const float*, double*);
+                                             const float*, const float*, double*, int);
 INST_SPMV_Q(float)
 INST_SPMV_Q(__hip_bfloat16)
 #define INST_SPMV_PLANE(TA, TV)                                                                              \

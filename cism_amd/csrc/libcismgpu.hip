@@ -169,8 +169,22 @@ Dims make_dims(const cismgpu_grid* g) {
 }
 
 inline int spmv_blocks(const Dims& d) { return (d.nxp / WAVE) * ((d.nyo + 3) / 4); }
-// workgroups, and so partial sums, of the FP64 solve's products
-inline int spmv64_parts(const cismgpu_system* S) { return S->elem_use ? elem_blocks(S->d) : spmv_blocks(S->d); }
+// Levels per workgroup of the row products.  A workgroup that walks all nz
+// levels pays the latency of a level nz times; below 512 tiles (two per CU)
+// the levels are dealt to as many workgroups as fill the chip four deep.
+inline int level_split(const Dims& d) {
+    const int b = spmv_blocks(d);
+    if (b >= 512) return d.nz;
+    const int split = std::min(d.nz, (1024 + b - 1) / b);
+    return (d.nz + split - 1) / split;
+}
+inline int level_shares(const Dims& d) { return (d.nz + level_split(d) - 1) / level_split(d); }
+inline dim3 spmv_grid(const Dims& d) { return dim3(spmv_blocks(d), level_shares(d)); }
+// workgroups, and so partial sums, of the products
+inline int spmv_parts(const Dims& d) { return spmv_blocks(d) * level_shares(d); }
+inline int spmv64_parts(const cismgpu_system* S) {
+    return S->elem_use ? elem_parts(S->d) : S->two_d ? spmv_blocks(S->d) : spmv_parts(S->d);
+}
 inline int col_blocks(const Dims& d) { return (int)nblocks((long long)d.nvx * d.nvy, 256); }
 
 template <typename TV>
@@ -209,10 +223,12 @@ static bool use_symx() {
 template <int MODE>
 void spmv_sym32(cismgpu_system* S, const float* A, const float* xu, const float* xv, float* yu, float* yv,
                 const float* bu, const float* bv, double* part) {
-    if (use_symx())
+    // with the levels split there is no previous level to pass on
+    if (use_symx() && level_shares(S->d) == 1)
         k_spmv_symx<MODE><<<spmv_blocks(S->d), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part);
     else
-        k_spmv_sym<float, MODE><<<spmv_blocks(S->d), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part);
+        k_spmv_sym<float, MODE><<<spmv_grid(S->d), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part,
+                                                                   level_split(S->d));
 }
 
 template <typename TA, typename TV, int MODE>
@@ -224,18 +240,21 @@ void spmv(cismgpu_system* S, const TA* A, const TV* xu, const TV* xv, TV* yu, TV
         k_spmv_plane<TA, TV, MODE><<<spmv_blocks(S->d), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part);
     else if constexpr (std::is_same<TA, double>::value) {
         if (S->elem_use && MODE != 0)   // an assembled system in element form
-            k_spmv_elem<MODE == 0 ? 1 : MODE><<<elem_blocks(S->d), WAVE * EL_J, 0, S->s>>>(
-                S->d, S->asm_in, S->elemq, S->elem_bd, xu, xv, yu, yv, bu, bv, part);
+            k_spmv_elem<MODE == 0 ? 1 : MODE>
+                <<<dim3(elem_blocks(S->d), elem_parts(S->d) / elem_blocks(S->d)), WAVE * EL_J, 0, S->s>>>(
+                    S->d, S->asm_in, S->elemq, S->elem_bd, xu, xv, yu, yv, bu, bv, part, elem_split(S->d));
         else if (S->a64_sym && (const double*)A == S->A64)   // FP64 half (symmetric) storage
-            k_spmv_sym64<MODE><<<spmv_blocks(S->d), 256, 0, S->s>>>(S->d, S->A64h, xu, xv, yu, yv, bu, bv, part);
+            k_spmv_sym64<MODE><<<spmv_grid(S->d), 256, 0, S->s>>>(S->d, S->A64h, xu, xv, yu, yv, bu, bv, part,
+                                                                  level_split(S->d));
         else
-            k_spmv<TA, TV, MODE><<<spmv_blocks(S->d), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part);
+            k_spmv<TA, TV, MODE><<<spmv_grid(S->d), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part,
+                                                                    level_split(S->d));
     }
     else if (std::is_same<TA, float>::value && S->a32_sym)   // FP32 half (symmetric) storage
         spmv_sym32<MODE>(S, (const float*)A, (const float*)xu, (const float*)xv, (float*)yu, (float*)yv,
                          (const float*)bu, (const float*)bv, part);
     else   // FP32 / BF16 copies in the quad layout
-        k_spmv_q<TA, MODE><<<spmv_blocks(S->d), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part);
+        k_spmv_q<TA, MODE><<<spmv_grid(S->d), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part, level_split(S->d));
     if (t) { hipEventRecord(S->ev[S->ev_used + 1], S->s); S->ev_used += 2; }
 }
 
@@ -519,7 +538,7 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
     TV *xu = v[0], *xv = v[1], *ru = v[2], *rv = v[3], *du = v[4], *dv = v[5], *qu = v[6], *qv = v[7];
     TV *zu = v[8], *zv = v[9], *Azu = v[10], *Azv = v[11];
     const TV* M = std::is_same<TV, double>::value ? (const TV*)S->M64 : (const TV*)S->M32;
-    const int nsp = std::is_same<TV, double>::value ? spmv64_parts(S) : spmv_blocks(d), ncb = col_blocks(d);
+    const int nsp = std::is_same<TV, double>::value ? spmv64_parts(S) : S->two_d ? spmv_blocks(d) : spmv_parts(d), ncb = col_blocks(d);
     const long long nv = d.vlen * sizeof(TV);
     // reprosum: the global sums of the FP64 solve are exact integer-vector
     // sums (the fused compensated partials are then not used)
@@ -770,7 +789,7 @@ int mixed_solve(cismgpu_system* S, const cismgpu_solve_opts* o, cismgpu_solve_in
     if (st) return st;
     double *xu = S->V(0), *xv = S->V(1), *bu = S->V(2), *bv = S->V(3), *ru = S->V(4), *rv = S->V(5);
     float* w[12] = {S->W(0), S->W(1), S->W(4), S->W(5), S->W(6), S->W(7), S->W(8), S->W(9), S->W(10), S->W(11), S->W(12), S->W(13)};
-    const int nsp = spmv_blocks(d);
+    const int nsp = spmv64_parts(S);
     const long long nvf = d.vlen * sizeof(float);
     // ||b|| once
     st = reset_scal(S);
@@ -884,7 +903,7 @@ static int32_t system_create(const cismgpu_grid* grid, bool two_d, cismgpu_syste
     if ((e = hipStreamCreateWithFlags(&S->s, hipStreamNonBlocking)) != hipSuccess) return fail(e, "stream");
     const long long n2 = (long long)d.nvx * d.nvy;
     const long long na = d.nrows * NCOEF;
-    const int nparts = std::max(std::max(spmv_blocks(d), elem_blocks(d)), std::max(col_blocks(d), dot_blocks<double>(d))) + 8;
+    const int nparts = std::max(std::max(spmv_parts(d), elem_parts(d)), std::max(col_blocks(d), dot_blocks<double>(d))) + 8;
     if ((e = hipMalloc(&S->active, n2)) != hipSuccess) return fail(e, "active");
     if ((e = hipMalloc(&S->A64, na * sizeof(double))) != hipSuccess) return fail(e, "A64");
     if ((e = hipMalloc(&S->M64, 8 * d.vlen * sizeof(double))) != hipSuccess) return fail(e, "M64");
@@ -1218,15 +1237,15 @@ int32_t cismgpu_system_bench_spmv(cismgpu_system* S, int32_t kind, int32_t nrep,
             else
                 k_spmv_plane<__hip_bfloat16, float, 1><<<spmv_blocks(d), 256, 0, S->s>>>(d, S->A16, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB);
         } else if (kind == 0 && S->a64_sym)
-            k_spmv_sym64<1><<<spmv_blocks(d), 256, 0, S->s>>>(d, S->A64h, S->V(0), S->V(1), S->V(12), S->V(13), nullptr, nullptr, S->partB);
+            k_spmv_sym64<1><<<spmv_grid(d), 256, 0, S->s>>>(d, S->A64h, S->V(0), S->V(1), S->V(12), S->V(13), nullptr, nullptr, S->partB, level_split(d));
         else if (kind == 0)
-            k_spmv<double, double, 1><<<spmv_blocks(d), 256, 0, S->s>>>(d, S->A64, S->V(0), S->V(1), S->V(12), S->V(13), nullptr, nullptr, S->partB);
+            k_spmv<double, double, 1><<<spmv_grid(d), 256, 0, S->s>>>(d, S->A64, S->V(0), S->V(1), S->V(12), S->V(13), nullptr, nullptr, S->partB, level_split(d));
         else if (kind == 1 && S->a32_sym)
             spmv_sym32<1>(S, S->A32, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB);
         else if (kind == 1)
-            k_spmv_q<float, 1><<<spmv_blocks(d), 256, 0, S->s>>>(d, S->A32, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB);
+            k_spmv_q<float, 1><<<spmv_grid(d), 256, 0, S->s>>>(d, S->A32, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB, level_split(d));
         else
-            k_spmv_q<__hip_bfloat16, 1><<<spmv_blocks(d), 256, 0, S->s>>>(d, S->A16, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB);
+            k_spmv_q<__hip_bfloat16, 1><<<spmv_grid(d), 256, 0, S->s>>>(d, S->A16, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB, level_split(d));
     };
     launch();   // warm-up
     CG_CHECK(hipEventRecord(e0, S->s));
@@ -2349,14 +2368,15 @@ extern "C" int32_t cismgpu_system_residual(cismgpu_system* S, double* ru, double
     CG_CHECK(hipMemsetAsync(r0, 0, 2 * d.vlen * sizeof(double), S->s));
     { const int st_ = reset_scal(S); if (st_) return st_; }
     // r = b - A x over owned rows with partial (r,r); resid = -r on owned active rows
-    k_spmv<double, double, 2><<<spmv_blocks(d), 256, 0, S->s>>>(d, S->A64, S->V(0), S->V(1), r0, r1, S->V(2), S->V(3), S->partB);
+    k_spmv<double, double, 2><<<spmv_grid(d), 256, 0, S->s>>>(d, S->A64, S->V(0), S->V(1), r0, r1, S->V(2), S->V(3), S->partB,
+                                                              level_split(d));
     if (S->repro) {
         rs_dot<double>(S, 3, r0, r0, r1, r1);
         k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->rs_out + 6, 1, 2, nullptr, 0, 0, S->scal, 0.0);
         rs_dot<double>(S, 0, S->V(2), S->V(2), S->V(3), S->V(3));
         k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_BB, S->rs_out, 1, 2, nullptr, 0, 0, S->scal, 0.0);
     } else {
-        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->partB, spmv_blocks(d), 2, nullptr, 0, 0, S->scal, 0.0);
+        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->partB, spmv_parts(d), 2, nullptr, 0, 0, S->scal, 0.0);
         k_dot<double><<<dot_blocks<double>(d), 256, 0, S->s>>>(d, S->V(2), S->V(2), S->V(3), S->V(3), S->partA);
         k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_BB, S->partA, dot_blocks<double>(d), 2, nullptr, 0, 0, S->scal, 0.0);
     }

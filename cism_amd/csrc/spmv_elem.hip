@@ -37,6 +37,22 @@ constexpr int EL_J = 8;
 __host__ __device__ inline int elem_tiles_i(const Dims& d) { return (d.nxo + WAVE - 2) / (WAVE - 1); }
 __host__ __device__ inline int elem_blocks(const Dims& d) { return elem_tiles_i(d) * ((d.nyo + EL_J - 2) / (EL_J - 1)); }
 
+// Levels per workgroup.  A share of kper levels below the first redoes the
+// layer above it, and one workgroup fits a CU, so the time goes as rounds of
+// 256 workgroups times layers per workgroup; the smallest product wins (one
+// layer stands for the start of a workgroup).
+inline int elem_split(const Dims& d) {
+    int best = d.nz;
+    long long cost = -1;
+    for (int kper = d.nz; kper >= 1; --kper) {
+        const long long shares = (d.nz + kper - 1) / kper;
+        const long long c = (elem_blocks(d) * shares + 255) / 256 * (kper + (shares > 1 ? 2 : 1));
+        if (cost < 0 || c < cost) { cost = c; best = kper; }
+    }
+    return best;
+}
+inline int elem_parts(const Dims& d) { return elem_blocks(d) * ((d.nz + elem_split(d) - 1) / elem_split(d)); }
+
 // Counts the vertices whose x varies along j or whose y varies along i: the
 // element form needs none (x a function of i alone, y of j alone).
 __global__ void k_rectilinear(Dims d, const double* __restrict__ xV, const double* __restrict__ yV,
@@ -96,11 +112,12 @@ __global__ __launch_bounds__(WAVE * EL_J) void k_spmv_elem(Dims d, AsmDev in, co
                                                            const double* __restrict__ xu, const double* __restrict__ xv,
                                                            double* __restrict__ yu, double* __restrict__ yv,
                                                            const double* __restrict__ bu, const double* __restrict__ bv,
-                                                           double* __restrict__ partials) {
+                                                           double* __restrict__ partials, int kper) {
     __shared__ double ex[2][2][EL_J][WAVE];
     const int nti = elem_tiles_i(d), nblk = elem_blocks(d);
     const int lin = xcd_remap(blockIdx.x, nblk);
     const int bx = lin % nti, by = lin / nti;
+    const int k0 = blockIdx.y * kper, k1 = min(d.nz, k0 + kper);       // the levels of this share
     const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
     const int ci = d.ilo + bx * (WAVE - 1) + lane, cj = d.jlo + by * (EL_J - 1) + w;   // cell; its NE vertex is (ci, cj)
     const bool on = ci <= d.ihi + 1 && cj <= d.jhi + 1 && cell_in_range(d, in.nhalo, ci, cj) && in.acell[c2(d, ci, cj)];
@@ -176,14 +193,15 @@ __global__ __launch_bounds__(WAVE * EL_J) void k_spmv_elem(Dims d, AsmDev in, co
         }
     };
     PlaneQ Uu, Uv, Du, Dv;                              // upper level's values, and its duals so far
-    plane(0, Uu, Uv);
+    const int ks = max(k0 - 1, 0);
+    plane(ks, Uu, Uv);
 #pragma unroll
     for (int q = 0; q < 2; ++q) Du.x[q] = Du.y[q] = Dv.x[q] = Dv.y[q] = 0.0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) Du.v[q] = Dv.v[q] = 0.0;
     const double wa = 0.5 * (1.0 + g), wb = 0.5 * (1.0 - g);   // weights of the near and far level at a point
 #pragma unroll 1
-    for (int k = 0; k + 1 < d.nz; ++k) {                // element layer between levels k and k + 1
+    for (int k = ks; k < k1 && k + 1 < d.nz; ++k) {     // element layer between levels k and k + 1
         double f[8];
 #pragma unroll
         for (int p = 0; p < 8; ++p) f[p] = on ? F[(long long)p * EQ * ne + k * lay] : 0.0;
@@ -219,15 +237,15 @@ __global__ __launch_bounds__(WAVE * EL_J) void k_spmv_elem(Dims d, AsmDev in, co
             Du.v[q] += Gu; Eu.v[q] = -Gu;
             Dv.v[q] += Gv; Ev.v[q] = -Gv;
         }
-        finish(k, Du, Dv);
+        if (k >= k0) finish(k, Du, Dv);
         Du = Eu; Dv = Ev; Uu = Lu; Uv = Lv;
     }
-    finish(d.nz - 1, Du, Dv);
+    if (k1 == d.nz) finish(d.nz - 1, Du, Dv);
     dd v[1] = {acc};
     block_reduce_dd<1, WAVE * EL_J>(v);
     if (threadIdx.x == 0) {
-        partials[2 * lin + 0] = v[0].hi;
-        partials[2 * lin + 1] = v[0].lo;
+        partials[2 * (blockIdx.y * nblk + lin) + 0] = v[0].hi;
+        partials[2 * (blockIdx.y * nblk + lin) + 1] = v[0].lo;
     }
 }
 

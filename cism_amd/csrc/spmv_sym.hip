@@ -114,7 +114,9 @@ template <typename TA, int MODE>
 __global__ __launch_bounds__(256) void k_spmv_sym(Dims d, const TA* __restrict__ S, const float* __restrict__ xu,
                                                   const float* __restrict__ xv, float* __restrict__ yu,
                                                   float* __restrict__ yv, const float* __restrict__ bu,
-                                                  const float* __restrict__ bv, double* __restrict__ partials) {
+                                                  const float* __restrict__ bv, double* __restrict__ partials,
+                                                  int kper) {
+    const int k0 = blockIdx.y * kper, k1 = min(d.nz, k0 + kper);   // the levels of this share
     // x of the tile (64 x 4 columns) plus a one-column ring, for levels k-1,
     // k, k+1, staged in LDS (a 3-level ring)
     __shared__ float xs[2][3][6][WAVE + 2];
@@ -157,9 +159,9 @@ __global__ __launch_bounds__(256) void k_spmv_sym(Dims d, const TA* __restrict__
             po[h] = pc < 0 ? -1 : (pc / WAVE) * (NSLOT * 4 * WAVE) + (pc % WAVE) * 4;
         }
     }
-    stage(-1);
-    stage(0);
-    for (int k = 0; k < d.nz; ++k) {
+    stage(k0 - 1);
+    stage(k0);
+    for (int k = k0; k < k1; ++k) {
         stage(k + 1);
         __syncthreads();
         if (live) {
@@ -215,8 +217,8 @@ __global__ __launch_bounds__(256) void k_spmv_sym(Dims d, const TA* __restrict__
         dd v[1] = {{acc, 0.0}};
         block_reduce_dd<1, 256>(v);
         if (threadIdx.x == 0) {
-            partials[2 * lin + 0] = v[0].hi;
-            partials[2 * lin + 1] = v[0].lo;
+            partials[2 * (blockIdx.y * nblk + lin) + 0] = v[0].hi;
+            partials[2 * (blockIdx.y * nblk + lin) + 1] = v[0].lo;
         }
     }
 }
@@ -441,7 +443,8 @@ __global__ __launch_bounds__(256) void k_spmv_sym64(Dims d, const double* __rest
                                                     const double* __restrict__ xu, const double* __restrict__ xv,
                                                     double* __restrict__ yu, double* __restrict__ yv,
                                                     const double* __restrict__ bu, const double* __restrict__ bv,
-                                                    double* __restrict__ partials) {
+                                                    double* __restrict__ partials, int kper) {
+    const int k0 = blockIdx.y * kper, k1 = min(d.nz, k0 + kper);   // the levels of this share
     __shared__ double xs[2][3][6][WAVE + 2];
     const int nbx = d.nxp / WAVE;
     const int nblk = nbx * ((d.nyo + 3) / 4);
@@ -478,9 +481,9 @@ __global__ __launch_bounds__(256) void k_spmv_sym64(Dims d, const double* __rest
             po[h] = pc < 0 ? -1 : (pc / WAVE) * (NSLOT * 4 * WAVE) + (pc % WAVE) * 4;
         }
     }
-    stage(-1);
-    stage(0);
-    for (int k = 0; k < d.nz; ++k) {
+    stage(k0 - 1);
+    stage(k0);
+    for (int k = k0; k < k1; ++k) {
         stage(k + 1);
         __syncthreads();
         if (live) {
@@ -537,8 +540,8 @@ __global__ __launch_bounds__(256) void k_spmv_sym64(Dims d, const double* __rest
         dd v[1] = {acc};
         block_reduce_dd<1, 256>(v);
         if (threadIdx.x == 0) {
-            partials[2 * lin + 0] = v[0].hi;
-            partials[2 * lin + 1] = v[0].lo;
+            partials[2 * (blockIdx.y * nblk + lin) + 0] = v[0].hi;
+            partials[2 * (blockIdx.y * nblk + lin) + 1] = v[0].lo;
         }
     }
 }
