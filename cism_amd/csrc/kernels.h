@@ -32,14 +32,6 @@ template <typename TV>
 __global__ void k_halo_ns(Dims d, TV* a, TV* b, int nlev);
 template <typename TV>
 __global__ void k_halo_zero(Dims d, TV* a, TV* b, int nlev, int lw, int uw);
-template <typename TV, int NZMAX, int PRE, int STD>
-__global__ void k_update(Dims d, const double* scal, TV* xu, TV* xv, TV* ru, TV* rv, TV* du, TV* dv, TV* qu,
-                         TV* qv, TV* zu, TV* zv, const TV* Azu, const TV* Azv, const TV* M, const int8_t* active,
-                         double* partials);
-template <typename TV, int NZMAX>
-__global__ void k_precond(Dims d, int kind, const double* scal, const TV* ru, const TV* rv, TV* zu, TV* zv,
-                          const TV* M, const TV* Dg, const int8_t* active, const TV* zvs_u, const TV* zvs_v,
-                          double* partials);
 template <typename TV>
 __global__ void k_vsum(Dims d, const TV* ru, const TV* rv, TV* su, TV* sv);
 

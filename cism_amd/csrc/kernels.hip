@@ -351,22 +351,44 @@ __global__ void k_halo_zero(Dims d, TV* __restrict__ a, TV* __restrict__ b, int 
 // elimination has just read: the sub-diagonal field is not read at all
 // (the same values, 4 or 8 bytes per node less).
 // ---------------------------------------------------------------------------
+//
+// The coefficients of COL_CH levels are loaded together (the last level's
+// again past the end): with a load and its use level by level a column waits
+// for memory nz times, which is all the time of a small grid.
+constexpr int COL_CH = 4;
+
 template <typename TV, int NZMAX>
 __device__ __forceinline__ void thomas_column(const Dims& d, const TV* __restrict__ Ms, const TV* __restrict__ Md,
                                               const TV* __restrict__ Mp, const TV (&rhs)[NZMAX], TV (&z)[NZMAX],
                                               long long c0, bool sym) {
     TV gam[NZMAX];
-    TV beta = Md[c0];
-    z[0] = rhs[0] / beta;
+    TV beta = TV(1), sp = TV(0);
 #pragma unroll
-    for (int k = 1; k < NZMAX; ++k) {
-        if (k < d.nz) {
-            const long long c = c0 + (long long)k * d.plane;
-            const TV sp = Mp[c - d.plane];
-            gam[k] = sp / beta;
-            const TV sb = sym ? sp : Ms[c];
-            beta = Md[c] - sb * gam[k];
-            z[k] = (rhs[k] - sb * z[k - 1]) / beta;
+    for (int kb = 0; kb < NZMAX; kb += COL_CH) {
+        if (kb < d.nz) {
+            TV md[COL_CH], mp[COL_CH], ms[COL_CH];
+#pragma unroll
+            for (int u = 0; u < COL_CH; ++u) {
+                const long long c = c0 + (long long)min(kb + u, d.nz - 1) * d.plane;
+                md[u] = Md[c];
+                mp[u] = Mp[c];
+                ms[u] = sym ? TV(0) : Ms[c];
+            }
+#pragma unroll
+            for (int u = 0; u < COL_CH; ++u) {
+                const int k = kb + u;
+                if (k >= NZMAX || k >= d.nz) continue;
+                if (k == 0) {
+                    beta = md[u];
+                    z[0] = rhs[0] / beta;
+                } else {
+                    gam[k] = sp / beta;
+                    const TV sb = sym ? sp : ms[u];
+                    beta = md[u] - sb * gam[k];
+                    z[k] = (rhs[k] - sb * z[k - 1]) / beta;
+                }
+                sp = mp[u];
+            }
         }
     }
 #pragma unroll
@@ -374,12 +396,19 @@ __device__ __forceinline__ void thomas_column(const Dims& d, const TV* __restric
         if (k < d.nz - 1) z[k] = z[k] - gam[k + 1] * z[k + 1];
 }
 
-// Fused Chronopoulos-Gear update (pcg.F90:3444-3459) over all levels of one
-// column, optionally followed by the SIA solve z = M^-1 r on the new
-// residual (the next iteration's first step, :3301-3381) and the partial
-// (r, z) over owned columns.  With PRE = 0 only the update is done.
+// Fused Chronopoulos-Gear update (pcg.F90:3444-3459) and SIA column solve
+// z = M^-1 r on the new residual (the next iteration's first step,
+// :3301-3381), with the partial (r, z) and (r, r) over owned columns.
 // scal[S_ALPHA], scal[S_BETA] are read on the device.
-template <typename TV, int NZMAX, int PRE, int STD, int SYM>
+//
+// Bound: HBM on large grids (26 values per node), the latency of a column's
+// serial work on small ones.  A thread takes one component of a column: the
+// two are independent, and with half the registers per thread and twice the
+// threads a 151^2 grid reaches 190 workgroups instead of 95.  The vectors are
+// loaded COL_CH levels at a time.
+constexpr int UPD_COLS = 128;       // columns per workgroup of 256 threads
+
+template <typename TV, int NZMAX, int STD, int SYM>
 __global__ __launch_bounds__(256) void k_update(Dims d, const double* __restrict__ scal,
                                                 TV* __restrict__ xu, TV* __restrict__ xv,
                                                 TV* __restrict__ ru, TV* __restrict__ rv,
@@ -389,7 +418,11 @@ __global__ __launch_bounds__(256) void k_update(Dims d, const double* __restrict
                                                 const TV* __restrict__ Azu, const TV* __restrict__ Azv,
                                                 const TV* __restrict__ M, const int8_t* __restrict__ active,
                                                 double* __restrict__ partials) {
-    const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+    const bool second = __builtin_amdgcn_readfirstlane(threadIdx.x) >= UPD_COLS;
+    TV *x = second ? xv : xu, *r = second ? rv : ru, *dd_ = second ? dv : du, *q = second ? qv : qu;
+    TV* z = second ? zv : zu;
+    const TV* Az = second ? Azv : Azu;
+    const long long t = blockIdx.x * (long long)UPD_COLS + threadIdx.x % UPD_COLS;
     const long long ncol = (long long)d.nvx * d.nvy;
     dd acc = {0.0, 0.0};
     dd acc2 = {0.0, 0.0};
@@ -397,60 +430,128 @@ __global__ __launch_bounds__(256) void k_update(Dims d, const double* __restrict
         const int i = 1 + (int)(t % d.nvx), j = 1 + (int)(t / d.nvx);
         const TV alpha = (TV)scal[S_ALPHA], beta = (TV)scal[S_BETA];
         const long long c0 = vidx(d, 0, i, j);
-        TV rU[NZMAX], rV[NZMAX];
+        TV rk[NZMAX];
 #pragma unroll
-        for (int k = 0; k < NZMAX; ++k) {
-            if (k < d.nz) {
-                const long long c = c0 + (long long)k * d.plane;
-                TV dU, dV;
-                if (STD) {   // standard PCG: x += alpha d; r -= alpha q (pcg.F90:1395-1401)
-                    dU = du[c]; dV = dv[c];
-                    xu[c] = xu[c] + alpha * dU; xv[c] = xv[c] + alpha * dV;
-                    rU[k] = ru[c] - alpha * qu[c]; rV[k] = rv[c] - alpha * qv[c];
-                } else {
-                    dU = zu[c] + beta * du[c]; dV = zv[c] + beta * dv[c];
-                    const TV qU = Azu[c] + beta * qu[c], qV = Azv[c] + beta * qv[c];
-                    du[c] = dU; dv[c] = dV; qu[c] = qU; qv[c] = qV;
-                    xu[c] = xu[c] + alpha * dU; xv[c] = xv[c] + alpha * dV;
-                    rU[k] = ru[c] - alpha * qU; rV[k] = rv[c] - alpha * qV;
+        for (int kb = 0; kb < NZMAX; kb += COL_CH) {
+            if (kb < d.nz) {
+                TV lz[COL_CH], ld[COL_CH], la[COL_CH], lq[COL_CH], lx[COL_CH], lr[COL_CH];
+#pragma unroll
+                for (int u = 0; u < COL_CH; ++u) {
+                    const long long c = c0 + (long long)min(kb + u, d.nz - 1) * d.plane;
+                    ld[u] = dd_[c];
+                    lq[u] = q[c];
+                    lx[u] = x[c];
+                    lr[u] = r[c];
+                    if (!STD) { lz[u] = z[c]; la[u] = Az[c]; }
                 }
-                ru[c] = rU[k]; rv[c] = rV[k];
+#pragma unroll
+                for (int u = 0; u < COL_CH; ++u) {
+                    const int k = kb + u;
+                    if (k >= NZMAX || k >= d.nz) continue;
+                    const long long c = c0 + (long long)k * d.plane;
+                    if (STD) {   // standard PCG: x += alpha d; r -= alpha q (pcg.F90:1395-1401)
+                        x[c] = lx[u] + alpha * ld[u];
+                        rk[k] = lr[u] - alpha * lq[u];
+                    } else {
+                        const TV dn = lz[u] + beta * ld[u], qn = la[u] + beta * lq[u];
+                        dd_[c] = dn;
+                        q[c] = qn;
+                        x[c] = lx[u] + alpha * dn;
+                        rk[k] = lr[u] - alpha * qn;
+                    }
+                    r[c] = rk[k];
+                }
             }
         }
-        if (PRE) {
-            const bool owned = i >= d.ilo && i <= d.ihi && j >= d.jlo && j <= d.jhi;
-            if (active[t]) {
-                TV zU[NZMAX], zV[NZMAX];
-                const long long vl = d.vlen;
-                thomas_column<TV, NZMAX>(d, M + 0 * vl, M + 1 * vl, M + 2 * vl, rU, zU, c0, SYM != 0);
-                thomas_column<TV, NZMAX>(d, M + 3 * vl, M + 4 * vl, M + 5 * vl, rV, zV, c0, SYM != 0);
+        const bool owned = i >= d.ilo && i <= d.ihi && j >= d.jlo && j <= d.jhi;
+        TV zk[NZMAX];
+        if (active[t]) {
+            const long long vl = d.vlen;
+            const TV* Mc = M + (second ? 3 * vl : 0);
+            thomas_column<TV, NZMAX>(d, Mc, Mc + vl, Mc + 2 * vl, rk, zk, c0, SYM != 0);
 #pragma unroll
-                for (int k = 0; k < NZMAX; ++k)
-                    if (k < d.nz) {
-                        const long long c = c0 + (long long)k * d.plane;
-                        zu[c] = zU[k]; zv[c] = zV[k];
-                        if (owned) {
-                            acc = dd_add_d(acc, (double)rU[k] * (double)zU[k]);
-                            acc = dd_add_d(acc, (double)rV[k] * (double)zV[k]);
-                            acc2 = dd_add_d(acc2, (double)rU[k] * (double)rU[k]);
-                            acc2 = dd_add_d(acc2, (double)rV[k] * (double)rV[k]);
-                        }
-                    }
-            } else if (owned) {
-                // inactive owned column: z keeps its value (zero on the solver path)
+            for (int k = 0; k < NZMAX; ++k)
+                if (k < d.nz) z[c0 + (long long)k * d.plane] = zk[k];
+        } else {
+            // inactive column: z keeps its value (zero on the solver path)
 #pragma unroll
-                for (int k = 0; k < NZMAX; ++k)
-                    if (k < d.nz) {
-                        const long long c = c0 + (long long)k * d.plane;
-                        acc = dd_add_d(acc, (double)rU[k] * (double)zu[c]);
-                        acc = dd_add_d(acc, (double)rV[k] * (double)zv[c]);
-                        acc2 = dd_add_d(acc2, (double)rU[k] * (double)rU[k]);
-                        acc2 = dd_add_d(acc2, (double)rV[k] * (double)rV[k]);
-                    }
+            for (int k = 0; k < NZMAX; ++k)
+                if (k < d.nz) zk[k] = owned ? z[c0 + (long long)k * d.plane] : TV(0);
+        }
+        if (owned) {
+#pragma unroll
+            for (int k = 0; k < NZMAX; ++k)
+                if (k < d.nz) {
+                    acc = dd_add_d(acc, (double)rk[k] * (double)zk[k]);
+                    acc2 = dd_add_d(acc2, (double)rk[k] * (double)rk[k]);
+                }
+        }
+    }
+    dd v[2] = {acc, acc2};
+    block_reduce_dd<2, 256>(v);
+    if (threadIdx.x == 0) {
+        partials[4 * blockIdx.x + 0] = v[0].hi;
+        partials[4 * blockIdx.x + 1] = v[0].lo;
+        partials[4 * blockIdx.x + 2] = v[1].hi;
+        partials[4 * blockIdx.x + 3] = v[1].lo;
+    }
+}
+
+// The same update without the column solve (DIAG 0) or with the diagonal
+// preconditioner (DIAG 1: z = r / D where D is not zero, Dg its two fields):
+// nothing runs along a column, so a thread takes one value of each component
+// at a time and the levels run in parallel.  At most FLAT_MAX workgroups, so
+// that the partial sums stay few.
+constexpr int FLAT_MAX = 2048;
+
+template <typename TV, int DIAG, int STD>
+__global__ __launch_bounds__(256) void k_update_flat(Dims d, const double* __restrict__ scal,
+                                                     TV* __restrict__ xu, TV* __restrict__ xv,
+                                                     TV* __restrict__ ru, TV* __restrict__ rv,
+                                                     TV* __restrict__ du, TV* __restrict__ dv,
+                                                     TV* __restrict__ qu, TV* __restrict__ qv,
+                                                     TV* __restrict__ zu, TV* __restrict__ zv,
+                                                     const TV* __restrict__ Azu, const TV* __restrict__ Azv,
+                                                     const TV* __restrict__ Dg, double* __restrict__ partials) {
+    dd acc = {0.0, 0.0}, acc2 = {0.0, 0.0};
+    if (scal[S_STOP] == 0.0) {
+        const TV alpha = (TV)scal[S_ALPHA], beta = (TV)scal[S_BETA];
+        const long long n = (long long)d.nz * d.plane;
+        for (long long t = blockIdx.x * 256LL + threadIdx.x; t < n; t += gridDim.x * 256LL) {
+            const long long c = d.plane + t;
+            TV r0, r1;
+            if (STD) {
+                xu[c] = xu[c] + alpha * du[c];
+                xv[c] = xv[c] + alpha * dv[c];
+                r0 = ru[c] - alpha * qu[c];
+                r1 = rv[c] - alpha * qv[c];
+            } else {
+                const TV d0 = zu[c] + beta * du[c], d1 = zv[c] + beta * dv[c];
+                const TV q0 = Azu[c] + beta * qu[c], q1 = Azv[c] + beta * qv[c];
+                du[c] = d0; dv[c] = d1; qu[c] = q0; qv[c] = q1;
+                xu[c] = xu[c] + alpha * d0;
+                xv[c] = xv[c] + alpha * d1;
+                r0 = ru[c] - alpha * q0;
+                r1 = rv[c] - alpha * q1;
+            }
+            ru[c] = r0;
+            rv[c] = r1;
+            if (DIAG) {
+                const TV g0 = Dg[c], g1 = Dg[d.vlen + c];
+                const TV z0 = g0 != TV(0) ? r0 / g0 : TV(0), z1 = g1 != TV(0) ? r1 / g1 : TV(0);
+                zu[c] = z0;
+                zv[c] = z1;
+                const int p = (int)(t % d.plane), i = p % d.px + 1, j = p / d.px + 1;
+                if (i >= d.ilo && i <= d.ihi && j >= d.jlo && j <= d.jhi) {
+                    acc = dd_add_d(acc, (double)r0 * (double)z0);
+                    acc = dd_add_d(acc, (double)r1 * (double)z1);
+                    acc2 = dd_add_d(acc2, (double)r0 * (double)r0);
+                    acc2 = dd_add_d(acc2, (double)r1 * (double)r1);
+                }
             }
         }
     }
-    if (PRE) {
+    if (DIAG) {
         dd v[2] = {acc, acc2};
         block_reduce_dd<2, 256>(v);
         if (threadIdx.x == 0) {
@@ -462,80 +563,98 @@ __global__ __launch_bounds__(256) void k_update(Dims d, const double* __restrict
     }
 }
 
+// z = r / D (0 where D is 0) with the partial sums of k_update_flat.
+template <typename TV>
+__global__ __launch_bounds__(256) void k_precond_diag(Dims d, const double* __restrict__ scal, const TV* __restrict__ ru,
+                                                      const TV* __restrict__ rv, TV* __restrict__ zu,
+                                                      TV* __restrict__ zv, const TV* __restrict__ Dg,
+                                                      double* __restrict__ partials) {
+    dd acc = {0.0, 0.0}, acc2 = {0.0, 0.0};
+    if (scal[S_STOP] == 0.0) {
+        const long long n = (long long)d.nz * d.plane;
+        for (long long t = blockIdx.x * 256LL + threadIdx.x; t < n; t += gridDim.x * 256LL) {
+            const long long c = d.plane + t;
+            const TV r0 = ru[c], r1 = rv[c], g0 = Dg[c], g1 = Dg[d.vlen + c];
+            const TV z0 = g0 != TV(0) ? r0 / g0 : TV(0), z1 = g1 != TV(0) ? r1 / g1 : TV(0);
+            zu[c] = z0;
+            zv[c] = z1;
+            const int p = (int)(t % d.plane), i = p % d.px + 1, j = p / d.px + 1;
+            if (i >= d.ilo && i <= d.ihi && j >= d.jlo && j <= d.jhi) {
+                acc = dd_add_d(acc, (double)r0 * (double)z0);
+                acc = dd_add_d(acc, (double)r1 * (double)z1);
+                acc2 = dd_add_d(acc2, (double)r0 * (double)r0);
+                acc2 = dd_add_d(acc2, (double)r1 * (double)r1);
+            }
+        }
+    }
+    dd v[2] = {acc, acc2};
+    block_reduce_dd<2, 256>(v);
+    if (threadIdx.x == 0) {
+        partials[4 * blockIdx.x + 0] = v[0].hi;
+        partials[4 * blockIdx.x + 1] = v[0].lo;
+        partials[4 * blockIdx.x + 2] = v[1].hi;
+        partials[4 * blockIdx.x + 3] = v[1].lo;
+    }
+}
+
 // Stand-alone preconditioner apply z = PC(r) with partial (r, z) and
-// (r, r) over owned columns.  kind: 0 none (copy), 1 diag, 2 SIA.
-// For kinds 3/4 the caller adds the horizontal line-solve correction; kind 5
-// (one-level systems) takes that line solution alone.
+// (r, r) over owned columns, one component of a column per thread.  kind: 0
+// none (copy), 2 SIA (1, the diagonal, is k_precond_diag).  For kinds 3/4 the
+// caller adds the horizontal line-solve correction; kind 5 (one-level systems)
+// takes that line solution alone.
 template <typename TV, int NZMAX>
 __global__ __launch_bounds__(256) void k_precond(Dims d, int kind, const double* __restrict__ scal,
                                                  const TV* __restrict__ ru, const TV* __restrict__ rv,
                                                  TV* __restrict__ zu, TV* __restrict__ zv,
-                                                 const TV* __restrict__ M, const TV* __restrict__ Dg,
-                                                 const int8_t* __restrict__ active,
+                                                 const TV* __restrict__ M, const int8_t* __restrict__ active,
                                                  const TV* __restrict__ zvs_u, const TV* __restrict__ zvs_v,
                                                  double* __restrict__ partials, int msym) {
-    const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+    const bool second = __builtin_amdgcn_readfirstlane(threadIdx.x) >= UPD_COLS;
+    const TV* r = second ? rv : ru;
+    TV* z = second ? zv : zu;
+    const TV* zvs = second ? zvs_v : zvs_u;
+    const long long t = blockIdx.x * (long long)UPD_COLS + threadIdx.x % UPD_COLS;
     const long long ncol = (long long)d.nvx * d.nvy;
     dd acc = {0.0, 0.0}, acc2 = {0.0, 0.0};
     if (scal[S_STOP] == 0.0 && t < ncol) {
         const int i = 1 + (int)(t % d.nvx), j = 1 + (int)(t / d.nvx);
         const bool owned = i >= d.ilo && i <= d.ihi && j >= d.jlo && j <= d.jhi;
-        const long long c0 = vidx(d, 0, i, j);
-        TV rU[NZMAX], rV[NZMAX], zU[NZMAX], zV[NZMAX];
+        const long long c0 = vidx(d, 0, i, j), vl = d.vlen;
+        TV rk[NZMAX], zk[NZMAX];
 #pragma unroll
         for (int k = 0; k < NZMAX; ++k)
-            if (k < d.nz) {
-                const long long c = c0 + (long long)k * d.plane;
-                rU[k] = ru[c]; rV[k] = rv[c];
-            }
+            if (k < d.nz) rk[k] = r[c0 + (long long)k * d.plane];
         if (kind == 0) {
 #pragma unroll
-            for (int k = 0; k < NZMAX; ++k) { zU[k] = rU[k]; zV[k] = rV[k]; }
-        } else if (kind == 1) {
-#pragma unroll
-            for (int k = 0; k < NZMAX; ++k)
-                if (k < d.nz) {
-                    const long long c = c0 + (long long)k * d.plane;
-                    const TV gu = Dg[c], gv = Dg[d.vlen + c];
-                    zU[k] = gu != TV(0) ? rU[k] / gu : TV(0);
-                    zV[k] = gv != TV(0) ? rV[k] / gv : TV(0);
-                }
+            for (int k = 0; k < NZMAX; ++k) zk[k] = rk[k];
         } else if (kind == 5) {
             // 2-D solves: z is the horizontal line solution itself on every
             // vertex (pcg.F90:456-620 standard, :2020-2140 and :2275-2420 C-G)
-            const long long c2 = (long long)(j - 1) * d.nvx + (i - 1);
+            const TV a = zvs[(long long)(j - 1) * d.nvx + (i - 1)];
 #pragma unroll
-            for (int k = 0; k < NZMAX; ++k) { zU[k] = zvs_u[c2]; zV[k] = zvs_v[c2]; }
+            for (int k = 0; k < NZMAX; ++k) zk[k] = a;
         } else {
             if (active[t]) {
-                const long long vl = d.vlen;
-                thomas_column<TV, NZMAX>(d, M + 0 * vl, M + 1 * vl, M + 2 * vl, rU, zU, c0, msym != 0);
-                thomas_column<TV, NZMAX>(d, M + 3 * vl, M + 4 * vl, M + 5 * vl, rV, zV, c0, msym != 0);
+                const TV* Mc = M + (second ? 3 * vl : 0);
+                thomas_column<TV, NZMAX>(d, Mc, Mc + vl, Mc + 2 * vl, rk, zk, c0, msym != 0);
             } else {
 #pragma unroll
                 for (int k = 0; k < NZMAX; ++k)
-                    if (k < d.nz) {
-                        const long long c = c0 + (long long)k * d.plane;
-                        zU[k] = zu[c]; zV[k] = zv[c];
-                    }
+                    if (k < d.nz) zk[k] = z[c0 + (long long)k * d.plane];
             }
             if (kind >= 3) {   // z = z_SIA + z_vsum(i,j) on every column (pcg.F90:4650-4656)
-                const long long c2 = (long long)(j - 1) * d.nvx + (i - 1);
-                const TV au = zvs_u[c2], av = zvs_v[c2];
+                const TV a = zvs[(long long)(j - 1) * d.nvx + (i - 1)];
 #pragma unroll
-                for (int k = 0; k < NZMAX; ++k) { zU[k] = zU[k] + au; zV[k] = zV[k] + av; }
+                for (int k = 0; k < NZMAX; ++k) zk[k] = zk[k] + a;
             }
         }
 #pragma unroll
         for (int k = 0; k < NZMAX; ++k)
             if (k < d.nz) {
-                const long long c = c0 + (long long)k * d.plane;
-                zu[c] = zU[k]; zv[c] = zV[k];
+                z[c0 + (long long)k * d.plane] = zk[k];
                 if (owned) {
-                    acc = dd_add_d(acc, (double)rU[k] * (double)zU[k]);
-                    acc = dd_add_d(acc, (double)rV[k] * (double)zV[k]);
-                    acc2 = dd_add_d(acc2, (double)rU[k] * (double)rU[k]);
-                    acc2 = dd_add_d(acc2, (double)rV[k] * (double)rV[k]);
+                    acc = dd_add_d(acc, (double)rk[k] * (double)zk[k]);
+                    acc2 = dd_add_d(acc2, (double)rk[k] * (double)rk[k]);
                 }
             }
     }

@@ -186,6 +186,10 @@ inline int spmv64_parts(const cismgpu_system* S) {
     return S->elem_use ? elem_parts(S->d) : S->two_d ? spmv_blocks(S->d) : spmv_parts(S->d);
 }
 inline int col_blocks(const Dims& d) { return (int)nblocks((long long)d.nvx * d.nvy, 256); }
+inline int upd_blocks(const Dims& d) { return (int)nblocks((long long)d.nvx * d.nvy, UPD_COLS); }
+inline int flat_blocks(const Dims& d) { return (int)std::min<long long>(FLAT_MAX, nblocks(d.nz * d.plane, 256)); }
+// partial sums of the (r, z), (r, r) of a preconditioner
+inline int pre_parts(const Dims& d, int precond) { return precond == 1 ? flat_blocks(d) : upd_blocks(d); }
 
 template <typename TV>
 void halo(cismgpu_system* S, TV* a, TV* b, int nlev) {
@@ -269,12 +273,17 @@ int precond_sym(const cismgpu_system* S) {
     return S->sym_exact ? 1 : 0;
 }
 
-template <typename TV, int PRE, int STD>
-void launch_update(cismgpu_system* S, TV* const* v, const TV* M) {
-    // v: xu xv ru rv du dv qu qv zu zv Azu Azv
+// The C-G or standard update of v = xu xv ru rv du dv qu qv zu zv Azu Azv,
+// with the preconditioner on the new residual when fused (precond 1 or 2).
+template <typename TV, int STD>
+void launch_update(cismgpu_system* S, TV* const* v, const TV* M, int precond, bool fused) {
     const Dims& d = S->d;
-#define UPD(NZM, SY) k_update<TV, NZM, PRE, STD, SY><<<col_blocks(d), 256, 0, S->s>>>(d, S->scal, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9], v[10], v[11], M, S->active, S->partA)
-    if (precond_sym<TV>(S)) {
+    const TV* Dg = M + 6 * d.vlen;
+#define FLAT(DIAG) k_update_flat<TV, DIAG, STD><<<flat_blocks(d), 256, 0, S->s>>>(d, S->scal, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9], v[10], v[11], Dg, S->partA)
+#define UPD(NZM, SY) k_update<TV, NZM, STD, SY><<<upd_blocks(d), 256, 0, S->s>>>(d, S->scal, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9], v[10], v[11], M, S->active, S->partA)
+    if (!fused) FLAT(0);
+    else if (precond == 1) FLAT(1);
+    else if (precond_sym<TV>(S)) {
         if (d.nz <= 16) UPD(16, 1);
         else if (d.nz <= 32) UPD(32, 1);
         else UPD(64, 1);
@@ -284,6 +293,7 @@ void launch_update(cismgpu_system* S, TV* const* v, const TV* M) {
         else UPD(64, 0);
     }
 #undef UPD
+#undef FLAT
 }
 
 template <typename TV>
@@ -291,8 +301,13 @@ void launch_precond(cismgpu_system* S, int kind, const TV* ru, const TV* rv, TV*
                     const TV* Dg, const TV* zsu, const TV* zsv) {
     const Dims& d = S->d;
     const int msym = precond_sym<TV>(S);
-#define PRC(NZM) k_precond<TV, NZM><<<col_blocks(d), 256, 0, S->s>>>(d, kind, S->scal, ru, rv, zu, zv, M, Dg, S->active, zsu, zsv, S->partA, msym)
-    if (d.nz <= 16) PRC(16);
+    if (kind == 1) {
+        k_precond_diag<TV><<<flat_blocks(d), 256, 0, S->s>>>(d, S->scal, ru, rv, zu, zv, Dg, S->partA);
+        return;
+    }
+#define PRC(NZM) k_precond<TV, NZM><<<upd_blocks(d), 256, 0, S->s>>>(d, kind, S->scal, ru, rv, zu, zv, M, S->active, zsu, zsv, S->partA, msym)
+    if (d.nz == 1) PRC(1);
+    else if (d.nz <= 16) PRC(16);
     else if (d.nz <= 32) PRC(32);
     else PRC(64);
 #undef PRC
@@ -538,7 +553,8 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
     TV *xu = v[0], *xv = v[1], *ru = v[2], *rv = v[3], *du = v[4], *dv = v[5], *qu = v[6], *qv = v[7];
     TV *zu = v[8], *zv = v[9], *Azu = v[10], *Azv = v[11];
     const TV* M = std::is_same<TV, double>::value ? (const TV*)S->M64 : (const TV*)S->M32;
-    const int nsp = std::is_same<TV, double>::value ? spmv64_parts(S) : S->two_d ? spmv_blocks(d) : spmv_parts(d), ncb = col_blocks(d);
+    const int nsp = std::is_same<TV, double>::value ? spmv64_parts(S) : S->two_d ? spmv_blocks(d) : spmv_parts(d);
+    const int ncb = col_blocks(d), nub = pre_parts(d, precond);
     const long long nv = d.vlen * sizeof(TV);
     // reprosum: the global sums of the FP64 solve are exact integer-vector
     // sums (the fused compensated partials are then not used)
@@ -572,7 +588,7 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
         rs_dot<TV>(S, 2, du, qu, dv, qv);
         scalars(S, ST_CG_FIRST, S->rs_out + 2, 1, 2, S->rs_out + 4, 1, 2);
     } else {
-        scalars(S, ST_CG_FIRST, S->partA, ncb, 4, S->partB, nsp, 2);
+        scalars(S, ST_CG_FIRST, S->partA, nub, 4, S->partB, nsp, 2);
     }
     halo<TV>(S, qu, qv, d.nz);
     k_first_update<TV><<<nblocks(d.nz * d.plane, 256), 256, 0, S->s>>>(d, S->scal, xu, xv, ru, rv, du, dv, qu, qv);
@@ -586,7 +602,7 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
             rs_dot<TV>(S, 2, Azu, zu, Azv, zv);
             scalars(S, ST_CG_ITER, S->rs_out + 2, 1, 2, S->rs_out + 4, 1, 2);
         } else {
-            scalars(S, ST_CG_ITER, S->partA, ncb, 4, S->partB, nsp, 2);
+            scalars(S, ST_CG_ITER, S->partA, nub, 4, S->partB, nsp, 2);
         }
         // The no-ice halo rule zeroes vertex columns 1, 2, nvx-1 and nvx
         // (rows likewise).  The product writes owned rows only, so columns
@@ -598,9 +614,8 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
               (S->edge_zero || (d.ihi <= d.nvx - 2 && d.jhi <= d.nvy - 2))))
             halo<TV>(S, Azu, Azv, d.nz);
         const bool check = (iter % ncheck == 0) || iter == 5;
-        const bool fuse = fuse_ok && precond == 2 && !(check && !given_r);
-        if (fuse) launch_update<TV, 1, 0>(S, vv, M);
-        else launch_update<TV, 0, 0>(S, vv, M);
+        const bool fuse = fuse_ok && (precond == 1 || precond == 2) && !(check && !given_r);
+        launch_update<TV, 0>(S, vv, M, precond, fuse);
         z_ready = fuse;
         if (check) {
             if (given_r) {
@@ -609,7 +624,7 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
                     apply_precond<TV>(S, precond, ru, rv, zu, zv);
                     z_ready = true;
                 }
-                scalars(S, ST_RR, S->partA + 2, ncb, 4, nullptr, 0, 0, tol);
+                scalars(S, ST_RR, S->partA + 2, nub, 4, nullptr, 0, 0, tol);
             } else {
                 spmv<TA, TV, 2>(S, A, xu, xv, ru, rv, bu, bv, S->partB);
                 k_ring<TV><<<ncb, 256, 0, S->s>>>(d, ru, rv, bu, bv);
@@ -639,7 +654,7 @@ int std_solve(cismgpu_system* S, int precond, int ncheck, double tol, int maxite
     const Dims& d = S->d;
     double *xu = S->V(0), *xv = S->V(1), *bu = S->V(2), *bv = S->V(3), *ru = S->V(4), *rv = S->V(5);
     double *du = S->V(6), *dv = S->V(7), *qu = S->V(8), *qv = S->V(9), *zu = S->V(10), *zv = S->V(11);
-    const int nsp = spmv64_parts(S), ncb = col_blocks(d);
+    const int nsp = spmv64_parts(S), ncb = col_blocks(d), nub = pre_parts(d, precond);
     const long long nv = d.vlen * sizeof(double);
     int st = reset_scal(S);
     if (st) return st;
@@ -666,7 +681,7 @@ int std_solve(cismgpu_system* S, int precond, int ncheck, double tol, int maxite
             rs_dot<double>(S, 1, ru, zu, rv, zv);
             scalars(S, ST_STD_ETA1, S->rs_out + 2, 1, 2, nullptr, 0, 0);
         } else {
-            scalars(S, ST_STD_ETA1, S->partA, ncb, 4, nullptr, 0, 0);
+            scalars(S, ST_STD_ETA1, S->partA, nub, 4, nullptr, 0, 0);
         }
         k_axpy_ops<double><<<nblocks(d.nz * d.plane, 256), 256, 0, S->s>>>(d, 0, S->scal, zu, zv, du, dv, nullptr, nullptr);
         halo<double>(S, du, dv, d.nz);
@@ -679,9 +694,8 @@ int std_solve(cismgpu_system* S, int precond, int ncheck, double tol, int maxite
             scalars(S, ST_STD_ETA2, S->partB, nsp, 2, nullptr, 0, 0);
         }
         const bool check = (iter % ncheck == 0) || iter == 5;
-        const bool fuse = precond == 2 && !check;
-        if (fuse) launch_update<double, 1, 1>(S, vv, S->M64);
-        else launch_update<double, 0, 1>(S, vv, S->M64);
+        const bool fuse = (precond == 1 || precond == 2) && !check;
+        launch_update<double, 1>(S, vv, S->M64, precond, fuse);
         z_ready = fuse;
         if (check) {
             halo<double>(S, xu, xv, d.nz);
@@ -903,7 +917,7 @@ static int32_t system_create(const cismgpu_grid* grid, bool two_d, cismgpu_syste
     if ((e = hipStreamCreateWithFlags(&S->s, hipStreamNonBlocking)) != hipSuccess) return fail(e, "stream");
     const long long n2 = (long long)d.nvx * d.nvy;
     const long long na = d.nrows * NCOEF;
-    const int nparts = std::max(std::max(spmv_parts(d), elem_parts(d)), std::max(col_blocks(d), dot_blocks<double>(d))) + 8;
+    const int nparts = std::max(std::max(spmv_parts(d), elem_parts(d)), std::max(std::max(upd_blocks(d), flat_blocks(d)), dot_blocks<double>(d))) + 8;
     if ((e = hipMalloc(&S->active, n2)) != hipSuccess) return fail(e, "active");
     if ((e = hipMalloc(&S->A64, na * sizeof(double))) != hipSuccess) return fail(e, "A64");
     if ((e = hipMalloc(&S->M64, 8 * d.vlen * sizeof(double))) != hipSuccess) return fail(e, "M64");
