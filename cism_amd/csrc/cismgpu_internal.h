@@ -50,7 +50,13 @@ struct Dims {
     long long vlen;                 // doubles per padded vector: (nz+2)*nvy*px
     long long nrows;                // padded owned rows: nz*nyo*nxp
     long long plane;                // nvy*px
+    int zw;                         // > 0: a product stores zero in the columns of the zeroing halo rule
 };
+
+// Columns that a halo rule of width w (rows and columns per side) zeroes.
+__host__ __device__ inline bool zero_halo(const Dims& d, int i, int j, int w) {
+    return w > 0 && (i <= w || i >= d.nvx - w + 1 || j <= w || j >= d.nvy - w + 1);
+}
 
 __host__ __device__ inline long long vidx(const Dims& d, int k, int i, int j) {
     return ((long long)(k + 1) * d.nvy + (j - 1)) * d.px + (i - 1);

@@ -78,8 +78,9 @@ __global__ __launch_bounds__(256) void k_spmv(Dims d, const TA* __restrict__ A,
                 acc = dd_add_d(acc, (double)ru * (double)ru);
                 acc = dd_add_d(acc, (double)rv * (double)rv);
             } else {
-                yu[c0] = su;
-                yv[c0] = sv;
+                const bool zr = MODE == 1 && zero_halo(d, i, j, d.zw);
+                yu[c0] = zr ? TV(0) : su;
+                yv[c0] = zr ? TV(0) : sv;
                 if (MODE == 1) {
                     acc = dd_add_d(acc, (double)su * (double)xu[c0]);
                     acc = dd_add_d(acc, (double)sv * (double)xv[c0]);
@@ -248,8 +249,9 @@ __global__ __launch_bounds__(256) void k_spmv_plane(Dims d, const TA* __restrict
             acc = dd_add_d(acc, (double)ru * (double)ru);
             acc = dd_add_d(acc, (double)rv * (double)rv);
         } else {
-            yu[c0] = su;
-            yv[c0] = sv;
+            const bool zr = MODE == 1 && zero_halo(d, i, j, d.zw);
+            yu[c0] = zr ? TV(0) : su;
+            yv[c0] = zr ? TV(0) : sv;
             if (MODE == 1) {
                 acc = dd_add_d(acc, (double)su * (double)xu[c0]);
                 acc = dd_add_d(acc, (double)sv * (double)xv[c0]);
@@ -791,21 +793,24 @@ __global__ void k_halo2d_zero(Dims d, TV* __restrict__ a, TV* __restrict__ b) {
 }
 
 // Whole-array updates used by the standard PCG and the first C-G pass.
-// op 0: d = z + beta d            (pcg.F90:1336-1337)
+// op 0: d = z + beta d            (pcg.F90:1336-1337), zero in the columns that
+//       the halo rule of width zw zeroes
 // op 1: d = z                      (pcg.F90:3240-3241)
 // op 2: r = b - y                  (residual from a matvec output)
 template <typename TV>
 __global__ void k_axpy_ops(Dims d, int op, const double* __restrict__ scal, const TV* __restrict__ s1u,
                            const TV* __restrict__ s1v, TV* __restrict__ tu, TV* __restrict__ tv,
-                           const TV* __restrict__ s2u, const TV* __restrict__ s2v) {
+                           const TV* __restrict__ s2u, const TV* __restrict__ s2v, int zw) {
     const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
     const long long lo = d.plane, hi = (long long)(d.nz + 1) * d.plane;   // real levels only
     const long long c = lo + t;
     if (c >= hi || scal[S_STOP] != 0.0) return;
     if (op == 0) {
         const TV beta = (TV)scal[S_BETA];
-        tu[c] = s1u[c] + beta * tu[c];
-        tv[c] = s1v[c] + beta * tv[c];
+        const int p = (int)(t % d.plane);
+        const bool zr = zero_halo(d, p % d.px + 1, p / d.px + 1, zw);
+        tu[c] = zr ? TV(0) : s1u[c] + beta * tu[c];
+        tv[c] = zr ? TV(0) : s1v[c] + beta * tv[c];
     } else if (op == 1) {
         tu[c] = s1u[c];
         tv[c] = s1v[c];
@@ -854,15 +859,8 @@ __device__ __forceinline__ dd sum_partials(const double* __restrict__ p, int n, 
     return v;
 }
 
-__global__ __launch_bounds__(SCAL_THREADS) void k_scalars(int stage, const double* __restrict__ pa, int na, int sa,
-                                                          const double* __restrict__ pb, int nb, int sb,
-                                                          double* __restrict__ scal, double tolerance) {
-    const dd va = sum_partials(pa, na, sa);
-    const dd vb = pb ? sum_partials(pb, nb, sb) : dd{0.0, 0.0};
-    dd v[2] = {va, vb};
-    block_reduce_dd<2, SCAL_THREADS>(v);
-    if (threadIdx.x != 0) return;
-    const double A = v[0].hi + v[0].lo, B = v[1].hi + v[1].lo;
+__device__ __forceinline__ void scalar_stage(int stage, double A, double B, double* __restrict__ scal,
+                                             double tolerance) {
     if (scal[S_STOP] != 0.0 && stage != ST_BB && stage != ST_RR) return;
     switch (stage) {
     case ST_BB:   // L2_rhs = sqrt((b,b))
@@ -917,6 +915,27 @@ __global__ __launch_bounds__(SCAL_THREADS) void k_scalars(int stage, const doubl
         scal[S_DOT2] = B;
         break;
     }
+}
+
+// The last one-workgroup stage of every global sum.  mirror (host memory): the
+// host reads the scalars there as soon as they are final, without a copy.
+__global__ __launch_bounds__(SCAL_THREADS) void k_scalars(int stage, const double* __restrict__ pa, int na, int sa,
+                                                          const double* __restrict__ pb, int nb, int sb,
+                                                          double* __restrict__ scal, double tolerance,
+                                                          double* __restrict__ mirror, double seq) {
+    const dd va = sum_partials(pa, na, sa);
+    const dd vb = pb ? sum_partials(pb, nb, sb) : dd{0.0, 0.0};
+    dd v[2] = {va, vb};
+    block_reduce_dd<2, SCAL_THREADS>(v);
+    if (threadIdx.x != 0) return;
+    const double A = v[0].hi + v[0].lo, B = v[1].hi + v[1].lo;
+    scalar_stage(stage, A, B, scal, tolerance);
+    if (!mirror) return;
+    // the scalars for the host, then the sequence number it waits for
+#pragma unroll
+    for (int q = 0; q < S_NSLOTS; ++q)
+        __hip_atomic_store(mirror + q, scal[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(mirror + S_NSLOTS, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ---------------------------------------------------------------------------

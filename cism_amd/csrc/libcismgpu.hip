@@ -71,7 +71,9 @@ struct cismgpu_system {
     double* partA = nullptr;
     double* partB = nullptr;
     double* scal = nullptr;
-    double* scal_h = nullptr;      // pinned mirror
+    double* scal_h = nullptr;      // pinned mirror, then the sequence number of its last fill
+    double scal_seq = 0.0;
+    int zw = 0;                    // halo width that the next products store as zero (Dims::zw)
     TriPC tri;
     // assembly inputs on the device
     void* asm_buf = nullptr;
@@ -239,19 +241,21 @@ template <typename TA, typename TV, int MODE>
 void spmv(cismgpu_system* S, const TA* A, const TV* xu, const TV* xv, TV* yu, TV* yv, const TV* bu, const TV* bv,
           double* part) {
     const bool t = S->timing && S->ev_used + 2 <= (int)S->ev.size();
+    Dims d = S->d;
+    d.zw = S->zw;
     if (t) hipEventRecord(S->ev[S->ev_used], S->s);
     if (S->two_d)   // one level: only the kA = 0 plane of the rows is read
-        k_spmv_plane<TA, TV, MODE><<<spmv_blocks(S->d), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part);
+        k_spmv_plane<TA, TV, MODE><<<spmv_blocks(S->d), 256, 0, S->s>>>(d, A, xu, xv, yu, yv, bu, bv, part);
     else if constexpr (std::is_same<TA, double>::value) {
         if (S->elem_use && MODE != 0)   // an assembled system in element form
             k_spmv_elem<MODE == 0 ? 1 : MODE>
                 <<<dim3(elem_blocks(S->d), elem_parts(S->d) / elem_blocks(S->d)), WAVE * EL_J, 0, S->s>>>(
                     S->d, S->asm_in, S->elemq, S->elem_bd, xu, xv, yu, yv, bu, bv, part, elem_split(S->d));
         else if (S->a64_sym && (const double*)A == S->A64)   // FP64 half (symmetric) storage
-            k_spmv_sym64<MODE><<<spmv_grid(S->d), 256, 0, S->s>>>(S->d, S->A64h, xu, xv, yu, yv, bu, bv, part,
+            k_spmv_sym64<MODE><<<spmv_grid(S->d), 256, 0, S->s>>>(d, S->A64h, xu, xv, yu, yv, bu, bv, part,
                                                                   level_split(S->d));
         else
-            k_spmv<TA, TV, MODE><<<spmv_grid(S->d), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part,
+            k_spmv<TA, TV, MODE><<<spmv_grid(S->d), 256, 0, S->s>>>(d, A, xu, xv, yu, yv, bu, bv, part,
                                                                     level_split(S->d));
     }
     else if (std::is_same<TA, float>::value && S->a32_sym)   // FP32 half (symmetric) storage
@@ -315,7 +319,39 @@ void launch_precond(cismgpu_system* S, int kind, const TV* ru, const TV* rv, TV*
 
 void scalars(cismgpu_system* S, int stage, const double* pa, int na, int sa, const double* pb, int nb, int sb,
              double tol = 0.0) {
-    k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(stage, pa, na, sa, pb, nb, sb, S->scal, tol);
+    k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(stage, pa, na, sa, pb, nb, sb, S->scal, tol, nullptr, 0.0);
+}
+
+// The same, and wait until the scalars are in scal_h: the kernel writes them
+// there itself and the host polls for the sequence number, so a check costs
+// neither a copy launch nor the wake-up of a blocked thread.  With the halo
+// and ring launches that change nothing left out, the 31^2 x 10 dome drop-in
+// (110 iterations, 22 checks) went from 6.7 to 5.6 ms.  The stream is asked
+// now and then, so that a failed launch ends the wait.
+int scalars_to_host(cismgpu_system* S, int stage, const double* pa, int na, int sa, double tol) {
+    S->scal_seq += 1.0;
+    k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(stage, pa, na, sa, nullptr, 0, 0, S->scal, tol, S->scal_h, S->scal_seq);
+    CG_CHECK(hipGetLastError());
+    double* flag = S->scal_h + S_NSLOTS;
+    double seen = 0.0;
+    for (unsigned n = 1;; ++n) {
+        __atomic_load(flag, &seen, __ATOMIC_ACQUIRE);
+        if (seen == S->scal_seq) return CISMGPU_OK;
+        if (n % 8192 == 0 && hipStreamQuery(S->s) != hipErrorNotReady) break;
+    }
+    CG_CHECK(hipStreamSynchronize(S->s));
+    return CISMGPU_OK;
+}
+
+// The zeroing halo rule changes nothing in a vector that is zero outside the
+// owned columns: outflow zeroes the outermost rows and columns, which are
+// never owned; no-ice two per side, of which the last owned row and column
+// is one.  There the rows of an assembled matrix are zero (k_matrix_noice_edge),
+// and so are the products and b, hence the residual.
+bool zero_halo_is_noop(const cismgpu_system* S) {
+    const Dims& d = S->d;
+    return d.bc == 1 || (d.bc == 3 && d.ilo >= 3 && d.jlo >= 3 &&
+                         (S->edge_zero || (d.ihi <= d.nvx - 2 && d.jhi <= d.nvy - 2)));
 }
 
 // Exact (reproducible) sum over owned vertices of the summands a1*b1 + a2*b2
@@ -554,7 +590,7 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
     TV *zu = v[8], *zv = v[9], *Azu = v[10], *Azv = v[11];
     const TV* M = std::is_same<TV, double>::value ? (const TV*)S->M64 : (const TV*)S->M32;
     const int nsp = std::is_same<TV, double>::value ? spmv64_parts(S) : S->two_d ? spmv_blocks(d) : spmv_parts(d);
-    const int ncb = col_blocks(d), nub = pre_parts(d, precond);
+    const int nub = pre_parts(d, precond);
     const long long nv = d.vlen * sizeof(TV);
     // reprosum: the global sums of the FP64 solve are exact integer-vector
     // sums (the fused compensated partials are then not used)
@@ -581,7 +617,7 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
     }
     halo<TV>(S, ru, rv, d.nz);
     apply_precond<TV>(S, precond, ru, rv, zu, zv);
-    k_axpy_ops<TV><<<nblocks(d.nz * d.plane, 256), 256, 0, S->s>>>(d, 1, S->scal, zu, zv, du, dv, nullptr, nullptr);
+    k_axpy_ops<TV><<<nblocks(d.nz * d.plane, 256), 256, 0, S->s>>>(d, 1, S->scal, zu, zv, du, dv, nullptr, nullptr, 0);
     spmv<TA, TV, 1>(S, A, du, dv, qu, qv, nullptr, nullptr, S->partB);
     if (rs) {
         rs_dot<TV>(S, 1, ru, zu, rv, zv);
@@ -594,9 +630,17 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
     k_first_update<TV><<<nblocks(d.nz * d.plane, 256), 256, 0, S->s>>>(d, S->scal, xu, xv, ru, rv, du, dv, qu, qv);
     TV* vv[12] = {xu, xv, ru, rv, du, dv, qu, qv, zu, zv, Azu, Azv};
     bool z_ready = false;
+    // The halo of A z: the product writes owned columns only, so the others
+    // keep the zero they got at the start.  Where the zeroing rule reaches
+    // owned columns, the FP64 products of caller-given rows store the zero
+    // themselves (their (A z, z) sums still take the values before it).
+    const bool noop = zero_halo_is_noop(S);
+    const bool fold = !noop && d.bc == 3 && !rs && std::is_same<TA, double>::value && !S->elem_use;
     for (int iter = 2; iter <= maxiters; ++iter) {
         if (!z_ready) apply_precond<TV>(S, precond, ru, rv, zu, zv);
+        S->zw = fold ? 2 : 0;
         spmv<TA, TV, 1>(S, A, zu, zv, Azu, Azv, nullptr, nullptr, S->partB);
+        S->zw = 0;
         if (rs) {
             rs_dot<TV>(S, 1, ru, zu, rv, zv);
             rs_dot<TV>(S, 2, Azu, zu, Azv, zv);
@@ -604,15 +648,7 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
         } else {
             scalars(S, ST_CG_ITER, S->partA, nub, 4, S->partB, nsp, 2);
         }
-        // The no-ice halo rule zeroes vertex columns 1, 2, nvx-1 and nvx
-        // (rows likewise).  The product writes owned rows only, so columns
-        // outside the owned range keep the zero they got at the start, and
-        // an owned last column holds zero rows after the assembly's edge
-        // pass, where A z is +0 already: then the halo pass of A z changes
-        // nothing and is skipped.
-        if (!(d.bc == 3 && d.ilo >= 3 && d.jlo >= 3 &&
-              (S->edge_zero || (d.ihi <= d.nvx - 2 && d.jhi <= d.nvy - 2))))
-            halo<TV>(S, Azu, Azv, d.nz);
+        if (!fold && !noop) halo<TV>(S, Azu, Azv, d.nz);
         const bool check = (iter % ncheck == 0) || iter == 5;
         const bool fuse = fuse_ok && (precond == 1 || precond == 2) && !(check && !given_r);
         launch_update<TV, 0>(S, vv, M, precond, fuse);
@@ -624,23 +660,22 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
                     apply_precond<TV>(S, precond, ru, rv, zu, zv);
                     z_ready = true;
                 }
-                scalars(S, ST_RR, S->partA + 2, nub, 4, nullptr, 0, 0, tol);
+                st = scalars_to_host(S, ST_RR, S->partA + 2, nub, 4, tol);
             } else {
+                // outside the owned columns r keeps what the halo rule left there
                 spmv<TA, TV, 2>(S, A, xu, xv, ru, rv, bu, bv, S->partB);
-                k_ring<TV><<<ncb, 256, 0, S->s>>>(d, ru, rv, bu, bv);
                 if (rs) {
                     rs_dot<TV>(S, 3, ru, ru, rv, rv);
-                    scalars(S, ST_RR, S->rs_out + 6, 1, 2, nullptr, 0, 0, tol);
+                    st = scalars_to_host(S, ST_RR, S->rs_out + 6, 1, 2, tol);
                 } else {
-                    scalars(S, ST_RR, S->partB, nsp, 2, nullptr, 0, 0, tol);
+                    st = scalars_to_host(S, ST_RR, S->partB, nsp, 2, tol);
                 }
             }
-            st = sync_scal(S);
             if (st) return st;
             if (S->scal_h[S_NAN] != 0.0) { cismgpu_set_error("Chron-Gear PCG solver has failed, alpha = NaN"); return CISMGPU_ERR_NAN; }
             *err = S->scal_h[S_ERR];
-            if (S->scal_h[S_CONV] != 0.0) { *niters = iter; break; }
-            if (!given_r) halo<TV>(S, ru, rv, d.nz);
+            if (S->scal_h[S_CONV] != 0.0) { *niters = iter; return CISMGPU_OK; }
+            if (!given_r && !noop) halo<TV>(S, ru, rv, d.nz);
         }
     }
     st = sync_scal(S);
@@ -683,10 +718,11 @@ int std_solve(cismgpu_system* S, int precond, int ncheck, double tol, int maxite
         } else {
             scalars(S, ST_STD_ETA1, S->partA, nub, 4, nullptr, 0, 0);
         }
-        k_axpy_ops<double><<<nblocks(d.nz * d.plane, 256), 256, 0, S->s>>>(d, 0, S->scal, zu, zv, du, dv, nullptr, nullptr);
-        halo<double>(S, du, dv, d.nz);
+        // d, and its halo where the rule zeroes
+        const int zw = d.bc == 1 ? 1 : d.bc == 3 ? 2 : 0;
+        k_axpy_ops<double><<<nblocks(d.nz * d.plane, 256), 256, 0, S->s>>>(d, 0, S->scal, zu, zv, du, dv, nullptr, nullptr, zw);
+        if (!zw) halo<double>(S, du, dv, d.nz);
         spmv<double, double, 1>(S, S->A64, du, dv, qu, qv, nullptr, nullptr, S->partB);
-        k_ring<double><<<ncb, 256, 0, S->s>>>(d, qu, qv, nullptr, nullptr);
         if (rs) {
             rs_dot<double>(S, 2, du, qu, dv, qv);
             scalars(S, ST_STD_ETA2, S->rs_out + 4, 1, 2, nullptr, 0, 0);
@@ -699,19 +735,18 @@ int std_solve(cismgpu_system* S, int precond, int ncheck, double tol, int maxite
         z_ready = fuse;
         if (check) {
             halo<double>(S, xu, xv, d.nz);
+            // outside the owned columns r keeps the b it got at the start (q is zero there)
             spmv<double, double, 2>(S, S->A64, xu, xv, ru, rv, bu, bv, S->partB);
-            k_ring<double><<<ncb, 256, 0, S->s>>>(d, ru, rv, bu, bv);
             if (rs) {
                 rs_dot<double>(S, 3, ru, ru, rv, rv);
-                scalars(S, ST_RR, S->rs_out + 6, 1, 2, nullptr, 0, 0, tol);
+                st = scalars_to_host(S, ST_RR, S->rs_out + 6, 1, 2, tol);
             } else {
-                scalars(S, ST_RR, S->partB, nsp, 2, nullptr, 0, 0, tol);
+                st = scalars_to_host(S, ST_RR, S->partB, nsp, 2, tol);
             }
-            st = sync_scal(S);
             if (st) return st;
             if (S->scal_h[S_NAN] != 0.0) { cismgpu_set_error("PCG solver has failed, alpha = NaN"); return CISMGPU_ERR_NAN; }
             *err = S->scal_h[S_ERR];
-            if (S->scal_h[S_CONV] != 0.0) { *niters = iter; break; }
+            if (S->scal_h[S_CONV] != 0.0) { *niters = iter; return CISMGPU_OK; }
         }
     }
     st = sync_scal(S);
@@ -832,9 +867,9 @@ int mixed_solve(cismgpu_system* S, const cismgpu_solve_opts* o, cismgpu_solve_in
         k_ring<double><<<col_blocks(d), 256, 0, S->s>>>(d, ru, rv, bu, bv);
         if (S->repro) {
             rs_dot<double>(S, 3, ru, ru, rv, rv);
-            k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->rs_out + 6, 1, 2, nullptr, 0, 0, S->scal, 0.0);
+            k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->rs_out + 6, 1, 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0.0);
         } else {
-            k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->partB, nsp, 2, nullptr, 0, 0, S->scal, 0.0);
+            k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->partB, nsp, 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0.0);
         }
         st = sync_scal(S);
         if (st) return st;
@@ -927,7 +962,8 @@ static int32_t system_create(const cismgpu_grid* grid, bool two_d, cismgpu_syste
     if ((e = hipMalloc(&S->partA, 4 * nparts * sizeof(double))) != hipSuccess) return fail(e, "partA");
     if ((e = hipMalloc(&S->partB, 4 * nparts * sizeof(double))) != hipSuccess) return fail(e, "partB");
     if ((e = hipMalloc(&S->scal, S_NSLOTS * sizeof(double))) != hipSuccess) return fail(e, "scal");
-    if ((e = hipHostMalloc(&S->scal_h, S_NSLOTS * sizeof(double), hipHostMallocDefault)) != hipSuccess) return fail(e, "scal_h");
+    if ((e = hipHostMalloc(&S->scal_h, (S_NSLOTS + 1) * sizeof(double), hipHostMallocCoherent)) != hipSuccess) return fail(e, "scal_h");
+    S->scal_h[S_NSLOTS] = 0.0;
     S->repro = grid->reprosum != 0;
     if (S->repro) {
         if ((e = hipMalloc(&S->rs_part, (size_t)RS_MAX_BLOCKS * RS_L * sizeof(unsigned long long))) != hipSuccess)
@@ -2386,13 +2422,13 @@ extern "C" int32_t cismgpu_system_residual(cismgpu_system* S, double* ru, double
                                                               level_split(d));
     if (S->repro) {
         rs_dot<double>(S, 3, r0, r0, r1, r1);
-        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->rs_out + 6, 1, 2, nullptr, 0, 0, S->scal, 0.0);
+        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->rs_out + 6, 1, 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0.0);
         rs_dot<double>(S, 0, S->V(2), S->V(2), S->V(3), S->V(3));
-        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_BB, S->rs_out, 1, 2, nullptr, 0, 0, S->scal, 0.0);
+        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_BB, S->rs_out, 1, 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0.0);
     } else {
-        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->partB, spmv_parts(d), 2, nullptr, 0, 0, S->scal, 0.0);
+        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->partB, spmv_parts(d), 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0.0);
         k_dot<double><<<dot_blocks<double>(d), 256, 0, S->s>>>(d, S->V(2), S->V(2), S->V(3), S->V(3), S->partA);
-        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_BB, S->partA, dot_blocks<double>(d), 2, nullptr, 0, 0, S->scal, 0.0);
+        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_BB, S->partA, dot_blocks<double>(d), 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0.0);
     }
     int st = sync_scal(S);
     if (st) return st;
