@@ -80,7 +80,7 @@ struct EnsPtrs {
     double* r64;
     float *r32, *d32, *q32, *z32, *Az32, *e32;
     double* part_mat;                // [ntile_mat] dd
-    double* part_col;                // [2][ntile_col][2] dd
+    double* part_col;                // [2][ntile_col][component][2] dd
     EnsState* st;                    // [2][nmem]
     unsigned* bar;                   // barrier: count, generation
     int* err_flag;                   // set when a barrier wait exceeded its bound
@@ -115,13 +115,22 @@ __device__ __forceinline__ void grid_barrier(unsigned* bar, unsigned nblocks, lo
 }
 
 // Deterministic reduction of a member's tile partials (stride = doubles per
-// tile) by one wavefront; every lane returns the sum.
+// tile) by one wavefront, four loads per lane in flight; every lane returns
+// the sum.
 __device__ double member_sum(const double* part, int t0, int n, int stride, int which) {
     dd acc = {0.0, 0.0};
     const int lane = threadIdx.x % WAVE;
-    for (int t = lane; t < n; t += WAVE) {
-        const double* p = part + (size_t)(t0 + t) * stride + 2 * which;
-        acc = dd_add(acc, dd{p[0], p[1]});
+    for (int tb = lane; tb < n; tb += 4 * WAVE) {
+        double h[4], l[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int t = tb + u * WAVE;
+            const double* p = part + (size_t)(t0 + min(t, n - 1)) * stride + 2 * which;
+            h[u] = t < n ? p[0] : 0.0;
+            l[u] = t < n ? p[1] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc = dd_add(acc, dd{h[u], l[u]});
     }
     for (int off = WAVE / 2; off > 0; off >>= 1) acc = dd_add(acc, dd_shfl_down(acc, off));
     return __shfl(acc.hi + acc.lo, 0, WAVE);
@@ -140,7 +149,7 @@ __device__ __forceinline__ int step_phase(const EnsState& st, const EnsMember& M
                                           const EnsParams& P) {
     if (st.phase != M_INNER || st.inner_it == 0) return st.phase;
     if (st.inner_it % P.ncheck != 0 && st.inner_it < P.inner_maxiters) return M_INNER;
-    const double rr = member_sum(pc_cur, M.t0_col, M.ntile_col, 4, 1);
+    const double rr = member_sum(pc_cur, 2 * M.t0_col, 2 * M.ntile_col, 4, 1);
     const double ie = sqrt(rr) / st.r0;
     return (ie < P.inner_tol || st.inner_it >= P.inner_maxiters || !(ie == ie)) ? M_FOLD : M_INNER;
 }
@@ -294,66 +303,63 @@ __device__ __forceinline__ dd matrix_tile_half(const EnsMember& M, int lt, const
 // ---------------------------------------------------------------- column phase work
 // One vertex column, one velocity component: the C-G vector update (START:
 // load r from the FP64 residual and clear e, d, q) followed by the SIA
-// Thomas solve z = M^-1 r (easy_sia_solver), streamed level by level; the
-// forward sweep leaves the partial solution in z, the back substitution
-// finishes it.  Accumulates (r,z) and (r,r) over owned columns.
+// Thomas solve z = M^-1 r (easy_sia_solver).  Accumulates (r,z) and (r,r)
+// over owned columns.  The vectors and coefficients come four levels at a
+// time and r and z stay in registers: a wavefront has about one item per
+// step, so what it takes is its chain of memory waits (20 members of 32..128
+// vertices a side: 60.7 ms a solve, against 73.5 with both components in one
+// wavefront, each level loaded when its turn comes and z read back).
 template <int NZMAX, bool START>
 __device__ __forceinline__ void column_component(const Dims& d, const EnsPtrs& Q, long long vb,
                                                  const float* __restrict__ Mm, long long c0, bool owned, bool act,
                                                  float fa, float fb, dd& a_rz, dd& a_rr) {
     const long long pl = d.plane;
-    const float *Ms = Mm, *Md = Mm + d.vlen, *Mp = Mm + 2 * d.vlen;
-    float gam[NZMAX];
-    float bet = 1.f, zprev = 0.f;
+    float rk[NZMAX];
 #pragma unroll
-    for (int k = 0; k < NZMAX; ++k)
-        if (k < d.nz) {
-            const long long cl = c0 + (long long)k * pl;
-            const long long c = vb + cl;
-            float rk;
-            if (START) {
-                rk = owned ? (float)Q.r64[c] : 0.f;
-                Q.e32[c] = 0.f;
-                Q.d32[c] = 0.f;
-                Q.q32[c] = 0.f;
-            } else {
-                const float dk = Q.z32[c] + fb * Q.d32[c];
-                const float qk = Q.Az32[c] + fb * Q.q32[c];
-                Q.d32[c] = dk;
-                Q.q32[c] = qk;
-                Q.e32[c] = Q.e32[c] + fa * dk;
-                rk = Q.r32[c] - fa * qk;
-            }
-            Q.r32[c] = rk;
-            if (act) {
-                float zt;
-                if (k == 0) {
-                    bet = Md[cl];
-                    zt = rk / bet;
+    for (int kb = 0; kb < NZMAX; kb += COL_CH)
+        if (kb < d.nz) {
+            float lz[COL_CH], ld[COL_CH], la[COL_CH], lq[COL_CH], le[COL_CH], lr[COL_CH];
+#pragma unroll
+            for (int u = 0; u < COL_CH; ++u) {
+                const long long c = vb + c0 + (long long)min(kb + u, d.nz - 1) * pl;
+                if (START) {
+                    lr[u] = owned ? (float)Q.r64[c] : 0.f;
                 } else {
-                    gam[k] = Mp[cl - pl] / bet;
-                    const float sb = Ms[cl];
-                    bet = Md[cl] - sb * gam[k];
-                    zt = (rk - sb * zprev) / bet;
+                    lz[u] = Q.z32[c]; ld[u] = Q.d32[c]; la[u] = Q.Az32[c];
+                    lq[u] = Q.q32[c]; le[u] = Q.e32[c]; lr[u] = Q.r32[c];
                 }
-                Q.z32[c] = zt;
-                zprev = zt;
-            } else if (START) {
-                Q.z32[c] = 0.f;
             }
-            if (owned) a_rr = dd_add_d(a_rr, (double)rk * (double)rk);
+#pragma unroll
+            for (int u = 0; u < COL_CH; ++u) {
+                const int k = kb + u;
+                if (k >= d.nz) continue;
+                const long long c = vb + c0 + (long long)k * pl;
+                if (START) {
+                    rk[k] = lr[u];
+                    Q.e32[c] = 0.f;
+                    Q.d32[c] = 0.f;
+                    Q.q32[c] = 0.f;
+                    if (!act) Q.z32[c] = 0.f;
+                } else {
+                    const float dk = lz[u] + fb * ld[u];
+                    const float qk = la[u] + fb * lq[u];
+                    Q.d32[c] = dk;
+                    Q.q32[c] = qk;
+                    Q.e32[c] = le[u] + fa * dk;
+                    rk[k] = lr[u] - fa * qk;
+                }
+                Q.r32[c] = rk[k];
+                if (owned) a_rr = dd_add_d(a_rr, (double)rk[k] * (double)rk[k]);
+            }
         }
     if (act) {
-        float znext = zprev;
-        if (owned) a_rz = dd_add_d(a_rz, (double)Q.r32[vb + c0 + (long long)(d.nz - 1) * pl] * (double)znext);
+        float zk[NZMAX];
+        thomas_column<float, NZMAX>(d, Mm, Mm + d.vlen, Mm + 2 * d.vlen, rk, zk, c0, false);
 #pragma unroll
-        for (int k = NZMAX - 2; k >= 0; --k)
-            if (k < d.nz - 1) {
-                const long long c = vb + c0 + (long long)k * pl;
-                const float zk = Q.z32[c] - gam[k + 1] * znext;
-                Q.z32[c] = zk;
-                znext = zk;
-                if (owned) a_rz = dd_add_d(a_rz, (double)Q.r32[c] * (double)zk);
+        for (int k = 0; k < NZMAX; ++k)
+            if (k < d.nz) {
+                Q.z32[vb + c0 + (long long)k * pl] = zk[k];
+                if (owned) a_rz = dd_add_d(a_rz, (double)rk[k] * (double)zk[k]);
             }
     }
 }
@@ -371,8 +377,8 @@ __global__ __launch_bounds__(ENS_BS) void k_ensemble(EnsParams P, EnsPtrs Q) {
         const int cur = step & 1, nxt = cur ^ 1;
         const EnsState* S0 = Q.st + (size_t)cur * P.nmem;
         EnsState* S1 = Q.st + (size_t)nxt * P.nmem;
-        const double* pc_cur = Q.part_col + (size_t)cur * P.ntile_col * 4;
-        double* pc_nxt = Q.part_col + (size_t)nxt * P.ntile_col * 4;
+        const double* pc_cur = Q.part_col + (size_t)cur * P.ntile_col * 8;
+        double* pc_nxt = Q.part_col + (size_t)nxt * P.ntile_col * 8;
         // all members done?  (every workgroup reads the same states)
         if (threadIdx.x == 0) s_any = 0;
         __syncthreads();
@@ -410,12 +416,14 @@ __global__ __launch_bounds__(ENS_BS) void k_ensemble(EnsParams P, EnsPtrs Q) {
         }
         grid_barrier(Q.bar, G, P.spin_limit, Q.err_flag);
         // ------------------------------------------------ column phase
-        for (int tile = gw; tile < P.ntile_col; tile += W) {
+        // an item is one velocity component of a column tile
+        for (int item = gw; item < 2 * P.ntile_col; item += W) {
+            const int tile = item >> 1, comp = item & 1;
             const int m = Q.tile_mem_col[tile];
             const EnsMember& M = Q.mem[m];
             const Dims& d = M.d;
             const EnsState st = S0[m];
-            const bool lead = (tile == M.t0_col);
+            const bool lead = (item == 2 * M.t0_col);
             if (st.phase == M_DONE) {
                 if (lead && lane == 0) S1[m] = st;
                 continue;
@@ -426,10 +434,10 @@ __global__ __launch_bounds__(ENS_BS) void k_ensemble(EnsParams P, EnsPtrs Q) {
             const bool incol = t < (long long)d.nvx * d.nvy;
             const int i = 1 + (int)(t % d.nvx), j = 1 + (int)(t / d.nvx);
             const bool owned = incol && i >= d.ilo && i <= d.ihi && j >= d.jlo && j <= d.jhi;
-            const long long vo = M.v_off, vl = d.vlen;
+            const long long vo = M.v_off + comp * d.vlen;
             const long long c0 = incol ? vidx(d, 0, i, j) : 0;
             const bool act = incol && Q.active[M.c_off + t] != 0;
-            const float* Mm = Q.M32 + 3 * vo;
+            const float* Mm = Q.M32 + 3 * vo;     // the component's three fields
             dd a_rz = {0.0, 0.0}, a_rr = {0.0, 0.0};
             EnsState ns = st;
             bool partials = false;
@@ -445,21 +453,17 @@ __global__ __launch_bounds__(ENS_BS) void k_ensemble(EnsParams P, EnsPtrs Q) {
                     ns.inner_it = 0;
                     ns.outer_it = st.outer_it + 1;
                     partials = true;
-                    if (incol) {
-                        column_component<NZMAX, true>(d, Q, vo, Mm, c0, owned, act, 0.f, 0.f, a_rz, a_rr);
-                        column_component<NZMAX, true>(d, Q, vo + vl, Mm + 3 * vl, c0, owned, act, 0.f, 0.f, a_rz,
-                                                      a_rr);
-                    }
+                    if (incol) column_component<NZMAX, true>(d, Q, vo, Mm, c0, owned, act, 0.f, 0.f, a_rz, a_rr);
                 }
             } else if (ph == M_INNER) {
-                const double rho = member_sum(pc_cur, M.t0_col, M.ntile_col, 4, 0);
+                const double rho = member_sum(pc_cur, 2 * M.t0_col, 2 * M.ntile_col, 4, 0);
                 const double delta = member_sum(Q.part_mat, M.t0_mat, M.ntile_mat, 2, 0);
                 double beta = 0.0, sigma = delta;
                 if (st.inner_it > 0) {
                     beta = rho / st.rho;
                     sigma = delta - beta * rho / st.alpha;
                 } else {
-                    ns.r0 = sqrt(member_sum(pc_cur, M.t0_col, M.ntile_col, 4, 1));
+                    ns.r0 = sqrt(member_sum(pc_cur, 2 * M.t0_col, 2 * M.ntile_col, 4, 1));
                 }
                 const double alpha = rho / sigma;
                 ns.rho = rho;
@@ -473,14 +477,12 @@ __global__ __launch_bounds__(ENS_BS) void k_ensemble(EnsParams P, EnsPtrs Q) {
                 } else if (incol) {
                     const float fa = (float)alpha, fb = (float)beta;
                     column_component<NZMAX, false>(d, Q, vo, Mm, c0, owned, act, fa, fb, a_rz, a_rr);
-                    column_component<NZMAX, false>(d, Q, vo + vl, Mm + 3 * vl, c0, owned, act, fa, fb, a_rz, a_rr);
                 }
             } else {  // M_FOLD: x64 += e, then the next outer residual
                 if (incol)
                     for (int k = 0; k < d.nz; ++k) {
                         const long long c = vo + c0 + (long long)k * d.plane;
                         Q.x64[c] = Q.x64[c] + (double)Q.e32[c];
-                        Q.x64[c + vl] = Q.x64[c + vl] + (double)Q.e32[c + vl];
                     }
                 ns.phase = M_OUTER;
             }
@@ -488,7 +490,7 @@ __global__ __launch_bounds__(ENS_BS) void k_ensemble(EnsParams P, EnsPtrs Q) {
                 a_rz = wave_reduce(a_rz);
                 a_rr = wave_reduce(a_rr);
                 if (lane == 0) {
-                    double* p = pc_nxt + (size_t)tile * 4;
+                    double* p = pc_nxt + (size_t)item * 4;
                     p[0] = a_rz.hi; p[1] = a_rz.lo; p[2] = a_rr.hi; p[3] = a_rr.lo;
                 }
             }

@@ -2676,7 +2676,7 @@ static int ens_tiles(cismgpu_ensemble* E) {
     CG_CHECK(hipMemcpy(E->d_tile_mem_mat, tm.data(), tm.size() * sizeof(int), hipMemcpyHostToDevice));
     CG_CHECK(hipMemcpy(E->d_tile_mem_col, tc.data(), tc.size() * sizeof(int), hipMemcpyHostToDevice));
     CG_CHECK(hipMalloc(&E->part_mat, 2 * (size_t)tmat * sizeof(double)));
-    CG_CHECK(hipMalloc(&E->part_col, 2 * 4 * (size_t)tcol * sizeof(double)));
+    CG_CHECK(hipMalloc(&E->part_col, 2 * 8 * (size_t)tcol * sizeof(double)));
     CG_CHECK(hipMemcpy(E->d_mem, E->mem.data(), E->nmem * sizeof(EnsMember), hipMemcpyHostToDevice));
     return CISMGPU_OK;
 }
