@@ -219,6 +219,11 @@ void halo2d(cismgpu_system* S, TV* a, TV* b) {
     }
 }
 
+static bool elem_form_wanted() {
+    const char* e = getenv("CISMGPU_SPMV_FULL");
+    return !(e && e[0] == '1');
+}
+
 // FP32 half storage: the kernel with the level-to-level LDS exchange of the
 // partner slots (default) or the one that re-reads them (CISMGPU_SPMV_SYMX=0)
 static bool use_symx() {
@@ -797,6 +802,10 @@ int ensure_lowp(cismgpu_system* S, int precision) {
         ok = false;
         const char* env = getenv("CISMGPU_SPMV_FULL");
         if (S->two_d || (env && env[0] == '1') || !half_storage_fits(d)) return CISMGPU_OK;
+        if (S->sym_exact) {   // exactly symmetric in FP64 (the assembly's count), so also rounded
+            ok = true;
+            return CISMGPU_OK;
+        }
         unsigned long long* cnt = nullptr;
         unsigned long long h = 1;
         CG_CHECK(hipMalloc(&cnt, sizeof(unsigned long long)));
@@ -838,7 +847,6 @@ int mixed_solve(cismgpu_system* S, const cismgpu_solve_opts* o, cismgpu_solve_in
     if (st) return st;
     double *xu = S->V(0), *xv = S->V(1), *bu = S->V(2), *bv = S->V(3), *ru = S->V(4), *rv = S->V(5);
     float* w[12] = {S->W(0), S->W(1), S->W(4), S->W(5), S->W(6), S->W(7), S->W(8), S->W(9), S->W(10), S->W(11), S->W(12), S->W(13)};
-    const int nsp = spmv64_parts(S);
     const long long nvf = d.vlen * sizeof(float);
     // ||b|| once
     st = reset_scal(S);
@@ -862,7 +870,10 @@ int mixed_solve(cismgpu_system* S, const cismgpu_solve_opts* o, cismgpu_solve_in
         halo<double>(S, xu, xv, d.nz);
         const int tspmv = S->timing;
         S->timing = false;   // time the inner (dominant) SpMV only
+        S->elem_use = S->elem_ok;
+        const int nsp = spmv64_parts(S);
         spmv<double, double, 2>(S, S->A64, xu, xv, ru, rv, bu, bv, S->partB);
+        S->elem_use = false;
         S->timing = tspmv;
         k_ring<double><<<col_blocks(d), 256, 0, S->s>>>(d, ru, rv, bu, bv);
         if (S->repro) {
@@ -1175,12 +1186,13 @@ int32_t cismgpu_system_solve(cismgpu_system* S, const cismgpu_solve_opts* o, cis
     // new matrix and cached until the next: the line-solve factors, the
     // exact-symmetry checks and the half-storage / low-precision copies
     {
-        // FP64 products of an assembled system in element form
-        // (CISMGPU_SPMV_FULL=1 keeps the full rows)
-        const char* full = getenv("CISMGPU_SPMV_FULL");
-        S->elem_use = S->elem_ok && o->precision == CISMGPU_FP64 && !(full && full[0] == '1');
+        // FP64 products of an assembled system in element form, the
+        // refinement residuals of a mixed solve among them
+        // (CISMGPU_SPMV_FULL=1 keeps the full rows in an FP64 solve)
+        const bool elem = S->elem_ok && (o->precision != CISMGPU_FP64 || elem_form_wanted());
+        S->elem_use = elem && o->precision == CISMGPU_FP64;
         const bool fresh = ((o->precond == 3 || o->precond == 4) && S->tri.mode != o->precond) ||
-                           (!S->elem_use && !S->a64h_ready) ||
+                           (!elem && !S->a64h_ready) ||
                            (o->precision == CISMGPU_MIXED_FP32 && !S->a32_ready) ||
                            (o->precision == CISMGPU_MIXED_BF16 && !S->a16_ready) ||
                            (o->precision != CISMGPU_FP64 && !S->m32_ready);
@@ -1189,7 +1201,7 @@ int32_t cismgpu_system_solve(cismgpu_system* S, const cismgpu_solve_opts* o, cis
             st = setup_tri(S, o->precond);
             if (st) { S->elem_use = false; return st; }
         }
-        if (!S->elem_use) {
+        if (!elem) {
             st = ensure_half64(S);
             if (st) return st;
         }
@@ -2418,15 +2430,21 @@ extern "C" int32_t cismgpu_system_residual(cismgpu_system* S, double* ru, double
     CG_CHECK(hipMemsetAsync(r0, 0, 2 * d.vlen * sizeof(double), S->s));
     { const int st_ = reset_scal(S); if (st_) return st_; }
     // r = b - A x over owned rows with partial (r,r); resid = -r on owned active rows
-    k_spmv<double, double, 2><<<spmv_grid(d), 256, 0, S->s>>>(d, S->A64, S->V(0), S->V(1), r0, r1, S->V(2), S->V(3), S->partB,
-                                                              level_split(d));
+    S->elem_use = S->elem_ok && elem_form_wanted();
+    const int nsp = spmv64_parts(S);
+    if (S->elem_use || S->two_d)
+        spmv<double, double, 2>(S, S->A64, S->V(0), S->V(1), r0, r1, S->V(2), S->V(3), S->partB);
+    else
+        k_spmv<double, double, 2><<<spmv_grid(d), 256, 0, S->s>>>(d, S->A64, S->V(0), S->V(1), r0, r1, S->V(2), S->V(3),
+                                                                  S->partB, level_split(d));
+    S->elem_use = false;
     if (S->repro) {
         rs_dot<double>(S, 3, r0, r0, r1, r1);
         k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->rs_out + 6, 1, 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0.0);
         rs_dot<double>(S, 0, S->V(2), S->V(2), S->V(3), S->V(3));
         k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_BB, S->rs_out, 1, 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0.0);
     } else {
-        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->partB, spmv_parts(d), 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0.0);
+        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->partB, nsp, 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0.0);
         k_dot<double><<<dot_blocks<double>(d), 256, 0, S->s>>>(d, S->V(2), S->V(2), S->V(3), S->V(3), S->partA);
         k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_BB, S->partA, dot_blocks<double>(d), 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0.0);
     }
