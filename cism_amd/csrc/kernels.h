@@ -45,9 +45,6 @@ __global__ void k_halo2d_ns(Dims d, TV* a, TV* b);
 template <typename TV>
 __global__ void k_halo2d_zero(Dims d, TV* a, TV* b);
 template <typename TV>
-__global__ void k_axpy_ops(Dims d, int op, const double* scal, const TV* s1u, const TV* s1v, TV* tu, TV* tv,
-                           const TV* s2u, const TV* s2v, int zw);
-template <typename TV>
 __global__ void k_first_update(Dims d, const double* scal, TV* xu, TV* xv, TV* ru, TV* rv, const TV* du,
                                const TV* dv, const TV* qu, const TV* qv);
 __global__ void k_scalars(int stage, const double* pa, int na, int sa, const double* pb, int nb, int sb,

@@ -343,6 +343,119 @@ __global__ void k_halo_zero(Dims d, TV* __restrict__ a, TV* __restrict__ b, int 
     }
 }
 
+// Sum of n compensated partials (stride s) by one thread of a BS-thread
+// workgroup: four independent loads in flight, then their adds, so the loop
+// waits for memory once per four partials.
+template <int BS>
+__device__ __forceinline__ dd sum_partials(const double* __restrict__ p, int n, int s) {
+    dd v = {0.0, 0.0};
+    for (int b0 = threadIdx.x; b0 < n; b0 += 4 * BS) {
+        double h[4], l[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int b = b0 + u * BS;
+            h[u] = b < n ? p[(long long)s * b] : 0.0;
+            l[u] = b < n ? p[(long long)s * b + 1] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (b0 + u * BS < n) v = dd_add(v, dd{h[u], l[u]});
+    }
+    return v;
+}
+
+__device__ __forceinline__ void scalar_stage(int stage, double A, double B, double* __restrict__ scal,
+                                             double tolerance) {
+    if (scal[S_STOP] != 0.0 && stage != ST_BB && stage != ST_RR) return;
+    switch (stage) {
+    case ST_BB:   // L2_rhs = sqrt((b,b))
+        scal[S_BB] = A;
+        scal[S_L2RHS] = sqrt(A);
+        break;
+    case ST_RR: {  // err = sqrt((r,r)) / L2_rhs
+        scal[S_RR] = A;
+        const double err = sqrt(A) / scal[S_L2RHS];
+        scal[S_ERR] = err;
+        scal[S_CONV] = (err < tolerance) ? 1.0 : 0.0;
+        break;
+    }
+    case ST_CG_FIRST: {   // rho_old = (r,z); sigma = (d,q); alpha = rho_old/sigma
+        scal[S_RHO] = A;
+        scal[S_SIGMA] = B;
+        const double alpha = A / B;
+        scal[S_ALPHA] = alpha;
+        if (alpha != alpha) { scal[S_NAN] = 1.0; scal[S_STOP] = 1.0; }
+        break;
+    }
+    case ST_CG_ITER: {    // beta = rho/rho_old; sigma = delta - beta*rho/alpha; alpha = rho/sigma
+        const double rho = A, delta = B;
+        const double beta = rho / scal[S_RHO];
+        const double sigma = delta - beta * rho / scal[S_ALPHA];
+        const double alpha = rho / sigma;
+        scal[S_BETA] = beta;
+        scal[S_SIGMA] = sigma;
+        scal[S_ALPHA] = alpha;
+        scal[S_RHO] = rho;
+        if (alpha != alpha) { scal[S_NAN] = 1.0; scal[S_STOP] = 1.0; }
+        break;
+    }
+    case ST_STD_ETA1: {   // eta1 = (r,z); beta = eta1/eta0
+        const double eta1 = A;
+        scal[S_RHO] = eta1;
+        scal[S_BETA] = eta1 / scal[S_ETA0];
+        if (eta1 != eta1) { scal[S_NAN] = 1.0; scal[S_STOP] = 1.0; }
+        break;
+    }
+    case ST_STD_ETA2: {   // eta0 = eta1; eta2 = (d,q); alpha = eta1/eta2
+        const double eta1 = scal[S_RHO];
+        scal[S_ETA0] = eta1;
+        scal[S_SIGMA] = A;
+        const double alpha = eta1 / A;
+        scal[S_ALPHA] = alpha;
+        if (alpha != alpha) { scal[S_NAN] = 1.0; scal[S_STOP] = 1.0; }
+        break;
+    }
+    case ST_DOT:          // plain dot product into S_DOT
+        scal[S_DOT] = A;
+        scal[S_DOT2] = B;
+        break;
+    }
+}
+
+// The scalar stage in front of the kernel that reads its results: every
+// workgroup sums the partials itself, in the same order, and workgroup 0 keeps
+// the new scalars in `out` (the other workgroups may still read `in`).  For up
+// to FUSE_MAX partial sums this takes less than a launch of its own (5 us):
+// 31^2 x 10 drop-in 5.65 -> 4.65 ms, 384^2 SSA Picard 22.2 -> 20.7 ms.  Beyond,
+// the sums of every workgroup would cost more than one workgroup's.
+constexpr int FUSE_MAX = 2048;
+
+struct ScalIn {
+    int stage;                       // -1: the scalars in `in` are current
+    const double *pa, *pb;           // partial sums, counts and strides as k_scalars
+    int na, sa, nb, sb;
+    const double* in;
+    double* out;
+};
+
+template <int BS>
+__device__ __forceinline__ void fused_scalars(const ScalIn& R, double (&sc)[S_NSLOTS]) {
+    if (R.stage >= 0) {
+        dd v[2] = {sum_partials<BS>(R.pa, R.na, R.sa), {0.0, 0.0}};
+        if (R.pb) v[1] = sum_partials<BS>(R.pb, R.nb, R.sb);
+        if (threadIdx.x < S_NSLOTS) sc[threadIdx.x] = R.in[threadIdx.x];
+        block_reduce_dd<2, BS>(v);   // its barrier also covers sc
+        if (threadIdx.x == 0) {
+            scalar_stage(R.stage, v[0].hi + v[0].lo, v[1].hi + v[1].lo, sc, 0.0);
+            if (blockIdx.x == 0)
+                for (int q = 0; q < S_NSLOTS; ++q) R.out[q] = sc[q];
+        }
+    } else if (threadIdx.x < S_NSLOTS) {
+        sc[threadIdx.x] = R.in[threadIdx.x];
+    }
+    __syncthreads();
+}
+
 // ---------------------------------------------------------------------------
 // Preconditioners, one thread per vertex column over the full extent.
 // SIA: easy_sia_solver -- Thomas solve of the vertical tridiagonal part of
@@ -401,7 +514,7 @@ __device__ __forceinline__ void thomas_column(const Dims& d, const TV* __restric
 // Fused Chronopoulos-Gear update (pcg.F90:3444-3459) and SIA column solve
 // z = M^-1 r on the new residual (the next iteration's first step,
 // :3301-3381), with the partial (r, z) and (r, r) over owned columns.
-// scal[S_ALPHA], scal[S_BETA] are read on the device.
+// The scalars come from R, summed here where the partial sums are few.
 //
 // Bound: HBM on large grids (26 values per node), the latency of a column's
 // serial work on small ones.  A thread takes one component of a column: the
@@ -411,7 +524,7 @@ __device__ __forceinline__ void thomas_column(const Dims& d, const TV* __restric
 constexpr int UPD_COLS = 128;       // columns per workgroup of 256 threads
 
 template <typename TV, int NZMAX, int STD, int SYM>
-__global__ __launch_bounds__(256) void k_update(Dims d, const double* __restrict__ scal,
+__global__ __launch_bounds__(256) void k_update(Dims d, ScalIn R,
                                                 TV* __restrict__ xu, TV* __restrict__ xv,
                                                 TV* __restrict__ ru, TV* __restrict__ rv,
                                                 TV* __restrict__ du, TV* __restrict__ dv,
@@ -420,6 +533,8 @@ __global__ __launch_bounds__(256) void k_update(Dims d, const double* __restrict
                                                 const TV* __restrict__ Azu, const TV* __restrict__ Azv,
                                                 const TV* __restrict__ M, const int8_t* __restrict__ active,
                                                 double* __restrict__ partials) {
+    __shared__ double scal[S_NSLOTS];
+    fused_scalars<256>(R, scal);
     const bool second = __builtin_amdgcn_readfirstlane(threadIdx.x) >= UPD_COLS;
     TV *x = second ? xv : xu, *r = second ? rv : ru, *dd_ = second ? dv : du, *q = second ? qv : qu;
     TV* z = second ? zv : zu;
@@ -507,7 +622,7 @@ __global__ __launch_bounds__(256) void k_update(Dims d, const double* __restrict
 constexpr int FLAT_MAX = 2048;
 
 template <typename TV, int DIAG, int STD>
-__global__ __launch_bounds__(256) void k_update_flat(Dims d, const double* __restrict__ scal,
+__global__ __launch_bounds__(256) void k_update_flat(Dims d, ScalIn R,
                                                      TV* __restrict__ xu, TV* __restrict__ xv,
                                                      TV* __restrict__ ru, TV* __restrict__ rv,
                                                      TV* __restrict__ du, TV* __restrict__ dv,
@@ -515,6 +630,8 @@ __global__ __launch_bounds__(256) void k_update_flat(Dims d, const double* __res
                                                      TV* __restrict__ zu, TV* __restrict__ zv,
                                                      const TV* __restrict__ Azu, const TV* __restrict__ Azv,
                                                      const TV* __restrict__ Dg, double* __restrict__ partials) {
+    __shared__ double scal[S_NSLOTS];
+    fused_scalars<256>(R, scal);
     dd acc = {0.0, 0.0}, acc2 = {0.0, 0.0};
     if (scal[S_STOP] == 0.0) {
         const TV alpha = (TV)scal[S_ALPHA], beta = (TV)scal[S_BETA];
@@ -798,9 +915,11 @@ __global__ void k_halo2d_zero(Dims d, TV* __restrict__ a, TV* __restrict__ b) {
 // op 1: d = z                      (pcg.F90:3240-3241)
 // op 2: r = b - y                  (residual from a matvec output)
 template <typename TV>
-__global__ void k_axpy_ops(Dims d, int op, const double* __restrict__ scal, const TV* __restrict__ s1u,
+__global__ __launch_bounds__(256) void k_axpy_ops(Dims d, int op, ScalIn R, const TV* __restrict__ s1u,
                            const TV* __restrict__ s1v, TV* __restrict__ tu, TV* __restrict__ tv,
                            const TV* __restrict__ s2u, const TV* __restrict__ s2v, int zw) {
+    __shared__ double scal[S_NSLOTS];
+    fused_scalars<256>(R, scal);
     const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
     const long long lo = d.plane, hi = (long long)(d.nz + 1) * d.plane;   // real levels only
     const long long c = lo + t;
@@ -839,92 +958,14 @@ __global__ void k_first_update(Dims d, const double* __restrict__ scal, TV* __re
 // Scalar stage: one block sums the per-block compensated partials in a fixed
 // order and advances the Krylov scalars on the device.
 // ---------------------------------------------------------------------------
-// Sum of n compensated partials (stride s) by one thread of a
-// SCAL_THREADS-thread workgroup: four independent loads in flight, then
-// their adds, so the loop waits for memory once per four partials.
-__device__ __forceinline__ dd sum_partials(const double* __restrict__ p, int n, int s) {
-    dd v = {0.0, 0.0};
-    for (int b0 = threadIdx.x; b0 < n; b0 += 4 * SCAL_THREADS) {
-        double h[4], l[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int b = b0 + u * SCAL_THREADS;
-            h[u] = b < n ? p[(long long)s * b] : 0.0;
-            l[u] = b < n ? p[(long long)s * b + 1] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (b0 + u * SCAL_THREADS < n) v = dd_add(v, dd{h[u], l[u]});
-    }
-    return v;
-}
-
-__device__ __forceinline__ void scalar_stage(int stage, double A, double B, double* __restrict__ scal,
-                                             double tolerance) {
-    if (scal[S_STOP] != 0.0 && stage != ST_BB && stage != ST_RR) return;
-    switch (stage) {
-    case ST_BB:   // L2_rhs = sqrt((b,b))
-        scal[S_BB] = A;
-        scal[S_L2RHS] = sqrt(A);
-        break;
-    case ST_RR: {  // err = sqrt((r,r)) / L2_rhs
-        scal[S_RR] = A;
-        const double err = sqrt(A) / scal[S_L2RHS];
-        scal[S_ERR] = err;
-        scal[S_CONV] = (err < tolerance) ? 1.0 : 0.0;
-        break;
-    }
-    case ST_CG_FIRST: {   // rho_old = (r,z); sigma = (d,q); alpha = rho_old/sigma
-        scal[S_RHO] = A;
-        scal[S_SIGMA] = B;
-        const double alpha = A / B;
-        scal[S_ALPHA] = alpha;
-        if (alpha != alpha) { scal[S_NAN] = 1.0; scal[S_STOP] = 1.0; }
-        break;
-    }
-    case ST_CG_ITER: {    // beta = rho/rho_old; sigma = delta - beta*rho/alpha; alpha = rho/sigma
-        const double rho = A, delta = B;
-        const double beta = rho / scal[S_RHO];
-        const double sigma = delta - beta * rho / scal[S_ALPHA];
-        const double alpha = rho / sigma;
-        scal[S_BETA] = beta;
-        scal[S_SIGMA] = sigma;
-        scal[S_ALPHA] = alpha;
-        scal[S_RHO] = rho;
-        if (alpha != alpha) { scal[S_NAN] = 1.0; scal[S_STOP] = 1.0; }
-        break;
-    }
-    case ST_STD_ETA1: {   // eta1 = (r,z); beta = eta1/eta0
-        const double eta1 = A;
-        scal[S_RHO] = eta1;
-        scal[S_BETA] = eta1 / scal[S_ETA0];
-        if (eta1 != eta1) { scal[S_NAN] = 1.0; scal[S_STOP] = 1.0; }
-        break;
-    }
-    case ST_STD_ETA2: {   // eta0 = eta1; eta2 = (d,q); alpha = eta1/eta2
-        const double eta1 = scal[S_RHO];
-        scal[S_ETA0] = eta1;
-        scal[S_SIGMA] = A;
-        const double alpha = eta1 / A;
-        scal[S_ALPHA] = alpha;
-        if (alpha != alpha) { scal[S_NAN] = 1.0; scal[S_STOP] = 1.0; }
-        break;
-    }
-    case ST_DOT:          // plain dot product into S_DOT
-        scal[S_DOT] = A;
-        scal[S_DOT2] = B;
-        break;
-    }
-}
-
 // The last one-workgroup stage of every global sum.  mirror (host memory): the
 // host reads the scalars there as soon as they are final, without a copy.
 __global__ __launch_bounds__(SCAL_THREADS) void k_scalars(int stage, const double* __restrict__ pa, int na, int sa,
                                                           const double* __restrict__ pb, int nb, int sb,
                                                           double* __restrict__ scal, double tolerance,
                                                           double* __restrict__ mirror, double seq) {
-    const dd va = sum_partials(pa, na, sa);
-    const dd vb = pb ? sum_partials(pb, nb, sb) : dd{0.0, 0.0};
+    const dd va = sum_partials<SCAL_THREADS>(pa, na, sa);
+    const dd vb = pb ? sum_partials<SCAL_THREADS>(pb, nb, sb) : dd{0.0, 0.0};
     dd v[2] = {va, vb};
     block_reduce_dd<2, SCAL_THREADS>(v);
     if (threadIdx.x != 0) return;

@@ -70,7 +70,10 @@ struct cismgpu_system {
     float* v32 = nullptr;          // inner: 0 eu 1 ev 2 r0u 3 r0v 4 ru 5 rv 6 du 7 dv 8 qu 9 qv 10 zu 11 zv 12 Azu 13 Azv
     double* partA = nullptr;
     double* partB = nullptr;
+    double* partA_alt = nullptr;   // where an update that sums partA itself writes the next ones (swapped with partA)
     double* scal = nullptr;
+    double* scal_alt = nullptr;    // the same for the scalars; both halves of scal_buf
+    double* scal_buf = nullptr;
     double* scal_h = nullptr;      // pinned mirror, then the sequence number of its last fill
     double scal_seq = 0.0;
     int zw = 0;                    // halo width that the next products store as zero (Dims::zw)
@@ -282,14 +285,28 @@ int precond_sym(const cismgpu_system* S) {
     return S->sym_exact ? 1 : 0;
 }
 
+// The scalars of a kernel that reads them: as they are, or summed by it from
+// these partial sums (then the result is in the other scalar buffer, which
+// becomes the current one after the launch).
+ScalIn scal_in(cismgpu_system* S) {
+    return ScalIn{-1, nullptr, nullptr, 0, 0, 0, 0, S->scal, S->scal_alt};
+}
+ScalIn scal_in(cismgpu_system* S, int stage, const double* pa, int na, int sa, const double* pb, int nb, int sb) {
+    return ScalIn{stage, pa, pb, na, sa, nb, sb, S->scal, S->scal_alt};
+}
+void scal_done(cismgpu_system* S, const ScalIn& R) {
+    if (R.stage >= 0) std::swap(S->scal, S->scal_alt);
+}
+
 // The C-G or standard update of v = xu xv ru rv du dv qu qv zu zv Azu Azv,
 // with the preconditioner on the new residual when fused (precond 1 or 2).
 template <typename TV, int STD>
-void launch_update(cismgpu_system* S, TV* const* v, const TV* M, int precond, bool fused) {
+void launch_update(cismgpu_system* S, const ScalIn& R, TV* const* v, const TV* M, int precond, bool fused) {
     const Dims& d = S->d;
+    if (R.stage >= 0 && R.pa == S->partA) std::swap(S->partA, S->partA_alt);   // its reader writes the other
     const TV* Dg = M + 6 * d.vlen;
-#define FLAT(DIAG) k_update_flat<TV, DIAG, STD><<<flat_blocks(d), 256, 0, S->s>>>(d, S->scal, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9], v[10], v[11], Dg, S->partA)
-#define UPD(NZM, SY) k_update<TV, NZM, STD, SY><<<upd_blocks(d), 256, 0, S->s>>>(d, S->scal, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9], v[10], v[11], M, S->active, S->partA)
+#define FLAT(DIAG) k_update_flat<TV, DIAG, STD><<<flat_blocks(d), 256, 0, S->s>>>(d, R, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9], v[10], v[11], Dg, S->partA)
+#define UPD(NZM, SY) k_update<TV, NZM, STD, SY><<<upd_blocks(d), 256, 0, S->s>>>(d, R, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9], v[10], v[11], M, S->active, S->partA)
     if (!fused) FLAT(0);
     else if (precond == 1) FLAT(1);
     else if (precond_sym<TV>(S)) {
@@ -303,6 +320,7 @@ void launch_update(cismgpu_system* S, TV* const* v, const TV* M, int precond, bo
     }
 #undef UPD
 #undef FLAT
+    scal_done(S, R);
 }
 
 template <typename TV>
@@ -622,7 +640,7 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
     }
     halo<TV>(S, ru, rv, d.nz);
     apply_precond<TV>(S, precond, ru, rv, zu, zv);
-    k_axpy_ops<TV><<<nblocks(d.nz * d.plane, 256), 256, 0, S->s>>>(d, 1, S->scal, zu, zv, du, dv, nullptr, nullptr, 0);
+    k_axpy_ops<TV><<<nblocks(d.nz * d.plane, 256), 256, 0, S->s>>>(d, 1, scal_in(S), zu, zv, du, dv, nullptr, nullptr, 0);
     spmv<TA, TV, 1>(S, A, du, dv, qu, qv, nullptr, nullptr, S->partB);
     if (rs) {
         rs_dot<TV>(S, 1, ru, zu, rv, zv);
@@ -640,6 +658,7 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
     // owned columns, the FP64 products of caller-given rows store the zero
     // themselves (their (A z, z) sums still take the values before it).
     const bool noop = zero_halo_is_noop(S);
+    const bool fuse_scal = !rs && nub + nsp <= FUSE_MAX;   // the update sums the partials itself
     const bool fold = !noop && d.bc == 3 && !rs && std::is_same<TA, double>::value && !S->elem_use;
     for (int iter = 2; iter <= maxiters; ++iter) {
         if (!z_ready) apply_precond<TV>(S, precond, ru, rv, zu, zv);
@@ -650,13 +669,14 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
             rs_dot<TV>(S, 1, ru, zu, rv, zv);
             rs_dot<TV>(S, 2, Azu, zu, Azv, zv);
             scalars(S, ST_CG_ITER, S->rs_out + 2, 1, 2, S->rs_out + 4, 1, 2);
-        } else {
+        } else if (!fuse_scal) {
             scalars(S, ST_CG_ITER, S->partA, nub, 4, S->partB, nsp, 2);
         }
         if (!fold && !noop) halo<TV>(S, Azu, Azv, d.nz);
         const bool check = (iter % ncheck == 0) || iter == 5;
         const bool fuse = fuse_ok && (precond == 1 || precond == 2) && !(check && !given_r);
-        launch_update<TV, 0>(S, vv, M, precond, fuse);
+        launch_update<TV, 0>(S, fuse_scal ? scal_in(S, ST_CG_ITER, S->partA, nub, 4, S->partB, nsp, 2) : scal_in(S), vv,
+                             M, precond, fuse);
         z_ready = fuse;
         if (check) {
             if (given_r) {
@@ -714,29 +734,33 @@ int std_solve(cismgpu_system* S, int precond, int ncheck, double tol, int maxite
         scalars(S, ST_BB, S->partB, dot_blocks<double>(d), 2, nullptr, 0, 0);
     }
     double* vv[12] = {xu, xv, ru, rv, du, dv, qu, qv, zu, zv, nullptr, nullptr};
+    const bool fuse_scal = !rs && std::max(nub, nsp) <= FUSE_MAX;   // the readers sum the partials themselves
     bool z_ready = false;
     for (int iter = 1; iter <= maxiters; ++iter) {
         if (!z_ready) apply_precond<double>(S, precond, ru, rv, zu, zv);
         if (rs) {
             rs_dot<double>(S, 1, ru, zu, rv, zv);
             scalars(S, ST_STD_ETA1, S->rs_out + 2, 1, 2, nullptr, 0, 0);
-        } else {
+        } else if (!fuse_scal) {
             scalars(S, ST_STD_ETA1, S->partA, nub, 4, nullptr, 0, 0);
         }
+        const ScalIn r1 = fuse_scal ? scal_in(S, ST_STD_ETA1, S->partA, nub, 4, nullptr, 0, 0) : scal_in(S);
         // d, and its halo where the rule zeroes
         const int zw = d.bc == 1 ? 1 : d.bc == 3 ? 2 : 0;
-        k_axpy_ops<double><<<nblocks(d.nz * d.plane, 256), 256, 0, S->s>>>(d, 0, S->scal, zu, zv, du, dv, nullptr, nullptr, zw);
+        k_axpy_ops<double><<<nblocks(d.nz * d.plane, 256), 256, 0, S->s>>>(d, 0, r1, zu, zv, du, dv, nullptr, nullptr, zw);
+        scal_done(S, r1);
         if (!zw) halo<double>(S, du, dv, d.nz);
         spmv<double, double, 1>(S, S->A64, du, dv, qu, qv, nullptr, nullptr, S->partB);
         if (rs) {
             rs_dot<double>(S, 2, du, qu, dv, qv);
             scalars(S, ST_STD_ETA2, S->rs_out + 4, 1, 2, nullptr, 0, 0);
-        } else {
+        } else if (!fuse_scal) {
             scalars(S, ST_STD_ETA2, S->partB, nsp, 2, nullptr, 0, 0);
         }
         const bool check = (iter % ncheck == 0) || iter == 5;
         const bool fuse = (precond == 1 || precond == 2) && !check;
-        launch_update<double, 1>(S, vv, S->M64, precond, fuse);
+        launch_update<double, 1>(S, fuse_scal ? scal_in(S, ST_STD_ETA2, S->partB, nsp, 2, nullptr, 0, 0) : scal_in(S), vv,
+                                 S->M64, precond, fuse);
         z_ready = fuse;
         if (check) {
             halo<double>(S, xu, xv, d.nz);
@@ -972,7 +996,10 @@ static int32_t system_create(const cismgpu_grid* grid, bool two_d, cismgpu_syste
     if ((e = hipMalloc(&S->v32, 14 * d.vlen * sizeof(float))) != hipSuccess) return fail(e, "v32");
     if ((e = hipMalloc(&S->partA, 4 * nparts * sizeof(double))) != hipSuccess) return fail(e, "partA");
     if ((e = hipMalloc(&S->partB, 4 * nparts * sizeof(double))) != hipSuccess) return fail(e, "partB");
-    if ((e = hipMalloc(&S->scal, S_NSLOTS * sizeof(double))) != hipSuccess) return fail(e, "scal");
+    if ((e = hipMalloc(&S->partA_alt, 4 * nparts * sizeof(double))) != hipSuccess) return fail(e, "partA_alt");
+    if ((e = hipMalloc(&S->scal_buf, 2 * S_NSLOTS * sizeof(double))) != hipSuccess) return fail(e, "scal");
+    S->scal = S->scal_buf;
+    S->scal_alt = S->scal_buf + S_NSLOTS;
     if ((e = hipHostMalloc(&S->scal_h, (S_NSLOTS + 1) * sizeof(double), hipHostMallocCoherent)) != hipSuccess) return fail(e, "scal_h");
     S->scal_h[S_NSLOTS] = 0.0;
     S->repro = grid->reprosum != 0;
@@ -1009,7 +1036,7 @@ int32_t cismgpu_system_destroy(cismgpu_system* S) {
     if (!S) return CISMGPU_OK;
     if (S->s) hipStreamSynchronize(S->s);
     for (void* p : {(void*)S->active, (void*)S->A64, (void*)S->A32, (void*)S->A16, (void*)S->stage, (void*)S->M64,
-                    (void*)S->M32, (void*)S->v64, (void*)S->v32, (void*)S->partA, (void*)S->partB, (void*)S->scal,
+                    (void*)S->M32, (void*)S->v64, (void*)S->v32, (void*)S->partA, (void*)S->partB, (void*)S->partA_alt, (void*)S->scal_buf,
                     (void*)S->tri.a, (void*)S->tri.a32, S->asm_buf, (void*)S->efvs, (void*)S->Atmp, (void*)S->saved, (void*)S->work, (void*)S->load3, (void*)S->A64h, (void*)S->diva_buf, (void*)S->efva2, (void*)S->rs_part, (void*)S->rs_bad,
                     (void*)S->rs_out, (void*)S->elemq, (void*)S->elem_bd, S->cb_buf})
         if (p) hipFree(p);
