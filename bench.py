@@ -160,13 +160,13 @@ def main():
     # HBM bytes per launch of the same kernel from the rocprofv3 FETCH_SIZE / WRITE_SIZE
     # passes of this workload, scaled by the counters' reading of a copy kernel of known size
     traffic = None
-    kname = {1: "cg::k_spmv_q<float, 1>", 2: "cg::k_spmv_q<__hip_bfloat16, 1>", 3: "cg::k_spmv_symx<1>"}[spmv_kind]
+    kname = {1: "cg::k_spmv_q<float, 1>", 2: "cg::k_spmv_q<__hip_bfloat16, 1>", 3: "cg::k_spmv_symj<1>"}[spmv_kind]
     pmc_path = os.path.join(ROOT, "profiles", "spmv_pmc_icestream1024.json")
     if args.n == 1024 and args.nz == 11 and os.path.exists(pmc_path):
         with open(pmc_path) as f:
             traffic = json.load(f)["kernels"].get(kname, {}).get("traffic_bytes")
     sp64_ms = sum(a for a, _ in sp64) / max(sum(b for _, b in sp64), 1)
-    coef64 = 56 * 8 if r64_kind == 4 else 108 * 8      # FP64 half (symmetric) or full rows
+    coef64 = 8 * 8 if r64_kind == 4 else 108 * 8       # FP64 element form (8 factors) or full rows
     ach64 = nodes * (coef64 + 4 * 8) / (sp64_ms * 1e-3) / 1e9
 
     # ---- BF16-storage variant of the mixed solve (same system, same tolerance)

@@ -120,8 +120,42 @@ __device__ __forceinline__ void ld_quad(const __hip_bfloat16* p, float& a, float
     e = __uint_as_float(q.y & 0xffff0000u);
 }
 
+// The sum of a node's 27 products (pairs: u and v row) in the one association
+// that every FP32 product uses, so that they agree bit for bit: the centre
+// and the upper couplings, then the lower ones, by rows of three along i.
+// The products round as fma(second, x_v, first * x_u).  term(m, y) adds
+// product m to y (nothing where there is none).
+__device__ __forceinline__ float2 prod2(float cuu, float cuv, float cvu, float cvv, float xu, float xv) {
+    return make_float2(__builtin_fmaf(cuv, xv, cuu * xu), __builtin_fmaf(cvv, xv, cvu * xu));
+}
+__device__ __forceinline__ float2 add2(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
+
+template <typename F>
+__device__ __forceinline__ float2 node_sum(F term) {
+    float2 y = make_float2(0.f, 0.f);
+    auto row = [&](int m) {
+        float2 g = make_float2(0.f, 0.f);
+        term(m, g);
+        term(m + 1, g);
+        term(m + 2, g);
+        y = add2(y, g);
+    };
+    term(13, y);
+    term(14, y);
+    row(15);
+    row(18);
+    row(21);
+    row(24);
+    term(12, y);
+    row(9);
+    row(0);
+    row(3);
+    row(6);
+    return y;
+}
+
 template <typename TA, int MODE>
-__global__ __launch_bounds__(256) void k_spmv_q(Dims d, const TA* __restrict__ A, const float* __restrict__ xu,
+__global__ __launch_bounds__(256, 5) void k_spmv_q(Dims d, const TA* __restrict__ A, const float* __restrict__ xu,
                                                 const float* __restrict__ xv, float* __restrict__ yu,
                                                 float* __restrict__ yv, const float* __restrict__ bu,
                                                 const float* __restrict__ bv, double* __restrict__ partials,
@@ -132,7 +166,7 @@ __global__ __launch_bounds__(256) void k_spmv_q(Dims d, const TA* __restrict__ A
     const int lane = threadIdx.x % WAVE;
     const int io = bx * WAVE + lane;
     const int jo = by * 4 + threadIdx.x / WAVE;
-    double acc = 0.0;     // per-column sum in FP64; the cross-column reduction is compensated
+    dd acc = {0.0, 0.0};
     if (io < d.nxo && jo < d.nyo) {
         const int i = d.ilo + io, j = d.jlo + jo;
         const long long pl = d.plane;
@@ -157,26 +191,25 @@ __global__ __launch_bounds__(256) void k_spmv_q(Dims d, const TA* __restrict__ A
             }
             const long long r = ((long long)k * d.nyo + jo) * d.nxp + io;
             const TA* a = A + (r / WAVE) * (27 * 4 * WAVE) + (r % WAVE) * 4;
-            float su = 0.f, sv = 0.f;
-#pragma unroll
-            for (int m = 0; m < 27; ++m) {
+            const float2 y = node_sum([&](int m, float2& g) {
                 float cuu, cuv, cvu, cvv;
                 ld_quad(a + m * (4 * WAVE), cuu, cuv, cvu, cvv);
-                const float xun = wu[m / 9][m % 9], xvn = wv[m / 9][m % 9];
-                su = su + cuu * xun + cuv * xvn;
-                sv = sv + cvu * xun + cvv * xvn;
-            }
+                g = add2(g, prod2(cuu, cuv, cvu, cvv, wu[m / 9][m % 9], wv[m / 9][m % 9]));
+            });
+            const float su = y.x, sv = y.y;
             const long long c0 = cb + (long long)(k + 1) * pl;
             if (MODE == 2) {
                 const float ru = bu[c0] - su, rv = bv[c0] - sv;
                 yu[c0] = ru;
                 yv[c0] = rv;
-                acc += (double)ru * (double)ru + (double)rv * (double)rv;
+                acc = dd_add_d(acc, (double)ru * (double)ru);
+                acc = dd_add_d(acc, (double)rv * (double)rv);
             } else {
                 yu[c0] = su;
                 yv[c0] = sv;
                 if (MODE == 1) {
-                    acc += (double)su * (double)wu[1][4] + (double)sv * (double)wv[1][4];
+                    acc = dd_add_d(acc, (double)su * (double)wu[1][4]);
+                    acc = dd_add_d(acc, (double)sv * (double)wv[1][4]);
                 }
             }
 #pragma unroll
@@ -187,7 +220,7 @@ __global__ __launch_bounds__(256) void k_spmv_q(Dims d, const TA* __restrict__ A
         }
     }
     if (MODE != 0) {
-        dd v[1] = {{acc, 0.0}};
+        dd v[1] = {acc};
         block_reduce_dd<1, 256>(v);
         if (threadIdx.x == 0) {
             const int lin = blockIdx.y * gridDim.x + blockIdx.x;

@@ -227,22 +227,37 @@ static bool elem_form_wanted() {
     return !(e && e[0] == '1');
 }
 
-// FP32 half storage: the kernel with the level-to-level LDS exchange of the
-// partner slots (default) or the one that re-reads them (CISMGPU_SPMV_SYMX=0)
-static bool use_symx() {
+// FP32 half storage: the marching kernel that reads every slot once needs a
+// tile and a share of rows for each CU to be worth its ghost rows, which is
+// where the levels are no longer split (level_split).
+// CISMGPU_SPMV_SYMX=0: the re-reading kernel always; 1: the marching one
+// wherever it can run.
+static bool use_symj(const Dims& d) {
     const char* e = getenv("CISMGPU_SPMV_SYMX");
-    return !(e && e[0] == '0');
+    if (!symj_fits(d)) return false;
+    if (e && (e[0] == '0' || e[0] == '1')) return e[0] == '1';
+    return level_shares(d) == 1;
 }
 
 template <int MODE>
 void spmv_sym32(cismgpu_system* S, const float* A, const float* xu, const float* xv, float* yu, float* yv,
                 const float* bu, const float* bv, double* part) {
-    // with the levels split there is no previous level to pass on
-    if (use_symx() && level_shares(S->d) == 1)
-        k_spmv_symx<MODE><<<spmv_blocks(S->d), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part);
-    else
-        k_spmv_sym<float, MODE><<<spmv_grid(S->d), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part,
-                                                                   level_split(S->d));
+    const Dims& d = S->d;
+    if (use_symj(d)) {
+        const SjCut c = symj_cut(d);
+        k_spmv_symj<MODE><<<dim3((d.nxp / WAVE) * c.nj, c.nk), WAVE * c.waves, symj_lds(c), S->s>>>(
+            d, A, xu, xv, yu, yv, bu, bv, part, c.jper, c.kper);
+    } else {
+        k_spmv_sym<float, MODE><<<spmv_grid(d), 256, 0, S->s>>>(d, A, xu, xv, yu, yv, bu, bv, part, level_split(d));
+    }
+}
+
+// partial sums of a low-precision product
+template <typename TA>
+int spmv32_parts(const cismgpu_system* S) {
+    const Dims& d = S->d;
+    if (S->two_d) return spmv_blocks(d);
+    return std::is_same<TA, float>::value && S->a32_sym && use_symj(d) ? symj_blocks(d) : spmv_parts(d);
 }
 
 template <typename TA, typename TV, int MODE>
@@ -612,7 +627,7 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
     TV *xu = v[0], *xv = v[1], *ru = v[2], *rv = v[3], *du = v[4], *dv = v[5], *qu = v[6], *qv = v[7];
     TV *zu = v[8], *zv = v[9], *Azu = v[10], *Azv = v[11];
     const TV* M = std::is_same<TV, double>::value ? (const TV*)S->M64 : (const TV*)S->M32;
-    const int nsp = std::is_same<TV, double>::value ? spmv64_parts(S) : S->two_d ? spmv_blocks(d) : spmv_parts(d);
+    const int nsp = std::is_same<TV, double>::value ? spmv64_parts(S) : spmv32_parts<TA>(S);
     const int nub = pre_parts(d, precond);
     const long long nv = d.vlen * sizeof(TV);
     // reprosum: the global sums of the FP64 solve are exact integer-vector
@@ -987,7 +1002,7 @@ static int32_t system_create(const cismgpu_grid* grid, bool two_d, cismgpu_syste
     if ((e = hipStreamCreateWithFlags(&S->s, hipStreamNonBlocking)) != hipSuccess) return fail(e, "stream");
     const long long n2 = (long long)d.nvx * d.nvy;
     const long long na = d.nrows * NCOEF;
-    const int nparts = std::max(std::max(spmv_parts(d), elem_parts(d)), std::max(std::max(upd_blocks(d), flat_blocks(d)), dot_blocks<double>(d))) + 8;
+    const int nparts = std::max(std::max(spmv_parts(d), std::max(elem_parts(d), symj_blocks(d))), std::max(std::max(upd_blocks(d), flat_blocks(d)), dot_blocks<double>(d))) + 8;
     if ((e = hipMalloc(&S->active, n2)) != hipSuccess) return fail(e, "active");
     if ((e = hipMalloc(&S->A64, na * sizeof(double))) != hipSuccess) return fail(e, "A64");
     if ((e = hipMalloc(&S->M64, 8 * d.vlen * sizeof(double))) != hipSuccess) return fail(e, "M64");

@@ -13,19 +13,12 @@
 // node instead of 432.
 //
 // k_spmv_sym walks a column up the levels like k_spmv_q and loads the 13
-// lower quads from the partner rows, the neighbouring columns of the same
-// level or of the previous level; k_spmv_symx (the default) takes the nine
-// previous-level quads from the tile's own threads through LDS and lane
-// shuffles instead (0.651 against 0.669 ms at 1024^2 x 11 on MI355X).  The
-// products are summed in the same order (m = 0..26) with the same values as
-// the full-storage kernel, so when the FP32 matrix is exactly symmetric
-// (k_check_sym finds no mismatch) all three kernels give identical results;
-// the solver uses this layout only then.  x is staged in LDS per 64 x 4
-// tile with a one-vertex ring: a 3-level ring of slots in k_spmv_sym and
-// k_spmv_sym64, a 4-level ring in k_spmv_symx (so that one barrier per
-// level less is needed).  A 3-level x window in registers instead cost 54
-// VGPRs and limited the kernel to 3 waves per SIMD (0.87 ms against 0.73 ms
-// at 1024^2 x 11).
+// lower quads from the partner rows; k_spmv_symj (large grids) forms both
+// products of a slot where it is read and passes the lower one on.  The
+// products and their association (node_sum) are those of the full-storage
+// kernel, so when the FP32 matrix is exactly symmetric (k_check_sym finds no
+// mismatch) all three kernels give identical results; the solver uses this
+// layout only then.  x is staged in LDS per tile with a one-vertex ring.
 //
 // Partner offsets within a level are 32-bit (po[] below): the half layouts
 // are used only while one level of slots, nyo * nxp * 56 elements, stays
@@ -111,7 +104,7 @@ __global__ void k_check_sym(Dims d, const double* __restrict__ A, unsigned long 
 __device__ __forceinline__ void ld_slot(const float* p, float& a, float& b, float& c, float& e) { ld_quad(p, a, b, c, e); }
 
 template <typename TA, int MODE>
-__global__ __launch_bounds__(256) void k_spmv_sym(Dims d, const TA* __restrict__ S, const float* __restrict__ xu,
+__global__ __launch_bounds__(256, 4) void k_spmv_sym(Dims d, const TA* __restrict__ S, const float* __restrict__ xu,
                                                   const float* __restrict__ xv, float* __restrict__ yu,
                                                   float* __restrict__ yv, const float* __restrict__ bu,
                                                   const float* __restrict__ bv, double* __restrict__ partials,
@@ -146,7 +139,7 @@ __global__ __launch_bounds__(256) void k_spmv_sym(Dims d, const TA* __restrict__
             xs[1][slot][r][c] = b;
         }
     };
-    double acc = 0.0;
+    dd acc = {0.0, 0.0};
     int po[9];
     const long long LS = (long long)d.nyo * d.nxp / WAVE * (NSLOT * 4 * WAVE);   // elements per level
     if (live) {
@@ -168,19 +161,14 @@ __global__ __launch_bounds__(256) void k_spmv_sym(Dims d, const TA* __restrict__
             const long long ck = vidx(d, k, d.ilo + io, d.jlo + jo);
             const TA* Sk = S + (long long)k * LS;     // level k
             const TA* Sb = Sk - LS;                   // level k - 1
-            float su = 0.f, sv = 0.f;
-#pragma unroll
-            for (int m = 0; m < 27; ++m) {
-                float cuu = 0.f, cuv = 0.f, cvu = 0.f, cvv = 0.f;
-                bool have = true;
+            const float2 y = node_sum([&](int m, float2& g) {
+                float cuu, cuv, cvu, cvv;
                 if (m < 13) {
                     const int h = m % 9;
-                    have = po[h] >= 0 && (m >= 9 || k > 0);
-                    if (have) {
-                        float a, b, c, e;
-                        ld_slot((m < 9 ? Sb : Sk) + po[h] + (13 - m) * (4 * WAVE), a, b, c, e);
-                        cuu = a; cuv = c; cvu = b; cvv = e;     // transposed 2x2 block
-                    }
+                    if (!(po[h] >= 0 && (m >= 9 || k > 0))) return;
+                    float a, b, c, e;
+                    ld_slot((m < 9 ? Sb : Sk) + po[h] + (13 - m) * (4 * WAVE), a, b, c, e);
+                    cuu = a; cuv = c; cvu = b; cvv = e;     // transposed 2x2 block
                 } else if (m == 13) {
                     float a, b, c, e;
                     ld_slot(Sk + po[4], a, b, c, e);
@@ -188,33 +176,31 @@ __global__ __launch_bounds__(256) void k_spmv_sym(Dims d, const TA* __restrict__
                 } else {
                     ld_slot(Sk + po[4] + (m - 13) * (4 * WAVE), cuu, cuv, cvu, cvv);
                 }
-                if (have) {
-                    const int slot = (k + m / 9) % 3;          // level k + kA lives in slot (k + kA + 1) % 3
-                    const int r = w + 1 + ((m / 3) % 3 - 1), c = lane + 1 + (m % 3 - 1);
-                    const float xun = xs[0][slot][r][c], xvn = xs[1][slot][r][c];
-                    su = su + cuu * xun + cuv * xvn;
-                    sv = sv + cvu * xun + cvv * xvn;
-                }
-            }
+                const int slot = (k + m / 9) % 3;              // level k + kA lives in slot (k + kA + 1) % 3
+                const int r = w + 1 + ((m / 3) % 3 - 1), c = lane + 1 + (m % 3 - 1);
+                g = add2(g, prod2(cuu, cuv, cvu, cvv, xs[0][slot][r][c], xs[1][slot][r][c]));
+            });
+            const float su = y.x, sv = y.y;
             if (MODE == 2) {
                 const float ru = bu[ck] - su, rv = bv[ck] - sv;
                 yu[ck] = ru;
                 yv[ck] = rv;
-                acc += (double)ru * (double)ru + (double)rv * (double)rv;
+                acc = dd_add_d(acc, (double)ru * (double)ru);
+                acc = dd_add_d(acc, (double)rv * (double)rv);
             } else {
                 yu[ck] = su;
                 yv[ck] = sv;
                 if (MODE == 1) {
                     const int slot = (k + 1) % 3;
-                    acc += (double)su * (double)xs[0][slot][w + 1][lane + 1] +
-                           (double)sv * (double)xs[1][slot][w + 1][lane + 1];
+                    acc = dd_add_d(acc, (double)su * (double)xs[0][slot][w + 1][lane + 1]);
+                    acc = dd_add_d(acc, (double)sv * (double)xs[1][slot][w + 1][lane + 1]);
                 }
             }
         }
         __syncthreads();   // the slot of level k-1 is restaged next
     }
     if (MODE != 0) {
-        dd v[1] = {{acc, 0.0}};
+        dd v[1] = {acc};
         block_reduce_dd<1, 256>(v);
         if (threadIdx.x == 0) {
             partials[2 * (blockIdx.y * nblk + lin) + 0] = v[0].hi;
@@ -223,186 +209,217 @@ __global__ __launch_bounds__(256) void k_spmv_sym(Dims d, const TA* __restrict__
     }
 }
 
-// FP32 half storage with a level-to-level exchange of the partner slots.
-// The lower couplings of row (k, i, j) to level k-1 (m = 0..8) are the
-// transposed slots 13 - m of the rows (k-1, i+iA, j+jA), which the tile's
-// own threads loaded one level earlier as their couplings to level k
-// (slots 5..13).  Instead of re-reading them (they fall out of L2 between
-// two levels: one level step of all resident tiles exceeds an XCD's 4 MB),
-// each thread keeps its slots 8, 9, 10 in registers for itself and its two
-// lane neighbours (cross-lane shuffles) and writes slots 5, 6, 7 and 11, 12,
-// 13 to LDS for the threads of the neighbouring tile rows; only partners
-// outside the 64 x 4 tile are read from memory.  The products are summed in
-// the order and with the values of k_spmv_sym, so the results are identical.
+// FP32 half storage, every slot read once.  A row's stored couplings serve two
+// rows: its own sum, and the transposed block in the sum of the row it couples
+// to.  Here the row that holds a slot forms both products and passes the two
+// numbers on, instead of the other row fetching the four again: k_spmv_sym
+// reads 4.1 GB a product at 1024^2 x 11, of 2.8 GB of slots and vectors.
+//
+// A workgroup takes 64 columns of a vertex row (lanes) on all levels (one
+// wavefront each, at most SJ_WAVES; deeper columns are cut into shares, whose
+// first wavefront recomputes the level above) and marches along j.  Products
+// for the neighbouring lanes go by shuffle, for the next vertex row they stay
+// in registers, for the level below they go through LDS (three pairs per lane
+// and step, two buffers, one barrier per step).  What remains to be read twice
+// are the columns next to the tile (five slots of one lane, four of another,
+// per row) and one ghost row before and after the march; the march before,
+// along the levels, re-read a tile's rim on every level.  A row waits one step
+// for the products of the next row on the level above.
+//
+// x of rows j-1 .. j+1 is in LDS, a ring of four rows.  Sums are associated as
+// in the other FP32 products (node_sum), so the results are the same bits.
+// Columns without a stored row (outside the owned region) hold zero slots; the
+// image of a periodic neighbour is read where the shuffle has another row.
+constexpr int SJ_WAVES = 12;
+
+struct SjCut { int nj, jper, nk, kper, waves; };   // shares along j and k; wavefronts per workgroup
+
+// 16 wavefronts with 128 registers fit a CU: the number of shares along j that
+// takes the fewest steps in all, with two ghost rows per share.
+inline SjCut symj_cut(const Dims& d) {
+    SjCut c{};
+    c.nk = d.nz <= SJ_WAVES ? 1 : (d.nz + SJ_WAVES - 2) / (SJ_WAVES - 1);
+    c.kper = (d.nz + c.nk - 1) / c.nk;
+    c.nk = (d.nz + c.kper - 1) / c.kper;
+    c.waves = c.kper + (c.nk > 1 ? 1 : 0);
+    const long long nb = (long long)(d.nxp / WAVE) * c.nk;
+    const int per_cu = 16 / c.waves;
+    long long best = -1;
+    for (int jper = d.nyo; jper >= 4 || jper == d.nyo; --jper) {
+        const int nj = (d.nyo + jper - 1) / jper;
+        const long long cost = (nb * nj + 256 * per_cu - 1) / (256 * per_cu) * (jper + 2);
+        if (best < 0 || cost < best) { best = cost; c.jper = jper; c.nj = nj; }
+        if (jper <= 1) break;
+    }
+    return c;
+}
+inline bool symj_fits(const Dims& d) { return (long long)d.nyo * d.nxp * NSLOT * 16 < (1LL << 31); }
+inline int symj_blocks(const Dims& d) { const SjCut c = symj_cut(d); return (d.nxp / WAVE) * c.nj * c.nk; }
+inline size_t symj_lds(const SjCut& c) {
+    return sizeof(float2) * (4 * (c.waves + 1) * (WAVE + 2) + 2 * 3 * c.waves * WAVE);
+}
+
 template <int MODE>
-__global__ __launch_bounds__(256) void k_spmv_symx(Dims d, const float* __restrict__ S, const float* __restrict__ xu,
-                                                   const float* __restrict__ xv, float* __restrict__ yu,
-                                                   float* __restrict__ yv, const float* __restrict__ bu,
-                                                   const float* __restrict__ bv, double* __restrict__ partials) {
-    __shared__ float xs[2][4][6][WAVE + 2];
-    // ex[q][c][w][lane]: q 0..2 slots 11, 12, 13 (read by tile row w + 1),
-    // q 3..5 slots 5, 6, 7 (read by tile row w - 1), of the previous level
-    __shared__ float ex[6][4][4][WAVE];
+__global__ __launch_bounds__(WAVE * SJ_WAVES) void k_spmv_symj(Dims d, const float* __restrict__ S,
+                                                               const float* __restrict__ xu, const float* __restrict__ xv,
+                                                               float* __restrict__ yu, float* __restrict__ yv,
+                                                               const float* __restrict__ bu, const float* __restrict__ bv,
+                                                               double* __restrict__ partials, int jper, int kper) {
+    extern __shared__ float2 sj_lds[];
+    const int nw = blockDim.x / WAVE;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
+    auto xs = [&](int q, int l, int c) -> float2& {       // row q (ring of 4), level index l, column c - 1 of the tile
+        return sj_lds[((q & 3) * (nw + 1) + l) * (WAVE + 2) + c];
+    };
+    float2* ex = sj_lds + 4 * (nw + 1) * (WAVE + 2);      // [2][3][nw][64]
     const int nbx = d.nxp / WAVE;
-    const int nblk = nbx * ((d.nyo + 3) / 4);
-    const int lin = xcd_remap(blockIdx.x, nblk);
-    const int bx = lin % nbx, by = lin / nbx;
-    const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
-    const int io = bx * WAVE + lane;
-    const int jo = by * 4 + w;
-    const bool live = io < d.nxo && jo < d.nyo;
-    const int i0 = d.ilo + bx * WAVE - 1, j0 = d.jlo + by * 4 - 1;
-    auto stage = [&](int kk) {
-        const int slot = (kk + 1) % 4;
-        for (int e = threadIdx.x; e < 6 * (WAVE + 2); e += 256) {
-            const int r = e / (WAVE + 2), c = e % (WAVE + 2);
-            const int vi = i0 + c, vj = j0 + r;
-            float a = 0.f, b = 0.f;
-            if (vi >= 1 && vi <= d.nvx && vj >= 1 && vj <= d.nvy) {
-                const long long n = vidx(d, kk, vi, vj);
-                a = xu[n];
-                b = xv[n];
+    const int lin = xcd_remap(blockIdx.x, gridDim.x);
+    const int bx = lin % nbx, jt = lin / nbx;
+    const int kc0 = blockIdx.y * kper, ghost = kc0 > 0 ? 1 : 0;
+    const int kend = min(d.nz, kc0 + kper);
+    const int k = kc0 - ghost + w;                        // level of this wavefront
+    const bool kon = k < kend;
+    const int io = bx * WAVE + lane, i = d.ilo + io;
+    const bool live = io < d.nxo && kon;
+    const int q0 = jt * jper, q1 = min(d.nyo, q0 + jper);
+    const bool edge_l = lane == 0, edge_r = lane == WAVE - 1;
+    const long long LS = (long long)d.nyo * d.nxp / WAVE * (NSLOT * 4 * WAVE);
+    const float* Sk = S + (long long)(kon ? k : 0) * LS;
+    // raw buffer over the level's slots (below 2 GiB, symj_fits): a load past
+    // it reads zero, which is what a row that is not stored holds
+    constexpr unsigned NONE = 0x80000000u;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)Sk, (short)0, (int)(LS * 4), 0x00020000);
+    auto offset = [&](int col) { return col < 0 ? NONE : (unsigned)((col / WAVE) * (NSLOT * 4 * WAVE) + (col % WAVE) * 4) * 4u; };
+    auto slot = [&](unsigned off, int s) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(rs, off, s * (4 * WAVE * 4), 0);
+        return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]));
+    };
+    float4 own[NSLOT], ed[5];
+    // slots of row q; of the ghost rows only those that couple into the share
+    auto load = [&](int q) {
+        // the lane past the last owned column holds the row beyond it, if there is one (periodic)
+        const unsigned o = offset(io <= d.nxo && kon ? partner_col(d, i, d.jlo + q) : -1);
+        const unsigned fwd = q >= q1 ? NONE : o, back = q < q0 ? NONE : o, both = q < q0 ? NONE : fwd;
+#pragma unroll
+        for (int s = 0; s < NSLOT; ++s)
+            own[s] = slot((s >= 2 && s <= 4) || s >= 11 ? fwd : s >= 5 && s <= 7 ? back : both, s);
+        // left: slots 1, 4, 7, 10, 13 of column i - 1 (coupling to i), right: 2, 5, 8, 11 of column i + 1
+        const unsigned oe = offset(live && (edge_l || edge_r) ? partner_col(d, edge_l ? i - 1 : i + 1, d.jlo + q) : -1);
+        const unsigned os = oe == NONE ? NONE : oe + (edge_l ? 1u : 2u) * (4 * WAVE * 4);
+#pragma unroll
+        for (int s = 0; s < 5; ++s) ed[s] = slot(s == 4 && !edge_l ? NONE : os, 3 * s);
+    };
+    const int nst = (nw + 1) * (WAVE + 2);
+    const int ci0 = d.ilo + bx * WAVE - 1, kl0 = kc0 - ghost;
+    auto stage = [&](int q) {              // x of row q, levels kl0 .. kl0 + nw
+        const int vj = d.jlo + q;
+        for (int e = threadIdx.x; e < nst; e += blockDim.x) {
+            const int l = e / (WAVE + 2), c = e % (WAVE + 2), vi = ci0 + c;
+            float2 v = make_float2(0.f, 0.f);
+            if (vi >= 1 && vi <= d.nvx && vj >= 1 && vj <= d.nvy && kl0 + l <= d.nz) {
+                const long long n = vidx(d, kl0 + l, vi, vj);
+                v = make_float2(xu[n], xv[n]);
             }
-            xs[0][slot][r][c] = a;
-            xs[1][slot][r][c] = b;
+            xs(q, l, c) = v;
         }
     };
-    double acc = 0.0;
-    int po[9];
-    unsigned inl = 0;   // bit h: partner h is the tile's own neighbouring thread
-    const long long LS = (long long)d.nyo * d.nxp / WAVE * (NSLOT * 4 * WAVE);
-    if (live) {
-        const int i = d.ilo + io, j = d.jlo + jo;
-#pragma unroll
-        for (int h = 0; h < 9; ++h) {
-            const int iA = h % 3 - 1, jA = h / 3 - 1;
-            const int pc = partner_col(d, i + iA, j + jA);
-            po[h] = pc < 0 ? -1 : (pc / WAVE) * (NSLOT * 4 * WAVE) + (pc % WAVE) * 4;
-            const int li = lane + iA, wj = w + jA;
-            if (pc >= 0 && li >= 0 && li < WAVE && wj >= 0 && wj < 4 && pc == (jo + jA) * d.nxp + (io + iA))
-                inl |= 1u << h;
+    auto prod = [](float cuu, float cuv, float cvu, float cvv, float2 x) { return prod2(cuu, cuv, cvu, cvv, x.x, x.y); };
+    auto up = [&](float2 v) { return make_float2(__shfl_up(v.x, 1, WAVE), __shfl_up(v.y, 1, WAVE)); };
+    auto down = [&](float2 v) { return make_float2(__shfl_down(v.x, 1, WAVE), __shfl_down(v.y, 1, WAVE)); };
+    dd acc = {0.0, 0.0};
+    float2 pend = make_float2(0.f, 0.f), xp = pend, Bp = pend, Ep = pend;
+    load(q0 - 1);
+    stage(q0 - 2);
+    stage(q0 - 1);
+    stage(q0);
+    __syncthreads();
+#pragma unroll 1
+    for (int q = q0 - 1; q <= q1; ++q) {
+        const float2 x0 = xs(q, w, lane + 1);
+        const float2 xl = xs(q, w, lane), xr = xs(q, w, lane + 2);
+        // own sum: centre and upper couplings
+        auto c = [&](int s, int r, int l, int di) {
+            return prod(own[s].x, own[s].y, own[s].z, own[s].w, xs(q + r, w + l, lane + 1 + di));
+        };
+        float2 U = prod(own[0].x, own[0].y, own[0].y, own[0].z, x0);
+        U = add2(U, prod(own[1].x, own[1].y, own[1].z, own[1].w, xr));
+        U = add2(U, add2(add2(c(2, 1, 0, -1), c(3, 1, 0, 0)), c(4, 1, 0, 1)));
+        U = add2(U, add2(add2(c(5, -1, 1, -1), c(6, -1, 1, 0)), c(7, -1, 1, 1)));
+        U = add2(U, add2(add2(c(8, 0, 1, -1), c(9, 0, 1, 0)), c(10, 0, 1, 1)));
+        U = add2(U, add2(add2(c(11, 1, 1, -1), c(12, 1, 1, 0)), c(13, 1, 1, 1)));
+        // transposed products for the rows these slots couple to
+        auto t = [&](float4 s, float2 x) { return prod(s.x, s.z, s.y, s.w, x); };
+        auto from_l = [&](int s, int e) {  // the column i - 1's product for this column
+            const float2 v = up(t(own[s], x0)), m = t(ed[e], xl);
+            return edge_l ? m : v;
+        };
+        auto from_r = [&](int s, int e) {  // the column i + 1's
+            const float2 v = down(t(own[s], x0)), m = t(ed[e], xr);
+            return edge_r ? m : v;
+        };
+        const float2 L = from_l(1, 0);
+        const float2 B = add2(add2(from_l(4, 1), t(own[3], x0)), from_r(2, 0));       // row j + 1, this level
+        const float2 C = add2(add2(from_l(7, 2), t(own[6], x0)), from_r(5, 1));       // row j - 1, level k + 1
+        const float2 D = add2(add2(from_l(10, 3), t(own[9], x0)), from_r(8, 2));      // row j, level k + 1
+        const float2 E = add2(add2(from_l(13, 4), t(own[12], x0)), from_r(11, 3));    // row j + 1, level k + 1
+        float2* out = ex + (q & 1) * 3 * nw * WAVE + w * WAVE + lane;
+        out[0] = C;
+        out[nw * WAVE] = D;
+        out[2 * nw * WAVE] = E;
+        // The next row's loads take over this row's registers, so this row's sums
+        // are fixed here: the compiler would sink what is used after the barrier
+        // below the loads, and spill the slots.
+        float2 V = add2(U, L);
+        asm volatile("" : "+v"(V.x), "+v"(V.y));
+        float2 Bn = B;
+        asm volatile("" : "+v"(Bn.x), "+v"(Bn.y));
+        __builtin_amdgcn_sched_barrier(0);
+        if (q < q1) {
+            load(q + 1);
+            stage(q + 2);
         }
-    }
-    float p8[4] = {0.f, 0.f, 0.f, 0.f}, p9[4] = {0.f, 0.f, 0.f, 0.f}, p10[4] = {0.f, 0.f, 0.f, 0.f};
-    stage(-1);
-    stage(0);
-    // x of level kk sits in ring slot (kk + 1) % 4.  stage(k + 1) overwrites
-    // level k - 3, last read in step k - 2; every thread is past the mid
-    // barrier of step k - 1 by then, so two barriers per level suffice.
-    for (int k = 0; k < d.nz; ++k) {
-        stage(k + 1);
-        __syncthreads();   // x of levels k-1..k+1 staged; ex holds level k-1
-        float l10[4], r8[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            l10[c] = __shfl_up(p10[c], 1, WAVE);     // slot 10 of lane - 1
-            r8[c] = __shfl_down(p8[c], 1, WAVE);     // slot 8 of lane + 1
+        __syncthreads();
+        float2 Ci = make_float2(0.f, 0.f), Di = Ci, Ei = Ci;
+        if (w > 0) {
+            const float2* in = ex + (q & 1) * 3 * nw * WAVE + (w - 1) * WAVE + lane;
+            Ci = in[0];
+            Di = in[nw * WAVE];
+            Ei = in[2 * nw * WAVE];
         }
-        float su = 0.f, sv = 0.f;
-        const float* Sk = S + (long long)k * LS;
-        const float* Sb = Sk - LS;
-        // this level's own slots and same-level partner slots, loaded before
-        // the level k-1 part so that they are in flight across the barrier
-        float own[NSLOT][4];
-        if (live) {
-#pragma unroll
-            for (int q = 0; q < NSLOT; ++q) ld_slot(Sk + po[4] + q * (4 * WAVE), own[q][0], own[q][1], own[q][2], own[q][3]);
-        }
-        if (live && k > 0) {
-#pragma unroll
-            for (int m = 0; m < 9; ++m) {   // level k-1: transposed slots 13 - m of the partners
-                if (po[m] < 0) continue;
-                float a, b, c, e;
-                if (inl & (1u << m)) {
-                    const int li = lane + m % 3 - 1;
-                    if (m == 4) {
-                        a = p9[0]; b = p9[1]; c = p9[2]; e = p9[3];
-                    } else if (m == 3) {
-                        a = l10[0]; b = l10[1]; c = l10[2]; e = l10[3];
-                    } else if (m == 5) {
-                        a = r8[0]; b = r8[1]; c = r8[2]; e = r8[3];
-                    } else if (m < 3) {     // row j-1 (wave w-1), slot 13 - m = 11 + (2 - m)
-                        const int q = 2 - m;
-                        a = ex[q][0][w - 1][li]; b = ex[q][1][w - 1][li];
-                        c = ex[q][2][w - 1][li]; e = ex[q][3][w - 1][li];
-                    } else {                // row j+1 (wave w+1), slot 13 - m = 5 + (8 - m)
-                        const int q = 3 + (8 - m);
-                        a = ex[q][0][w + 1][li]; b = ex[q][1][w + 1][li];
-                        c = ex[q][2][w + 1][li]; e = ex[q][3][w + 1][li];
-                    }
-                } else {
-                    ld_slot(Sb + po[m] + (13 - m) * (4 * WAVE), a, b, c, e);
-                }
-                const float cuu = a, cuv = c, cvu = b, cvv = e;     // transposed 2x2 block
-                const int slot = k % 4;                              // level k-1
-                const int r = w + 1 + ((m / 3) % 3 - 1), cc = lane + 1 + (m % 3 - 1);
-                const float xun = xs[0][slot][r][cc], xvn = xs[1][slot][r][cc];
-                su = su + cuu * xun + cuv * xvn;
-                sv = sv + cvu * xun + cvv * xvn;
-            }
-        }
-        __syncthreads();   // every read of ex (level k-1) is done
-        if (live) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-#pragma unroll
-                for (int q = 0; q < 3; ++q) {
-                    ex[q][c][w][lane] = own[11 + q][c];
-                    ex[3 + q][c][w][lane] = own[5 + q][c];
-                }
-                p8[c] = own[8][c];
-                p9[c] = own[9][c];
-                p10[c] = own[10][c];
-            }
-#pragma unroll
-            for (int m = 9; m < 27; ++m) {
-                float cuu, cuv, cvu, cvv;
-                bool have = true;
-                if (m < 13) {   // same level: transposed slots of the partners
-                    const int h = m % 9;
-                    have = po[h] >= 0;
-                    cuu = cuv = cvu = cvv = 0.f;
-                    if (have) {
-                        float a, b, c, e;
-                        ld_slot(Sk + po[h] + (13 - m) * (4 * WAVE), a, b, c, e);
-                        cuu = a; cuv = c; cvu = b; cvv = e;
-                    }
-                } else if (m == 13) {
-                    cuu = own[0][0]; cuv = own[0][1]; cvu = own[0][1]; cvv = own[0][2];
-                } else {
-                    cuu = own[m - 13][0]; cuv = own[m - 13][1]; cvu = own[m - 13][2]; cvv = own[m - 13][3];
-                }
-                if (have) {
-                    const int slot = (k + m / 9) % 4;
-                    const int r = w + 1 + ((m / 3) % 3 - 1), c = lane + 1 + (m % 3 - 1);
-                    const float xun = xs[0][slot][r][c], xvn = xs[1][slot][r][c];
-                    su = su + cuu * xun + cuv * xvn;
-                    sv = sv + cvu * xun + cvv * xvn;
-                }
-            }
-            const long long ck = vidx(d, k, d.ilo + io, d.jlo + jo);
+        if (q > q0 && live && w >= ghost) {               // row q - 1 is complete
+            const float2 y = add2(pend, Ci);
+            const long long ck = vidx(d, k, i, d.jlo + q - 1);
             if (MODE == 2) {
-                const float ru = bu[ck] - su, rv = bv[ck] - sv;
+                const float ru = bu[ck] - y.x, rv = bv[ck] - y.y;
                 yu[ck] = ru;
                 yv[ck] = rv;
-                acc += (double)ru * (double)ru + (double)rv * (double)rv;
+                acc = dd_add_d(acc, (double)ru * (double)ru);
+                acc = dd_add_d(acc, (double)rv * (double)rv);
             } else {
-                yu[ck] = su;
-                yv[ck] = sv;
+                yu[ck] = y.x;
+                yv[ck] = y.y;
                 if (MODE == 1) {
-                    const int slot = (k + 1) % 4;
-                    acc += (double)su * (double)xs[0][slot][w + 1][lane + 1] +
-                           (double)sv * (double)xs[1][slot][w + 1][lane + 1];
+                    acc = dd_add_d(acc, (double)y.x * (double)xp.x);
+                    acc = dd_add_d(acc, (double)y.y * (double)xp.y);
                 }
             }
         }
+        pend = add2(add2(add2(V, Bp), Ep), Di);
+        Bp = Bn;
+        Ep = Ei;
+        xp = x0;
     }
     if (MODE != 0) {
-        dd v[1] = {{acc, 0.0}};
-        block_reduce_dd<1, 256>(v);
+        // one sum over the wavefronts, in wavefront order
+        __shared__ dd sh[SJ_WAVES];
+        for (int off = WAVE / 2; off > 0; off >>= 1) acc = dd_add(acc, dd_shfl_down(acc, off));
+        if (lane == 0) sh[w] = acc;
+        __syncthreads();
         if (threadIdx.x == 0) {
-            partials[2 * lin + 0] = v[0].hi;
-            partials[2 * lin + 1] = v[0].lo;
+            for (int u = 1; u < nw; ++u) acc = dd_add(acc, sh[u]);
+            const int b = blockIdx.y * gridDim.x + lin;
+            partials[2 * b + 0] = acc.hi;
+            partials[2 * b + 1] = acc.lo;
         }
     }
 }
