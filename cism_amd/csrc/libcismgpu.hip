@@ -227,16 +227,16 @@ static bool elem_form_wanted() {
     return !(e && e[0] == '1');
 }
 
-// FP32 half storage: the marching kernel that reads every slot once needs a
-// tile and a share of rows for each CU to be worth its ghost rows, which is
-// where the levels are no longer split (level_split).
+// FP32 half storage: the marching kernel that reads every slot once pays for
+// its ghost rows and its serial march from about 160 tiles on (193^2 x 11, 196
+// tiles: 24.8 against 31.1 us; 128^2 x 7, 64 tiles: 15.3 against 9.3 us).
 // CISMGPU_SPMV_SYMX=0: the re-reading kernel always; 1: the marching one
 // wherever it can run.
 static bool use_symj(const Dims& d) {
     const char* e = getenv("CISMGPU_SPMV_SYMX");
     if (!symj_fits(d)) return false;
     if (e && (e[0] == '0' || e[0] == '1')) return e[0] == '1';
-    return level_shares(d) == 1;
+    return spmv_blocks(d) >= 160;
 }
 
 template <int MODE>

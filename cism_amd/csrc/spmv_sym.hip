@@ -226,6 +226,11 @@ __global__ __launch_bounds__(256, 4) void k_spmv_sym(Dims d, const TA* __restric
 // along the levels, re-read a tile's rim on every level.  A row waits one step
 // for the products of the next row on the level above.
 //
+// At 1024^2 x 11 a product takes 561 us (4.94 TB/s of slots and vectors)
+// against 691 us for k_spmv_sym and 651 us for the march along the levels that
+// this replaced; 571 us with all loads of a row issued after the last one's
+// products, 193^2 x 11 24.8 against 28.9 us.
+//
 // x of rows j-1 .. j+1 is in LDS, a ring of four rows.  Sums are associated as
 // in the other FP32 products (node_sum), so the results are the same bits.
 // Columns without a stored row (outside the owned region) hold zero slots; the
@@ -234,7 +239,7 @@ constexpr int SJ_WAVES = 12;
 
 struct SjCut { int nj, jper, nk, kper, waves; };   // shares along j and k; wavefronts per workgroup
 
-// 16 wavefronts with 128 registers fit a CU: the number of shares along j that
+// 12 wavefronts with 168 registers fit a CU: the number of shares along j that
 // takes the fewest steps in all, with two ghost rows per share.
 inline SjCut symj_cut(const Dims& d) {
     SjCut c{};
@@ -243,7 +248,7 @@ inline SjCut symj_cut(const Dims& d) {
     c.nk = (d.nz + c.kper - 1) / c.kper;
     c.waves = c.kper + (c.nk > 1 ? 1 : 0);
     const long long nb = (long long)(d.nxp / WAVE) * c.nk;
-    const int per_cu = 16 / c.waves;
+    const int per_cu = SJ_WAVES / c.waves;
     long long best = -1;
     for (int jper = d.nyo; jper >= 4 || jper == d.nyo; --jper) {
         const int nj = (d.nyo + jper - 1) / jper;
@@ -295,32 +300,44 @@ __global__ __launch_bounds__(WAVE * SJ_WAVES) void k_spmv_symj(Dims d, const flo
         return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]));
     };
     float4 own[NSLOT], ed[5];
-    // slots of row q; of the ghost rows only those that couple into the share
-    auto load = [&](int q) {
+    // Offsets of row q's slots (o*: the ghost rows give only the slots that
+    // couple into the share) and of the column next to the tile.
+    unsigned of = NONE, ob = NONE, oo = NONE, oe = NONE;
+    auto locate = [&](int q) {
         // the lane past the last owned column holds the row beyond it, if there is one (periodic)
-        const unsigned o = offset(io <= d.nxo && kon ? partner_col(d, i, d.jlo + q) : -1);
-        const unsigned fwd = q >= q1 ? NONE : o, back = q < q0 ? NONE : o, both = q < q0 ? NONE : fwd;
-#pragma unroll
-        for (int s = 0; s < NSLOT; ++s)
-            own[s] = slot((s >= 2 && s <= 4) || s >= 11 ? fwd : s >= 5 && s <= 7 ? back : both, s);
+        const unsigned o = offset(io <= d.nxo && kon && q <= q1 ? partner_col(d, i, d.jlo + q) : -1);
+        of = q >= q1 ? NONE : o;
+        ob = q < q0 ? NONE : o;
+        oo = q < q0 ? NONE : of;
         // left: slots 1, 4, 7, 10, 13 of column i - 1 (coupling to i), right: 2, 5, 8, 11 of column i + 1
-        const unsigned oe = offset(live && (edge_l || edge_r) ? partner_col(d, edge_l ? i - 1 : i + 1, d.jlo + q) : -1);
-        const unsigned os = oe == NONE ? NONE : oe + (edge_l ? 1u : 2u) * (4 * WAVE * 4);
-#pragma unroll
-        for (int s = 0; s < 5; ++s) ed[s] = slot(s == 4 && !edge_l ? NONE : os, 3 * s);
+        const int ec = live && (edge_l || edge_r) && q <= q1 ? partner_col(d, edge_l ? i - 1 : i + 1, d.jlo + q) : -1;
+        oe = ec < 0 ? NONE : offset(ec) + (edge_l ? 1u : 2u) * (4 * WAVE * 4);
     };
+    auto refill = [&](int s) { own[s] = slot((s >= 2 && s <= 4) || s >= 11 ? of : s >= 5 && s <= 7 ? ob : oo, s); };
+    auto refill_edge = [&](int e) { ed[e] = slot(e == 4 && !edge_l ? NONE : oe, 3 * e); };
+    // x of row q, levels kl0 .. kl0 + nw, into LDS: at most XST values a thread
+    constexpr int XST = 2;                 // (nw + 1) * 66 <= 2 * 64 * nw from two wavefronts on
     const int nst = (nw + 1) * (WAVE + 2);
     const int ci0 = d.ilo + bx * WAVE - 1, kl0 = kc0 - ghost;
-    auto stage = [&](int q) {              // x of row q, levels kl0 .. kl0 + nw
+    float2 xr_[XST];
+    auto fetch = [&](int q) {
         const int vj = d.jlo + q;
-        for (int e = threadIdx.x; e < nst; e += blockDim.x) {
+#pragma unroll
+        for (int u = 0; u < XST; ++u) {
+            const int e = threadIdx.x + u * blockDim.x;
             const int l = e / (WAVE + 2), c = e % (WAVE + 2), vi = ci0 + c;
-            float2 v = make_float2(0.f, 0.f);
-            if (vi >= 1 && vi <= d.nvx && vj >= 1 && vj <= d.nvy && kl0 + l <= d.nz) {
+            xr_[u] = make_float2(0.f, 0.f);
+            if (e < nst && vi >= 1 && vi <= d.nvx && vj >= 1 && vj <= d.nvy && kl0 + l <= d.nz) {
                 const long long n = vidx(d, kl0 + l, vi, vj);
-                v = make_float2(xu[n], xv[n]);
+                xr_[u] = make_float2(xu[n], xv[n]);
             }
-            xs(q, l, c) = v;
+        }
+    };
+    auto put = [&](int q) {
+#pragma unroll
+        for (int u = 0; u < XST; ++u) {
+            const int e = threadIdx.x + u * blockDim.x;
+            if (e < nst) xs(q, e / (WAVE + 2), e % (WAVE + 2)) = xr_[u];
         }
     };
     auto prod = [](float cuu, float cuv, float cvu, float cvv, float2 x) { return prod2(cuu, cuv, cvu, cvv, x.x, x.y); };
@@ -328,27 +345,33 @@ __global__ __launch_bounds__(WAVE * SJ_WAVES) void k_spmv_symj(Dims d, const flo
     auto down = [&](float2 v) { return make_float2(__shfl_down(v.x, 1, WAVE), __shfl_down(v.y, 1, WAVE)); };
     dd acc = {0.0, 0.0};
     float2 pend = make_float2(0.f, 0.f), xp = pend, Bp = pend, Ep = pend;
-    load(q0 - 1);
-    stage(q0 - 2);
-    stage(q0 - 1);
-    stage(q0);
+    for (int q = q0 - 2; q <= q0; ++q) {
+        fetch(q);
+        put(q);
+    }
+    locate(q0 - 1);
+#pragma unroll
+    for (int s = 0; s < NSLOT; ++s) refill(s);
+#pragma unroll
+    for (int e = 0; e < 5; ++e) refill_edge(e);
     __syncthreads();
+    // Each group of slots is refilled with the next row's as soon as its
+    // products are fixed, so loads are under way through the whole step; the
+    // x row, whose LDS write must not wait for them, is fetched before.  The
+    // barriers keep the compiler from moving the products below the loads
+    // (and spilling the slots).
+#define SJ_FIX(v) asm volatile("" : "+v"(v.x), "+v"(v.y))
+#define SJ_FENCE __builtin_amdgcn_sched_barrier(0)
 #pragma unroll 1
     for (int q = q0 - 1; q <= q1; ++q) {
+        fetch(q + 2);
+        locate(q + 1);
         const float2 x0 = xs(q, w, lane + 1);
         const float2 xl = xs(q, w, lane), xr = xs(q, w, lane + 2);
-        // own sum: centre and upper couplings
-        auto c = [&](int s, int r, int l, int di) {
+        auto c = [&](int s, int r, int l, int di) {        // own product
             return prod(own[s].x, own[s].y, own[s].z, own[s].w, xs(q + r, w + l, lane + 1 + di));
         };
-        float2 U = prod(own[0].x, own[0].y, own[0].y, own[0].z, x0);
-        U = add2(U, prod(own[1].x, own[1].y, own[1].z, own[1].w, xr));
-        U = add2(U, add2(add2(c(2, 1, 0, -1), c(3, 1, 0, 0)), c(4, 1, 0, 1)));
-        U = add2(U, add2(add2(c(5, -1, 1, -1), c(6, -1, 1, 0)), c(7, -1, 1, 1)));
-        U = add2(U, add2(add2(c(8, 0, 1, -1), c(9, 0, 1, 0)), c(10, 0, 1, 1)));
-        U = add2(U, add2(add2(c(11, 1, 1, -1), c(12, 1, 1, 0)), c(13, 1, 1, 1)));
-        // transposed products for the rows these slots couple to
-        auto t = [&](float4 s, float2 x) { return prod(s.x, s.z, s.y, s.w, x); };
+        auto t = [&](float4 s, float2 x) { return prod(s.x, s.z, s.y, s.w, x); };   // transposed
         auto from_l = [&](int s, int e) {  // the column i - 1's product for this column
             const float2 v = up(t(own[s], x0)), m = t(ed[e], xl);
             return edge_l ? m : v;
@@ -357,27 +380,42 @@ __global__ __launch_bounds__(WAVE * SJ_WAVES) void k_spmv_symj(Dims d, const flo
             const float2 v = down(t(own[s], x0)), m = t(ed[e], xr);
             return edge_r ? m : v;
         };
-        const float2 L = from_l(1, 0);
-        const float2 B = add2(add2(from_l(4, 1), t(own[3], x0)), from_r(2, 0));       // row j + 1, this level
-        const float2 C = add2(add2(from_l(7, 2), t(own[6], x0)), from_r(5, 1));       // row j - 1, level k + 1
-        const float2 D = add2(add2(from_l(10, 3), t(own[9], x0)), from_r(8, 2));      // row j, level k + 1
-        const float2 E = add2(add2(from_l(13, 4), t(own[12], x0)), from_r(11, 3));    // row j + 1, level k + 1
+        float2 U = prod(own[0].x, own[0].y, own[0].y, own[0].z, x0);
+        U = add2(U, prod(own[1].x, own[1].y, own[1].z, own[1].w, xr));
+        float2 L = from_l(1, 0);
+        SJ_FIX(U); SJ_FIX(L); SJ_FENCE;
+        refill(0); refill(1);
+        SJ_FENCE;
+        // row j + 1, this level
+        U = add2(U, add2(add2(c(2, 1, 0, -1), c(3, 1, 0, 0)), c(4, 1, 0, 1)));
+        float2 B = add2(add2(from_l(4, 1), t(own[3], x0)), from_r(2, 0));
+        SJ_FIX(U); SJ_FIX(B); SJ_FENCE;
+        refill(2); refill(3); refill(4); refill_edge(0);
+        SJ_FENCE;
+        // row j - 1, level k + 1
+        U = add2(U, add2(add2(c(5, -1, 1, -1), c(6, -1, 1, 0)), c(7, -1, 1, 1)));
+        float2 C = add2(add2(from_l(7, 2), t(own[6], x0)), from_r(5, 1));
+        SJ_FIX(U); SJ_FIX(C); SJ_FENCE;
+        refill(5); refill(6); refill(7); refill_edge(1);
+        SJ_FENCE;
+        // row j, level k + 1
+        U = add2(U, add2(add2(c(8, 0, 1, -1), c(9, 0, 1, 0)), c(10, 0, 1, 1)));
+        float2 D = add2(add2(from_l(10, 3), t(own[9], x0)), from_r(8, 2));
+        SJ_FIX(U); SJ_FIX(D); SJ_FENCE;
+        refill(8); refill(9); refill(10); refill_edge(2);
+        SJ_FENCE;
+        // row j + 1, level k + 1
+        U = add2(U, add2(add2(c(11, 1, 1, -1), c(12, 1, 1, 0)), c(13, 1, 1, 1)));
+        float2 E = add2(add2(from_l(13, 4), t(own[12], x0)), from_r(11, 3));
+        const float2 V = add2(U, L);
+        SJ_FIX(U); SJ_FIX(E); SJ_FENCE;
+        refill(11); refill(12); refill(13); refill_edge(3); refill_edge(4);
+        SJ_FENCE;
         float2* out = ex + (q & 1) * 3 * nw * WAVE + w * WAVE + lane;
         out[0] = C;
         out[nw * WAVE] = D;
         out[2 * nw * WAVE] = E;
-        // The next row's loads take over this row's registers, so this row's sums
-        // are fixed here: the compiler would sink what is used after the barrier
-        // below the loads, and spill the slots.
-        float2 V = add2(U, L);
-        asm volatile("" : "+v"(V.x), "+v"(V.y));
-        float2 Bn = B;
-        asm volatile("" : "+v"(Bn.x), "+v"(Bn.y));
-        __builtin_amdgcn_sched_barrier(0);
-        if (q < q1) {
-            load(q + 1);
-            stage(q + 2);
-        }
+        put(q + 2);
         __syncthreads();
         float2 Ci = make_float2(0.f, 0.f), Di = Ci, Ei = Ci;
         if (w > 0) {
@@ -405,10 +443,12 @@ __global__ __launch_bounds__(WAVE * SJ_WAVES) void k_spmv_symj(Dims d, const flo
             }
         }
         pend = add2(add2(add2(V, Bp), Ep), Di);
-        Bp = Bn;
+        Bp = B;
         Ep = Ei;
         xp = x0;
     }
+#undef SJ_FIX
+#undef SJ_FENCE
     if (MODE != 0) {
         // one sum over the wavefronts, in wavefront order
         __shared__ dd sh[SJ_WAVES];
