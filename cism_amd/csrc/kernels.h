@@ -48,7 +48,7 @@ template <typename TV>
 __global__ void k_first_update(Dims d, const double* scal, TV* xu, TV* xv, TV* ru, TV* rv, const TV* du,
                                const TV* dv, const TV* qu, const TV* qv);
 __global__ void k_scalars(int stage, const double* pa, int na, int sa, const double* pb, int nb, int sb,
-                          double* scal, double tolerance, double* mirror, double seq);
+                          double* scal, double tolerance, unsigned long long* mirror, unsigned long long seq);
 template <typename TA>
 __global__ void k_pack_matrix(Dims d, int blk, const double* src, const int8_t* active, TA* dst);
 template <typename TA>

@@ -74,8 +74,8 @@ struct cismgpu_system {
     double* scal = nullptr;
     double* scal_alt = nullptr;    // the same for the scalars; both halves of scal_buf
     double* scal_buf = nullptr;
-    double* scal_h = nullptr;      // pinned mirror, then the sequence number of its last fill
-    double scal_seq = 0.0;
+    double* scal_h = nullptr;      // pinned copy of the scalars, then the three words of a check (k_scalars)
+    unsigned long long scal_seq = 0;
     int zw = 0;                    // halo width that the next products store as zero (Dims::zw)
     TriPC tri;
     // assembly inputs on the device
@@ -357,28 +357,37 @@ void launch_precond(cismgpu_system* S, int kind, const TV* ru, const TV* rv, TV*
 
 void scalars(cismgpu_system* S, int stage, const double* pa, int na, int sa, const double* pb, int nb, int sb,
              double tol = 0.0) {
-    k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(stage, pa, na, sa, pb, nb, sb, S->scal, tol, nullptr, 0.0);
+    k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(stage, pa, na, sa, pb, nb, sb, S->scal, tol, nullptr, 0);
 }
 
-// The same, and wait until the scalars are in scal_h: the kernel writes them
-// there itself and the host polls for the sequence number, so a check costs
-// neither a copy launch nor the wake-up of a blocked thread.  With the halo
-// and ring launches that change nothing left out, the 31^2 x 10 dome drop-in
-// (110 iterations, 22 checks) went from 6.7 to 5.6 ms.  The stream is asked
-// now and then, so that a failed launch ends the wait.
+int sync_scal(cismgpu_system* S);
+
+// The same, and wait for the error and the flags of the check in scal_h: the
+// kernel writes them to host memory itself and the host polls, so a check
+// costs neither a copy launch nor the wake-up of a blocked thread.  With the
+// halo and ring launches that change nothing left out, the 31^2 x 10 dome
+// drop-in (110 iterations, 22 checks) went from 6.7 to 5.6 ms.  The stream is
+// asked now and then, so that a failed launch ends the wait.
 int scalars_to_host(cismgpu_system* S, int stage, const double* pa, int na, int sa, double tol) {
-    S->scal_seq += 1.0;
-    k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(stage, pa, na, sa, nullptr, 0, 0, S->scal, tol, S->scal_h, S->scal_seq);
+    unsigned long long* m = (unsigned long long*)(S->scal_h + S_NSLOTS);
+    const unsigned long long seq = ++S->scal_seq;
+    k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(stage, pa, na, sa, nullptr, 0, 0, S->scal, tol, m, seq);
     CG_CHECK(hipGetLastError());
-    double* flag = S->scal_h + S_NSLOTS;
-    double seen = 0.0;
+    auto arrived = [&]() {
+        const unsigned long long code = __atomic_load_n(m + 1, __ATOMIC_ACQUIRE);
+        if (code / 4 != seq) return false;
+        const unsigned long long err = __atomic_load_n(m, __ATOMIC_RELAXED);
+        if ((err ^ code) != __atomic_load_n(m + 2, __ATOMIC_RELAXED)) return false;
+        memcpy(S->scal_h + S_ERR, &err, sizeof(err));
+        S->scal_h[S_CONV] = code & 1 ? 1.0 : 0.0;
+        S->scal_h[S_NAN] = code & 2 ? 1.0 : 0.0;
+        return true;
+    };
     for (unsigned n = 1;; ++n) {
-        __atomic_load(flag, &seen, __ATOMIC_ACQUIRE);
-        if (seen == S->scal_seq) return CISMGPU_OK;
+        if (arrived()) return CISMGPU_OK;
         if (n % 8192 == 0 && hipStreamQuery(S->s) != hipErrorNotReady) break;
     }
-    CG_CHECK(hipStreamSynchronize(S->s));
-    return CISMGPU_OK;
+    return sync_scal(S);
 }
 
 // The zeroing halo rule changes nothing in a vector that is zero outside the
@@ -917,9 +926,9 @@ int mixed_solve(cismgpu_system* S, const cismgpu_solve_opts* o, cismgpu_solve_in
         k_ring<double><<<col_blocks(d), 256, 0, S->s>>>(d, ru, rv, bu, bv);
         if (S->repro) {
             rs_dot<double>(S, 3, ru, ru, rv, rv);
-            k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->rs_out + 6, 1, 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0.0);
+            k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->rs_out + 6, 1, 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0);
         } else {
-            k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->partB, nsp, 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0.0);
+            k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->partB, nsp, 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0);
         }
         st = sync_scal(S);
         if (st) return st;
@@ -1015,8 +1024,8 @@ static int32_t system_create(const cismgpu_grid* grid, bool two_d, cismgpu_syste
     if ((e = hipMalloc(&S->scal_buf, 2 * S_NSLOTS * sizeof(double))) != hipSuccess) return fail(e, "scal");
     S->scal = S->scal_buf;
     S->scal_alt = S->scal_buf + S_NSLOTS;
-    if ((e = hipHostMalloc(&S->scal_h, (S_NSLOTS + 1) * sizeof(double), hipHostMallocCoherent)) != hipSuccess) return fail(e, "scal_h");
-    S->scal_h[S_NSLOTS] = 0.0;
+    if ((e = hipHostMalloc(&S->scal_h, (S_NSLOTS + 3) * sizeof(double), hipHostMallocCoherent)) != hipSuccess) return fail(e, "scal_h");
+    memset(S->scal_h, 0, (S_NSLOTS + 3) * sizeof(double));
     S->repro = grid->reprosum != 0;
     if (S->repro) {
         if ((e = hipMalloc(&S->rs_part, (size_t)RS_MAX_BLOCKS * RS_L * sizeof(unsigned long long))) != hipSuccess)
@@ -2482,13 +2491,13 @@ extern "C" int32_t cismgpu_system_residual(cismgpu_system* S, double* ru, double
     S->elem_use = false;
     if (S->repro) {
         rs_dot<double>(S, 3, r0, r0, r1, r1);
-        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->rs_out + 6, 1, 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0.0);
+        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->rs_out + 6, 1, 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0);
         rs_dot<double>(S, 0, S->V(2), S->V(2), S->V(3), S->V(3));
-        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_BB, S->rs_out, 1, 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0.0);
+        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_BB, S->rs_out, 1, 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0);
     } else {
-        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->partB, nsp, 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0.0);
+        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_DOT, S->partB, nsp, 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0);
         k_dot<double><<<dot_blocks<double>(d), 256, 0, S->s>>>(d, S->V(2), S->V(2), S->V(3), S->V(3), S->partA);
-        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_BB, S->partA, dot_blocks<double>(d), 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0.0);
+        k_scalars<<<1, SCAL_THREADS, 0, S->s>>>(ST_BB, S->partA, dot_blocks<double>(d), 2, nullptr, 0, 0, S->scal, 0.0, nullptr, 0);
     }
     int st = sync_scal(S);
     if (st) return st;
