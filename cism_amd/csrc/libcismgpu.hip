@@ -27,6 +27,8 @@
 
 using namespace cg;
 
+#include "host_copy.hip"
+
 static thread_local char g_err[1024] = "";
 extern "C" void cismgpu_set_error(const char* fmt, ...) {
     va_list ap;
@@ -111,6 +113,7 @@ struct cismgpu_system {
     bool a32_sym = false;        // FP32 copy in half (symmetric) storage
     double* A64h = nullptr;      // FP64 half (symmetric) storage, when the FP64 matrix is exactly symmetric
     bool a64h_ready = false, a64_sym = false;
+    HostPipe pipe;                 // pinned slots of large host copies
     std::vector<hipEvent_t> ev;    // SpMV timing events (pairs)
     int ev_used = 0;
     bool timing = false;
@@ -1065,6 +1068,7 @@ int32_t cismgpu_system_destroy(cismgpu_system* S) {
                     (void*)S->rs_out, (void*)S->elemq, (void*)S->elem_bd, S->cb_buf})
         if (p) hipFree(p);
     if (S->scal_h) hipHostFree(S->scal_h);
+    S->pipe.close();
     for (auto& x : S->ev) hipEventDestroy(x);
     if (S->s) hipStreamDestroy(S->s);
     delete S;
@@ -1198,11 +1202,12 @@ int32_t cismgpu_system_set_x(cismgpu_system* S, const double* xu, const double* 
     const long long nvec = (long long)d.nz * d.nvx * d.nvy;
     double* tmp = S->V(12);
     CG_CHECK(hipMemsetAsync(S->V(0), 0, 2 * d.vlen * sizeof(double), S->s));
+    double* tmp2 = S->V(13);
     CG_CHECK(hipMemcpyAsync(tmp, xu, nvec * sizeof(double), hipMemcpyHostToDevice, S->s));
+    CG_CHECK(hipMemcpyAsync(tmp2, xv, nvec * sizeof(double), hipMemcpyHostToDevice, S->s));
     k_vec_in<double, double><<<nblocks(nvec, 256), 256, 0, S->s>>>(d, tmp, S->V(0));
-    CG_CHECK(hipMemcpyAsync(tmp, xv, nvec * sizeof(double), hipMemcpyHostToDevice, S->s));
-    k_vec_in<double, double><<<nblocks(nvec, 256), 256, 0, S->s>>>(d, tmp, S->V(1));
-    CG_CHECK(hipMemsetAsync(tmp, 0, d.vlen * sizeof(double), S->s));
+    k_vec_in<double, double><<<nblocks(nvec, 256), 256, 0, S->s>>>(d, tmp2, S->V(1));
+    CG_CHECK(hipMemsetAsync(tmp, 0, 2 * d.vlen * sizeof(double), S->s));
     CG_CHECK(hipStreamSynchronize(S->s));
     return CISMGPU_OK;
 }
@@ -1211,14 +1216,13 @@ int32_t cismgpu_system_get_x(cismgpu_system* S, double* xu, double* xv) {
     if (!S || !xu || !xv) return CISMGPU_ERR_ARG;
     const Dims& d = S->d;
     const long long nvec = (long long)d.nz * d.nvx * d.nvy;
-    double* tmp = S->V(12);
+    double *tmp = S->V(12), *tmp2 = S->V(13);
     k_vec_out<double, double><<<nblocks(nvec, 256), 256, 0, S->s>>>(d, S->V(0), tmp);
-    CG_CHECK(hipMemcpyAsync(xu, tmp, nvec * sizeof(double), hipMemcpyDeviceToHost, S->s));
-    CG_CHECK(hipStreamSynchronize(S->s));
-    k_vec_out<double, double><<<nblocks(nvec, 256), 256, 0, S->s>>>(d, S->V(1), tmp);
-    CG_CHECK(hipMemcpyAsync(xv, tmp, nvec * sizeof(double), hipMemcpyDeviceToHost, S->s));
-    CG_CHECK(hipStreamSynchronize(S->s));
-    CG_CHECK(hipMemsetAsync(tmp, 0, d.vlen * sizeof(double), S->s));
+    k_vec_out<double, double><<<nblocks(nvec, 256), 256, 0, S->s>>>(d, S->V(1), tmp2);
+    const size_t nb = nvec * sizeof(double);
+    const int st = host_copy(S->pipe, S->s, {{xu, tmp, nb}, {xv, tmp2, nb}});
+    if (st) return st;
+    CG_CHECK(hipMemsetAsync(tmp, 0, 2 * d.vlen * sizeof(double), S->s));
     return CISMGPU_OK;
 }
 
@@ -2323,15 +2327,17 @@ extern "C" int32_t cismgpu_system_internal_stress(cismgpu_system* S, double* tau
     k_internal_stress<<<nblocks(nfl, 128), 128, 0, S->s>>>(d, S->asm_in, 2, 0, S->V(0), S->V(1), nullptr, tau);
     double* out[6] = {tau_xz, tau_yz, tau_xx, tau_yy, tau_xy, tau_eff};
     hipError_t e = hipGetLastError();
-    for (int q = 0; q < 6 && e == hipSuccess; ++q)
-        if (out[q]) e = hipMemcpyAsync(out[q], tau + q * nfl, nfl * sizeof(double), hipMemcpyDeviceToHost, S->s);
-    if (e == hipSuccess) e = hipStreamSynchronize(S->s);
+    std::vector<HostSeg> segs;
+    for (int q = 0; q < 6; ++q)
+        if (out[q]) segs.push_back({out[q], tau + q * nfl, nfl * sizeof(double)});
+    int st = CISMGPU_OK;
+    if (e == hipSuccess) st = host_copy(S->pipe, S->s, segs);
     hipFree(tau);
     if (e != hipSuccess) {
         cismgpu_set_error("internal_stress: %s", hipGetErrorString(e));
         return CISMGPU_ERR_HIP;
     }
-    return CISMGPU_OK;
+    return st;
 }
 
 extern "C" int32_t cismgpu_system_internal_stress_2d(cismgpu_system* S, const double* uvel, const double* vvel,
@@ -2375,15 +2381,17 @@ extern "C" int32_t cismgpu_system_internal_stress_2d(cismgpu_system* S, const do
         e = hipGetLastError();
     }
     double* out[6] = {tau_xz, tau_yz, tau_xx, tau_yy, tau_xy, tau_eff};
-    for (int q = 0; q < 6 && e == hipSuccess; ++q)
-        if (out[q]) e = hipMemcpyAsync(out[q], tau + q * nfl, nfl * sizeof(double), hipMemcpyDeviceToHost, S->s);
-    if (e == hipSuccess) e = hipStreamSynchronize(S->s);
+    std::vector<HostSeg> segs;
+    for (int q = 0; q < 6; ++q)
+        if (out[q]) segs.push_back({out[q], tau + q * nfl, nfl * sizeof(double)});
+    int st = CISMGPU_OK;
+    if (e == hipSuccess) st = host_copy(S->pipe, S->s, segs);
     hipFree(buf);
     if (e != hipSuccess) {
         cismgpu_set_error("internal_stress_2d: %s", hipGetErrorString(e));
         return CISMGPU_ERR_HIP;
     }
-    return CISMGPU_OK;
+    return st;
 }
 
 extern "C" int32_t cismgpu_system_basal_friction(cismgpu_system* S, int32_t which_bfric, const double* ubas,
@@ -2469,9 +2477,7 @@ extern "C" int32_t cismgpu_system_get_efvs(cismgpu_system* S, double* efvs) {
     if (!S || !S->efvs || !efvs) return CISMGPU_ERR_ARG;
     const int nzl = S->two_d ? S->nz_levels : S->d.nz;
     const long long nfl = (long long)(nzl - 1) * S->d.nx * S->d.ny;
-    CG_CHECK(hipMemcpyAsync(efvs, S->efvs, nfl * sizeof(double), hipMemcpyDeviceToHost, S->s));
-    CG_CHECK(hipStreamSynchronize(S->s));
-    return CISMGPU_OK;
+    return host_copy(S->pipe, S->s, {{efvs, S->efvs, nfl * sizeof(double)}});
 }
 
 extern "C" int32_t cismgpu_system_residual(cismgpu_system* S, double* ru, double* rv, double* L2, double* L2rel) {
