@@ -1,15 +1,15 @@
-// host_copy.hip -- large copies from device memory to a caller's pageable
+// host_copy.hip -- large copies between device memory and a caller's pageable
 // host memory.
 //
 // The runtime moves them through one bounce buffer with one host thread, which
-// also takes the page faults of a fresh destination: about 10 GB/s, a fifth
-// of the link.  Here HC_THREADS threads each own two pinned slots and take
-// every HC_THREADS-th chunk, one slot on the link while the other is copied
-// on the host.  Below HC_MIN bytes the threads cost more than they save and
-// the runtime's copy is used.  185 MB of velocities: 18.7 -> 5.7 ms (33 GB/s);
-// 9.6 ms with 512 KiB chunks and eight threads, which wait on the runtime's
-// locks; 4 MiB or eight threads of 2 MiB gain nothing.  (Upward the runtime
-// reaches 28 GB/s, and this way 21: those copies stay with it.)
+// on the way down also takes the page faults of a fresh destination: about
+// 10 GB/s, a fifth of the link, and 28 GB/s on the way up.  Here HC_THREADS
+// threads each own two pinned slots and take every HC_THREADS-th chunk, one
+// slot on the link while the other is copied on the host.  Below HC_MIN bytes
+// the threads cost more than they save and the runtime's copy is used.
+// 185 MB of velocities: down 18.7 -> 5.7 ms (33 GB/s), up 6.6 -> 4.9 ms; 9.6
+// and 8.9 ms with 512 KiB chunks and eight threads, which wait on the runtime's
+// locks; 4 MiB or eight threads of 2 MiB gain nothing.
 #include <atomic>
 #include <cstring>
 #include <system_error>
@@ -24,7 +24,7 @@ constexpr size_t HC_CHUNK = 2 << 20;
 constexpr size_t HC_MIN = 6 << 20;
 constexpr int HC_THREADS = 4;
 
-struct HostSeg { void* host; const void* dev; size_t n; };
+struct HostSeg { void* host; const void* dev; size_t n; };   // dev is written to on the way up
 
 // The pinned slots of one system (16 MiB), made by its first large copy.
 struct HostPipe {
@@ -46,23 +46,25 @@ struct HostPipe {
     }
 };
 
-// Copies the segments to host memory, ordered on stream s; returns when they
-// are complete.
-int host_copy(HostPipe& P, hipStream_t s, const std::vector<HostSeg>& segs) {
+// Copies the segments down to host memory (or up from it), ordered on stream
+// s; returns when they are complete.
+int host_copy(HostPipe& P, hipStream_t s, const std::vector<HostSeg>& segs, bool down = true) {
     size_t total = 0;
     for (const HostSeg& g : segs) total += g.n;
     if (total < HC_MIN) {
-        for (const HostSeg& g : segs) CG_CHECK(hipMemcpyAsync(g.host, g.dev, g.n, hipMemcpyDeviceToHost, s));
+        for (const HostSeg& g : segs)
+            CG_CHECK(down ? hipMemcpyAsync(g.host, g.dev, g.n, hipMemcpyDeviceToHost, s)
+                          : hipMemcpyAsync((void*)g.dev, g.host, g.n, hipMemcpyHostToDevice, s));
         CG_CHECK(hipStreamSynchronize(s));
         return CISMGPU_OK;
     }
     const int st = P.open();
     if (st) return st;
-    struct Chunk { char* host; const char* dev; size_t n; };
+    struct Chunk { char* host; char* dev; size_t n; };
     std::vector<Chunk> chunks;
     for (const HostSeg& g : segs)
         for (size_t o = 0; o < g.n; o += HC_CHUNK)
-            chunks.push_back({(char*)g.host + o, (const char*)g.dev + o, std::min(HC_CHUNK, g.n - o)});
+            chunks.push_back({(char*)g.host + o, (char*)g.dev + o, std::min(HC_CHUNK, g.n - o)});
     int dev = 0;
     CG_CHECK(hipGetDevice(&dev));
     std::atomic<int> err{hipSuccess};
@@ -78,11 +80,21 @@ int host_copy(HostPipe& P, hipStream_t s, const std::vector<HostSeg>& segs) {
         // the link's part of this thread's c-th chunk
         auto link = [&](size_t c, int b) {
             const Chunk& k = chunks[c];
-            return keep(hipMemcpyAsync(slot[b], k.dev, k.n, hipMemcpyDeviceToHost, s)) && keep(hipEventRecord(ev[b], s));
+            return keep(down ? hipMemcpyAsync(slot[b], k.dev, k.n, hipMemcpyDeviceToHost, s)
+                             : hipMemcpyAsync(k.dev, slot[b], k.n, hipMemcpyHostToDevice, s)) &&
+                   keep(hipEventRecord(ev[b], s));
         };
         const size_t n = chunks.size();
-        if ((size_t)t < n && !link(t, 0)) return;
         int b = 0;
+        if (!down) {
+            for (size_t c = t, m = 0; c < n; c += HC_THREADS, b ^= 1, ++m) {
+                if (m >= 2 && !keep(hipEventSynchronize(ev[b]))) return;
+                memcpy(slot[b], chunks[c].host, chunks[c].n);
+                if (!link(c, b)) return;
+            }
+            return;
+        }
+        if ((size_t)t < n && !link(t, 0)) return;
         for (size_t c = t; c < n; c += HC_THREADS, b ^= 1) {
             if (c + HC_THREADS < n && !link(c + HC_THREADS, b ^ 1)) return;
             if (!keep(hipEventSynchronize(ev[b]))) return;

@@ -1100,12 +1100,19 @@ static int set_matrix_impl(cismgpu_system* S, const int32_t* active_vertex, int 
     double* s1 = S->stage + nraw;
     const unsigned gp = nblocks(d.nrows * 27, 256);
     // Auv, Avu first through the staging pair, then Auu/Avv which stay staged
-    CG_CHECK(hipMemcpyAsync(s0, Auv, nraw * sizeof(double), kind, S->s));
-    CG_CHECK(hipMemcpyAsync(s1, Avu, nraw * sizeof(double), kind, S->s));
+    auto stage2 = [&](const double* a, const double* b) -> int {
+        const size_t n = nraw * sizeof(double);
+        if (!where_A) return host_copy(S->pipe, S->s, {{(void*)a, s0, n}, {(void*)b, s1, n}}, false);
+        CG_CHECK(hipMemcpyAsync(s0, a, n, kind, S->s));
+        CG_CHECK(hipMemcpyAsync(s1, b, n, kind, S->s));
+        return CISMGPU_OK;
+    };
+    int st = stage2(Auv, Avu);
+    if (st) return st;
     k_pack_matrix<double><<<gp, 256, 0, S->s>>>(d, 1, s0, S->active, S->A64);
     k_pack_matrix<double><<<gp, 256, 0, S->s>>>(d, 2, s1, S->active, S->A64);
-    CG_CHECK(hipMemcpyAsync(s0, Auu, nraw * sizeof(double), kind, S->s));
-    CG_CHECK(hipMemcpyAsync(s1, Avv, nraw * sizeof(double), kind, S->s));
+    st = stage2(Auu, Avv);
+    if (st) return st;
     k_pack_matrix<double><<<gp, 256, 0, S->s>>>(d, 0, s0, S->active, S->A64);
     k_pack_matrix<double><<<gp, 256, 0, S->s>>>(d, 3, s1, S->active, S->A64);
     k_setup_precond<double><<<nblocks(nvec, 256), 256, 0, S->s>>>(d, s0, s1, S->M64, S->M64 + 6 * d.vlen);
@@ -1203,8 +1210,9 @@ int32_t cismgpu_system_set_x(cismgpu_system* S, const double* xu, const double* 
     double* tmp = S->V(12);
     CG_CHECK(hipMemsetAsync(S->V(0), 0, 2 * d.vlen * sizeof(double), S->s));
     double* tmp2 = S->V(13);
-    CG_CHECK(hipMemcpyAsync(tmp, xu, nvec * sizeof(double), hipMemcpyHostToDevice, S->s));
-    CG_CHECK(hipMemcpyAsync(tmp2, xv, nvec * sizeof(double), hipMemcpyHostToDevice, S->s));
+    const size_t nb = nvec * sizeof(double);
+    const int st = host_copy(S->pipe, S->s, {{(void*)xu, tmp, nb}, {(void*)xv, tmp2, nb}}, false);
+    if (st) return st;
     k_vec_in<double, double><<<nblocks(nvec, 256), 256, 0, S->s>>>(d, tmp, S->V(0));
     k_vec_in<double, double><<<nblocks(nvec, 256), 256, 0, S->s>>>(d, tmp2, S->V(1));
     CG_CHECK(hipMemsetAsync(tmp, 0, 2 * d.vlen * sizeof(double), S->s));
