@@ -7,7 +7,7 @@ namespace cg {
 // slots of the device scalar block
 enum {
     S_ALPHA = 0, S_BETA, S_RHO, S_SIGMA, S_ETA0, S_BB, S_L2RHS, S_RR, S_ERR, S_CONV,
-    S_NAN, S_STOP, S_DOT, S_DOT2, S_NSLOTS = 16
+    S_NAN, S_STOP, S_DOT, S_DOT2, S_ALPHA_OLD, S_NSLOTS = 16
 };
 // stages of k_scalars
 enum { ST_BB = 0, ST_RR, ST_CG_FIRST, ST_CG_ITER, ST_STD_ETA1, ST_STD_ETA2, ST_DOT };

@@ -319,12 +319,22 @@ void scal_done(cismgpu_system* S, const ScalIn& R) {
 // The C-G or standard update of v = xu xv ru rv du dv qu qv zu zv Azu Azv,
 // with the preconditioner on the new residual when fused (precond 1 or 2).
 template <typename TV, int STD>
-void launch_update(cismgpu_system* S, const ScalIn& R, TV* const* v, const TV* M, int precond, bool fused) {
+void launch_update(cismgpu_system* S, const ScalIn& R, TV* const* v, const TV* M, int precond, bool fused,
+                   int xm = 0) {
     const Dims& d = S->d;
     if (R.stage >= 0 && R.pa == S->partA) std::swap(S->partA, S->partA_alt);   // its reader writes the other
     const TV* Dg = M + 6 * d.vlen;
 #define FLAT(DIAG) k_update_flat<TV, DIAG, STD><<<flat_blocks(d), 256, 0, S->s>>>(d, R, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9], v[10], v[11], Dg, S->partA)
-#define UPD(NZM, SY) k_update<TV, NZM, STD, SY><<<upd_blocks(d), 256, 0, S->s>>>(d, R, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9], v[10], v[11], M, S->active, S->partA)
+#define UPDX(NZM, SY, XM) k_update<TV, NZM, STD, SY, XM><<<upd_blocks(d), 256, 0, S->s>>>(d, R, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9], v[10], v[11], M, S->active, S->partA)
+    // x left for later only in the FP32 inner solve, whose systems are assembled (SYM) as a rule
+#define UPD(NZM, SY)                                                             \
+    do {                                                                         \
+        if constexpr (std::is_same<TV, float>::value && !STD) {                  \
+            if (xm == 1) UPDX(NZM, SY, 1);                                       \
+            else if (xm == 2) UPDX(NZM, SY, 2);                                  \
+            else UPDX(NZM, SY, 0);                                               \
+        } else UPDX(NZM, SY, 0);                                                 \
+    } while (0)
     if (!fused) FLAT(0);
     else if (precond == 1) FLAT(1);
     else if (precond_sym<TV>(S)) {
@@ -337,6 +347,7 @@ void launch_update(cismgpu_system* S, const ScalIn& R, TV* const* v, const TV* M
         else UPD(64, 0);
     }
 #undef UPD
+#undef UPDX
 #undef FLAT
     scal_done(S, R);
 }
@@ -686,6 +697,12 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
     // themselves (their (A z, z) sums still take the values before it).
     const bool noop = zero_halo_is_noop(S);
     const bool fuse_scal = !rs && nub + nsp <= FUSE_MAX;   // the update sums the partials itself
+    const bool defer_x = given_r && fuse_ok && precond == 2 && std::is_same<TV, float>::value;
+    bool late_x = false;
+    auto finish_x = [&]() {
+        if (late_x)
+            k_late_x<TV><<<nblocks(d.nz * d.plane, 256), 256, 0, S->s>>>(d, S->scal, xu, xv, du, dv);
+    };
     const bool fold = !noop && d.bc == 3 && !rs && std::is_same<TA, double>::value && !S->elem_use;
     for (int iter = 2; iter <= maxiters; ++iter) {
         if (!z_ready) apply_precond<TV>(S, precond, ru, rv, zu, zv);
@@ -702,8 +719,11 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
         if (!fold && !noop) halo<TV>(S, Azu, Azv, d.nz);
         const bool check = (iter % ncheck == 0) || iter == 5;
         const bool fuse = fuse_ok && (precond == 1 || precond == 2) && !(check && !given_r);
+        // the inner solve reads x only when it ends: every second update of x waits for the next
+        const int xm = !(defer_x && fuse) ? 0 : late_x ? 2 : 1;
         launch_update<TV, 0>(S, fuse_scal ? scal_in(S, ST_CG_ITER, S->partA, nub, 4, S->partB, nsp, 2) : scal_in(S), vv,
-                             M, precond, fuse);
+                             M, precond, fuse, xm);
+        late_x = xm == 1;
         z_ready = fuse;
         if (check) {
             if (given_r) {
@@ -726,10 +746,15 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
             if (st) return st;
             if (S->scal_h[S_NAN] != 0.0) { cismgpu_set_error("Chron-Gear PCG solver has failed, alpha = NaN"); return CISMGPU_ERR_NAN; }
             *err = S->scal_h[S_ERR];
-            if (S->scal_h[S_CONV] != 0.0) { *niters = iter; return CISMGPU_OK; }
+            if (S->scal_h[S_CONV] != 0.0) {
+                *niters = iter;
+                finish_x();
+                return CISMGPU_OK;
+            }
             if (!given_r && !noop) halo<TV>(S, ru, rv, d.nz);
         }
     }
+    finish_x();
     st = sync_scal(S);
     if (st) return st;
     if (S->scal_h[S_NAN] != 0.0) { cismgpu_set_error("Chron-Gear PCG solver has failed, alpha = NaN"); return CISMGPU_ERR_NAN; }
