@@ -129,6 +129,11 @@ __device__ __forceinline__ float2 prod2(float cuu, float cuv, float cvu, float c
     return make_float2(__builtin_fmaf(cuv, xv, cuu * xu), __builtin_fmaf(cvv, xv, cvu * xu));
 }
 __device__ __forceinline__ float2 add2(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
+// a node's share of a dot product: both products are exact in FP64, so this is
+// their sum rounded once, whichever kernel forms it
+__device__ __forceinline__ double dot2(float a, float b, float c, float e) {
+    return fma((double)a, (double)b, (double)c * (double)e);
+}
 
 template <typename F>
 __device__ __forceinline__ float2 node_sum(F term) {
@@ -154,8 +159,11 @@ __device__ __forceinline__ float2 node_sum(F term) {
     return y;
 }
 
+// FP32 rows at 5 wavefronts per SIMD; BF16 rows are half the bytes and want the
+// loads of 3 (149 registers: 0.52 ms at 1024^2 x 11 against 0.71 ms at 5), and
+// sum in the order of storage, since no other kernel has to give their bits.
 template <typename TA, int MODE>
-__global__ __launch_bounds__(256, 5) void k_spmv_q(Dims d, const TA* __restrict__ A, const float* __restrict__ xu,
+__global__ __launch_bounds__(256, sizeof(TA) == 4 ? 5 : 3) void k_spmv_q(Dims d, const TA* __restrict__ A, const float* __restrict__ xu,
                                                 const float* __restrict__ xv, float* __restrict__ yu,
                                                 float* __restrict__ yv, const float* __restrict__ bu,
                                                 const float* __restrict__ bv, double* __restrict__ partials,
@@ -191,25 +199,36 @@ __global__ __launch_bounds__(256, 5) void k_spmv_q(Dims d, const TA* __restrict_
             }
             const long long r = ((long long)k * d.nyo + jo) * d.nxp + io;
             const TA* a = A + (r / WAVE) * (27 * 4 * WAVE) + (r % WAVE) * 4;
-            const float2 y = node_sum([&](int m, float2& g) {
-                float cuu, cuv, cvu, cvv;
-                ld_quad(a + m * (4 * WAVE), cuu, cuv, cvu, cvv);
-                g = add2(g, prod2(cuu, cuv, cvu, cvv, wu[m / 9][m % 9], wv[m / 9][m % 9]));
-            });
-            const float su = y.x, sv = y.y;
+            float su = 0.f, sv = 0.f;
+            if constexpr (std::is_same<TA, float>::value) {
+                const float2 y = node_sum([&](int m, float2& g) {
+                    float cuu, cuv, cvu, cvv;
+                    ld_quad(a + m * (4 * WAVE), cuu, cuv, cvu, cvv);
+                    g = add2(g, prod2(cuu, cuv, cvu, cvv, wu[m / 9][m % 9], wv[m / 9][m % 9]));
+                });
+                su = y.x;
+                sv = y.y;
+            } else {
+#pragma unroll
+                for (int m = 0; m < 27; ++m) {
+                    float cuu, cuv, cvu, cvv;
+                    ld_quad(a + m * (4 * WAVE), cuu, cuv, cvu, cvv);
+                    const float xun = wu[m / 9][m % 9], xvn = wv[m / 9][m % 9];
+                    su = su + cuu * xun + cuv * xvn;
+                    sv = sv + cvu * xun + cvv * xvn;
+                }
+            }
             const long long c0 = cb + (long long)(k + 1) * pl;
             if (MODE == 2) {
                 const float ru = bu[c0] - su, rv = bv[c0] - sv;
                 yu[c0] = ru;
                 yv[c0] = rv;
-                acc = dd_add_d(acc, (double)ru * (double)ru);
-                acc = dd_add_d(acc, (double)rv * (double)rv);
+                acc = dd_add_d(acc, dot2(ru, ru, rv, rv));
             } else {
                 yu[c0] = su;
                 yv[c0] = sv;
                 if (MODE == 1) {
-                    acc = dd_add_d(acc, (double)su * (double)wu[1][4]);
-                    acc = dd_add_d(acc, (double)sv * (double)wv[1][4]);
+                    acc = dd_add_d(acc, dot2(su, wu[1][4], sv, wv[1][4]));
                 }
             }
 #pragma unroll

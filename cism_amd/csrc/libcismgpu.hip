@@ -399,7 +399,10 @@ int scalars_to_host(cismgpu_system* S, int stage, const double* pa, int na, int 
     };
     for (unsigned n = 1;; ++n) {
         if (arrived()) return CISMGPU_OK;
-        if (n % 8192 == 0 && hipStreamQuery(S->s) != hipErrorNotReady) break;
+        if (n % 8192 == 0) {
+            if (hipStreamQuery(S->s) != hipErrorNotReady) break;
+            (void)hipGetLastError();   // "not ready" is no error of the next call that asks
+        }
     }
     return sync_scal(S);
 }

@@ -185,15 +185,13 @@ __global__ __launch_bounds__(256, 4) void k_spmv_sym(Dims d, const TA* __restric
                 const float ru = bu[ck] - su, rv = bv[ck] - sv;
                 yu[ck] = ru;
                 yv[ck] = rv;
-                acc = dd_add_d(acc, (double)ru * (double)ru);
-                acc = dd_add_d(acc, (double)rv * (double)rv);
+                acc = dd_add_d(acc, dot2(ru, ru, rv, rv));
             } else {
                 yu[ck] = su;
                 yv[ck] = sv;
                 if (MODE == 1) {
                     const int slot = (k + 1) % 3;
-                    acc = dd_add_d(acc, (double)su * (double)xs[0][slot][w + 1][lane + 1]);
-                    acc = dd_add_d(acc, (double)sv * (double)xs[1][slot][w + 1][lane + 1]);
+                    acc = dd_add_d(acc, dot2(su, xs[0][slot][w + 1][lane + 1], sv, xs[1][slot][w + 1][lane + 1]));
                 }
             }
         }
@@ -431,14 +429,12 @@ __global__ __launch_bounds__(WAVE * SJ_WAVES) void k_spmv_symj(Dims d, const flo
                 const float ru = bu[ck] - y.x, rv = bv[ck] - y.y;
                 yu[ck] = ru;
                 yv[ck] = rv;
-                acc = dd_add_d(acc, (double)ru * (double)ru);
-                acc = dd_add_d(acc, (double)rv * (double)rv);
+                acc = dd_add_d(acc, dot2(ru, ru, rv, rv));
             } else {
                 yu[ck] = y.x;
                 yv[ck] = y.y;
                 if (MODE == 1) {
-                    acc = dd_add_d(acc, (double)y.x * (double)xp.x);
-                    acc = dd_add_d(acc, (double)y.y * (double)xp.y);
+                    acc = dd_add_d(acc, dot2(y.x, xp.x, y.y, xp.y));
                 }
             }
         }
