@@ -36,12 +36,13 @@ static __device__ __align__(256) double scratch[NA_MAX_BLOCKS * NA_PART];
 // node's row touches another cache line per lane and load, 4 x 64 lines at a
 // time, which the 32 KB L1 does not hold until the next coefficient wants
 // them.  Here wavefront w copies the 64 rows of block w (13.8 KB, contiguous)
-// to LDS with unit-stride loads, all 27 of them in flight, and then each lane
-// takes its node's row from LDS (a stride of 27 doubles is odd: no bank
-// conflicts).  55 KB of LDS per workgroup, two workgroups per CU.  At
+// to LDS with unit-stride loads, all 27 of them in flight, and then the lanes
+// of wavefronts 0 and 1 take their nodes' u and v rows from LDS (a stride of 27
+// doubles is odd: no bank conflicts), in the order of terms that one thread
+// per node had.  55 KB of LDS per workgroup, two workgroups per CU.  At
 // 400^2 x 11 (1.58 GB) 0.40 ms = 4.0 TB/s against 1.55 ms for one thread per
-// node reading its rows from memory; 9,000 nodes 12.0 against 12.7 us, which
-// is the two launches.
+// node reading its rows from memory; 9,000 nodes 12.6 us either way, which is
+// the two launches.
 __global__ __launch_bounds__(NA_THREADS) void k_resid_ref(Dims d, const int32_t* __restrict__ active,
                                                           const double* __restrict__ Auu, const double* __restrict__ Auv,
                                                           const double* __restrict__ Avu, const double* __restrict__ Avv,
@@ -50,12 +51,10 @@ __global__ __launch_bounds__(NA_THREADS) void k_resid_ref(Dims d, const int32_t*
                                                           double* __restrict__ ru, double* __restrict__ rv,
                                                           double* __restrict__ part) {
     __shared__ double rows[4][27 * NA_TILE];
-    __shared__ double sum[4][NA_TILE];
     const int n = d.nz * d.nvx * d.nvy;                 // at most NA_MAX_NODES
     const int ntile = (n + NA_TILE - 1) / NA_TILE;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
     const double* A = w == 0 ? Auu : w == 1 ? Auv : w == 2 ? Avu : Avv;
-    const double* x = (w & 1) ? v : u;
     dd acc[2] = {{0.0, 0.0}, {0.0, 0.0}};
     for (int tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
         const int t = tile * NA_TILE + lane;
@@ -68,20 +67,27 @@ __global__ __launch_bounds__(NA_THREADS) void k_resid_ref(Dims d, const int32_t*
             j = 1 + col / d.nvx;
             on = i >= d.ilo && i <= d.ihi && j >= d.jlo && j <= d.jhi && active[col] != 0;
         }
-        double s = 0.0;
-        if (__any(on)) {
+        const bool any = __any(on);                     // the same in all four wavefronts
+        double r[27];
+        if (any) {
             const long long e0 = 27LL * tile * NA_TILE, ne = 27LL * n;
-            double r[27];
 #pragma unroll
             for (int q = 0; q < 27; ++q) {
                 const long long e = e0 + q * WAVE + lane;
                 r[q] = e < ne ? A[e] : 0.0;
             }
+        }
+        __syncthreads();                                // the last tile's rows are no longer read
+        if (any) {
 #pragma unroll
             for (int q = 0; q < 27; ++q) rows[w][q * WAVE + lane] = r[q];
-            __builtin_amdgcn_wave_barrier();            // rows[w] is this wavefront's own
+        }
+        __syncthreads();
+        if (w < 2 && t < n) {                           // wavefront 0: the u rows, 1: the v rows
+            double res = 0.0;
             if (on) {
-                const double* a = rows[w] + 27 * lane;
+                const double *au = rows[2 * w] + 27 * lane, *av = rows[2 * w + 1] + 27 * lane;
+                double s = 0.0;
 #pragma unroll
                 for (int kA = -1; kA <= 1; ++kA) {
                     if (k + kA < 0 || k + kA >= d.nz) continue;
@@ -90,25 +96,18 @@ __global__ __launch_bounds__(NA_THREADS) void k_resid_ref(Dims d, const int32_t*
 #pragma unroll
                         for (int iA = -1; iA <= 1; ++iA) {
                             const int m = (iA + 1) + 3 * (jA + 1) + 9 * (kA + 1);
-                            s = s + a[m] * x[(k + kA) + (long long)d.nz * ((i + iA - 1) + (long long)d.nvx * (j + jA - 1))];
+                            const long long q = (k + kA) + (long long)d.nz * ((i + iA - 1) + (long long)d.nvx * (j + jA - 1));
+                            s = s + au[m] * u[q] + av[m] * v[q];
                         }
                 }
-            }
-        }
-        sum[w][lane] = s;
-        __syncthreads();
-        if (w < 2 && t < n) {                           // wavefront 0: the u rows, 1: the v rows
-            double r = 0.0;
-            if (on) {
                 const double bb = (w ? bv : bu)[t];
-                r = (sum[2 * w][lane] + sum[2 * w + 1][lane]) - bb;
-                acc[0] = dd_add_d(acc[0], r * r);
+                res = s - bb;
+                acc[0] = dd_add_d(acc[0], res * res);
                 acc[1] = dd_add_d(acc[1], bb * bb);
             }
             double* out = w ? rv : ru;
-            if (out) out[t] = r;
+            if (out) out[t] = res;
         }
-        __syncthreads();                                // sum is rewritten for the next tile
     }
     block_reduce_dd<2, NA_THREADS>(acc);
     if (threadIdx.x == 0) {
