@@ -1123,6 +1123,7 @@ static int set_matrix_impl(cismgpu_system* S, const int32_t* active_vertex, int 
     } else {
         for (long long i = 0; i < n2; ++i) act[i] = active_vertex[i] ? 1 : 0;
     }
+    S->elem_ok = false;          // also when a copy below fails
     CG_CHECK(hipMemcpyAsync(S->active, act.data(), n2, hipMemcpyHostToDevice, S->s));
     double* s0 = S->stage;
     double* s1 = S->stage + nraw;
@@ -1156,7 +1157,6 @@ static int set_matrix_impl(cismgpu_system* S, const int32_t* active_vertex, int 
     S->raw_ready = true;
     S->sym_exact = false;
     S->edge_zero = false;
-    S->elem_ok = false;
     S->m32_ready = S->a32_ready = S->a16_ready = S->a64h_ready = false;
     S->a32_sym = S->a64_sym = false;
     S->tri.mode = 0;
@@ -1633,9 +1633,15 @@ static int upload_assembly_inputs(cismgpu_system* S, const Dims& d, const cismgp
                              (in->flwa ? nfl : 0) + (in->stag_lsrf ? n2 : 0)),
                  ni = (size_t)(nc + n2 + 2 * nvec + (lateral ? nc : 0));
     const size_t bytes = nd * sizeof(double) + ni * sizeof(int32_t);
+    // The inputs of the last assembly are overwritten or freed from here on,
+    // and a copy or the allocation may fail: what reads them (the products in
+    // element form, the diagnostics) has to wait for the assembly to be done.
+    S->elem_ok = S->asm3_ready = false;
+    S->asm_in = AsmDev{};
     if (S->asm_bytes < bytes) {
         if (S->asm_buf) hipFree(S->asm_buf);
         S->asm_buf = nullptr;
+        S->asm_bytes = 0;
         CG_CHECK(hipMalloc(&S->asm_buf, bytes));
         S->asm_bytes = bytes;
     }
@@ -1728,7 +1734,6 @@ extern "C" int32_t cismgpu_system_assemble_3d(cismgpu_system* S, const cismgpu_a
     hipEvent_t e0, e1, e2;
     hipEventCreate(&e0); hipEventCreate(&e1); hipEventCreate(&e2);
     { const int st_ = reset_scal(S); if (st_) return st_; }
-    S->elem_ok = false;
     const double* uv = S->V(0);
     const double* vv = S->V(1);
     // element-once assembly (CISMGPU_ASSEMBLY=gather: the per-row gather
@@ -2087,7 +2092,7 @@ extern "C" int32_t cismgpu_system_diva_setup(cismgpu_system* S, const cismgpu_di
 // and the traction (nx-1, ny-1) to the host.  a.beta is the last assembly's.
 extern "C" int32_t cismgpu_system_diva_velocity(cismgpu_system* S, double* uvel, double* vvel, double* btractx,
                                                 double* btracty) {
-    if (!S || !S->diva_ready || !S->asm_buf) { cismgpu_set_error("diva_velocity: no DIVA assembly"); return CISMGPU_ERR_ARG; }
+    if (!S || !S->diva_ready || !S->asm_in.acell) { cismgpu_set_error("diva_velocity: no DIVA assembly"); return CISMGPU_ERR_ARG; }
     const Dims& d = S->d;
     const long long n2 = (long long)d.nvx * d.nvy, nz = S->nz_levels;
     double* u3 = nullptr;
@@ -2182,6 +2187,7 @@ extern "C" int32_t cismgpu_system_restore_assembly(cismgpu_system* S) {
     size_t sizes[NSAVED];
     saved_parts(S, S->saved, parts, sizes);
     double* dst[NSAVED] = {S->A64, S->V(2), S->M64, S->stage, S->dv.bex, S->dv.bey, S->dv.omega_k};
+    S->elem_ok = false;          // also when a copy below fails
     for (int q = 0; q < NSAVED; ++q)
         if (sizes[q]) CG_CHECK(hipMemcpyAsync(dst[q], parts[q], sizes[q] * sizeof(double), hipMemcpyDeviceToDevice, S->s));
     CG_CHECK(hipStreamSynchronize(S->s));
@@ -2189,7 +2195,6 @@ extern "C" int32_t cismgpu_system_restore_assembly(cismgpu_system* S) {
     S->raw_ready = S->saved_raw_ready;
     S->sym_exact = false;
     S->edge_zero = false;
-    S->elem_ok = false;
     S->m32_ready = S->a32_ready = S->a16_ready = S->a64h_ready = false;
     S->a32_sym = S->a64_sym = false;
     S->tri.mode = 0;

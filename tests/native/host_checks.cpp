@@ -1,0 +1,126 @@
+// host_checks.cpp -- host code of libcismgpu.so on a HIP runtime without a
+// device (hip_on_host.h).  Usage: host_checks LIB CHECK; exit status 0 when
+// the check holds.
+#include "hip_on_host.h"
+
+#include <dlfcn.h>
+
+#include "cismgpu.h"
+
+#define FN(name) static decltype(&name) p_##name
+FN(cismgpu_system_create);
+FN(cismgpu_system_destroy);
+FN(cismgpu_system_assemble_3d);
+FN(cismgpu_system_solve);
+FN(cismgpu_system_residual);
+FN(cismgpu_system_internal_stress);
+
+static int bad = 0;
+#define EXPECT(c)                                                       \
+    do {                                                                \
+        if (!(c)) { printf("line %d: not %s\n", __LINE__, #c); ++bad; } \
+    } while (0)
+
+// Flat ice on an n x n block of owned vertices, every cell and vertex of the
+// inner block active; nothing here is computed, the calls only have to pass.
+struct Ice {
+    cismgpu_grid g{};
+    cismgpu_system* S = nullptr;
+    std::vector<double> vert, levels, layers, cells;
+    std::vector<int32_t> acell, avert, ocean;
+    cismgpu_assembly_in in{};
+
+    Ice(int n, int nz) {
+        g.nx = g.ny = n + 4;
+        g.nz = nz;
+        g.ilo = g.jlo = 3;
+        g.ihi = g.jhi = n + 2;
+        g.global_bc = 3;
+        const int nv = g.nx - 1;
+        vert.assign((size_t)nv * nv, 1.0);
+        levels.resize(nz + 1);
+        for (int k = 0; k <= nz; ++k) levels[k] = (double)k / nz;
+        layers.assign((size_t)(nz - 1) * g.nx * g.ny, 1.0);
+        cells.assign((size_t)g.nx * g.ny, 1.0);
+        acell.assign(cells.size(), 1);
+        avert.assign(vert.size(), 1);
+        ocean.assign(cells.size(), 0);
+        in.dx = in.dy = 1.0;
+        in.sigma = in.stagwbndsigma = levels.data();
+        in.active_cell = acell.data();
+        in.active_vertex = avert.data();
+        for (const double** p : {&in.xVertex, &in.yVertex, &in.stagusrf, &in.stagthck, &in.dusrf_dx, &in.dusrf_dy})
+            *p = vert.data();
+        in.flwafact = layers.data();
+        in.whichefvs = 2;
+        in.n_glen = 3.0;
+        EXPECT(p_cismgpu_system_create(&g, &S) == 0);
+    }
+    ~Ice() { p_cismgpu_system_destroy(S); }
+
+    int assemble() { return p_cismgpu_system_assemble_3d(S, &in, nullptr); }
+    // the fields of the lateral condition too: a larger input block
+    int assemble_lateral() {
+        cismgpu_assembly_in b = in;
+        b.ocean_mask = ocean.data();
+        b.usrf = b.thck = cells.data();
+        b.stagusrf_lateral = b.stagthck_lateral = vert.data();
+        return p_cismgpu_system_assemble_3d(S, &b, nullptr);
+    }
+    int solve(int precision = CISMGPU_FP64, int maxiters = 6) {
+        onhost::launched.clear();
+        cismgpu_solve_opts o{CISMGPU_ALGO_CHRONGEAR, 2, 5, maxiters, 0.0, precision, 1e-4, 2, 0};
+        cismgpu_solve_info info;
+        return p_cismgpu_system_solve(S, &o, &info);
+    }
+};
+
+// A re-assembly that fails once its inputs are being replaced: the element
+// form of the products reads those inputs, so what follows keeps to the rows
+// of the old matrix, and the diagnostics, which have nothing else, refuse.
+static void failed_reassembly(bool copy_fails) {
+    Ice s(8, 3);
+    std::vector<double> tau(s.layers.size());
+    EXPECT(s.assemble() == 0);
+    s.solve();
+    EXPECT(onhost::count("k_spmv_elem") > 0);
+    if (copy_fails) onhost::copies_to_failure = 5;
+    else onhost::fail_malloc = true;
+    EXPECT((copy_fails ? s.assemble() : s.assemble_lateral()) != 0);
+    onhost::copies_to_failure = -1;
+    onhost::fail_malloc = false;
+    s.solve();
+    EXPECT(onhost::count("k_spmv_elem") == 0 && onhost::count("k_spmv") > 0);
+    onhost::launched.clear();
+    p_cismgpu_system_residual(s.S, nullptr, nullptr, nullptr, nullptr);
+    EXPECT(onhost::count("k_spmv_elem") == 0 && onhost::count("k_spmv") > 0);
+    onhost::launched.clear();
+    EXPECT(p_cismgpu_system_internal_stress(s.S, tau.data(), nullptr, nullptr, nullptr, nullptr, nullptr) != 0);
+    EXPECT(onhost::count("k_internal_stress") == 0);
+    EXPECT(s.assemble() == 0);            // an input block of the first size is there again
+    s.solve();
+    EXPECT(onhost::count("k_spmv_elem") > 0);
+    EXPECT(p_cismgpu_system_internal_stress(s.S, tau.data(), nullptr, nullptr, nullptr, nullptr, nullptr) == 0);
+}
+
+int main(int argc, char** argv) {
+    if (argc != 3) return 2;
+    void* lib = dlopen(argv[1], RTLD_NOW);
+    if (!lib) { printf("%s\n", dlerror()); return 2; }
+#define LOAD(name) p_##name = (decltype(p_##name))dlsym(lib, #name)
+    LOAD(cismgpu_system_create);
+    LOAD(cismgpu_system_destroy);
+    LOAD(cismgpu_system_assemble_3d);
+    LOAD(cismgpu_system_solve);
+    LOAD(cismgpu_system_residual);
+    LOAD(cismgpu_system_internal_stress);
+    const std::map<std::string, std::function<void()>> checks = {
+        {"reassembly_out_of_memory", [] { failed_reassembly(false); }},
+        {"reassembly_failed_copy", [] { failed_reassembly(true); }},
+    };
+    const auto c = checks.find(argv[2]);
+    if (c == checks.end()) { printf("no check %s\n", argv[2]); return 2; }
+    c->second();
+    fflush(stdout);
+    _Exit(bad ? 1 : 0);
+}
