@@ -1741,16 +1741,18 @@ extern "C" int32_t cismgpu_system_assemble_3d(cismgpu_system* S, const cismgpu_a
     const char* aenv = getenv("CISMGPU_ASSEMBLY");
     const bool gather = aenv && !strcmp(aenv, "gather");
     if (!gather && !S->elemq) CG_CHECK(hipMalloc(&S->elemq, (size_t)8 * EQ * nfl * sizeof(double)));
-    // counters: nnz, pairs left asymmetric by the fix, differing pairs, vertices off a rectilinear grid
+    // counters: nnz, pairs left asymmetric by the fix, differing pairs, then those of k_form_check
+    unsigned long long hc[5] = {0, 0, 0, 0, 0};
     unsigned long long* cnt = nullptr;
-    CG_CHECK(hipMalloc(&cnt, 4 * sizeof(unsigned long long)));
-    CG_CHECK(hipMemsetAsync(cnt, 0, 4 * sizeof(unsigned long long), S->s));
+    CG_CHECK(hipMalloc(&cnt, sizeof(hc)));
+    CG_CHECK(hipMemsetAsync(cnt, 0, sizeof(hc), S->s));
     // The element-once rows are symmetric by construction between owned
     // nodes; with no pass after them that changes couplings inside the
     // owned region (Dirichlet rows and columns, standard basal quadrature)
     // the symmetry check and the nonzero count visit only the rim rows, and
     // the other rows are counted as they are written (CISMGPU_SYMCHECK=full:
-    // every row checked and counted).
+    // every row checked and counted).  A vertex mask with inactive vertices
+    // inside the ice is the exception, found by k_form_check.
     const char* senv = getenv("CISMGPU_SYMCHECK");
     const bool plain = !gather && !in->umask_dirichlet && !in->vmask_dirichlet && !(has_beta(in) && a.beta_std);
     const bool rim_only = plain && !(senv && !strcmp(senv, "full"));
@@ -1779,7 +1781,7 @@ extern "C" int32_t cismgpu_system_assemble_3d(cismgpu_system* S, const cismgpu_a
         else
             k_basal_local<<<nblocks((long long)d.nxo * d.nyo, 256), 256, 0, S->s>>>(d, a, S->A64, S->elem_bd);
     }
-    if (elem_form) k_rectilinear<<<nblocks(n2, 256), 256, 0, S->s>>>(d, a.xV, a.yV, cnt + 3);
+    if (plain) k_form_check<<<nblocks(n2, 256), 256, 0, S->s>>>(d, a, cnt + 3);
     if (a.taud_std)
         k_load_gravity_std<<<nblocks(n2, 64), 64, 0, S->s>>>(d, a, S->V(2), S->V(3), S->scal + S_NAN);
     else
@@ -1797,15 +1799,23 @@ extern "C" int32_t cismgpu_system_assemble_3d(cismgpu_system* S, const cismgpu_a
     // pass runs only when one exists
     S->sym_exact = false;
     {
-        unsigned long long ndiff = 1;
-        if (rim_only)
-            k_symmetry_rim<<<nblocks(rim_rows_per_level(d) * d.nz, 256), 256, 0, S->s>>>(d, a.avert, S->A64, cnt + 2,
-                                                                                      cnt);
-        else
-            k_symmetry_count<<<nblocks(d.nrows, 256), 256, 0, S->s>>>(d, a.avert, S->A64, cnt + 2, cnt);
-        CG_CHECK(hipMemcpyAsync(&ndiff, cnt + 2, sizeof(ndiff), hipMemcpyDeviceToHost, S->s));
-        CG_CHECK(hipStreamSynchronize(S->s));
-        if (ndiff == 0) {
+        auto count = [&](bool rim) -> int {
+            if (rim)
+                k_symmetry_rim<<<nblocks(rim_rows_per_level(d) * d.nz, 256), 256, 0, S->s>>>(d, a.avert, S->A64,
+                                                                                          cnt + 2, cnt);
+            else
+                k_symmetry_count<<<nblocks(d.nrows, 256), 256, 0, S->s>>>(d, a.avert, S->A64, cnt + 2, cnt);
+            CG_CHECK(hipMemcpyAsync(hc, cnt, sizeof(hc), hipMemcpyDeviceToHost, S->s));
+            CG_CHECK(hipStreamSynchronize(S->s));
+            return CISMGPU_OK;
+        };
+        st = count(rim_only);
+        if (!st && rim_only && hc[4] != 0) {   // the rim does not tell: every row, both counts anew
+            CG_CHECK(hipMemsetAsync(cnt, 0, 3 * sizeof(unsigned long long), S->s));
+            st = count(false);
+        }
+        if (st) return st;
+        if (hc[2] == 0) {
             S->sym_exact = true;
         } else if (in->check_symmetry) {
             if (!S->Atmp) CG_CHECK(hipMalloc(&S->Atmp, d.nrows * NCOEF * sizeof(double)));
@@ -1824,7 +1834,6 @@ extern "C" int32_t cismgpu_system_assemble_3d(cismgpu_system* S, const cismgpu_a
     // the raw Auu/Avv of the line-solve preconditioners are built when first needed
     S->raw_ready = false;
     hipEventRecord(e2, S->s);
-    unsigned long long hc[4] = {0, 0, 0, 0};
     CG_CHECK(hipMemcpyAsync(hc, cnt, sizeof(hc), hipMemcpyDeviceToHost, S->s));
     CG_CHECK(sync_scal(S) ? hipErrorUnknown : hipSuccess);
     hipFree(cnt);
@@ -1838,7 +1847,7 @@ extern "C" int32_t cismgpu_system_assemble_3d(cismgpu_system* S, const cismgpu_a
         info->assemble_ms = ms1;
         info->total_ms = ms2;
     }
-    S->elem_ok = elem_form && S->sym_exact && hc[3] == 0 && S->scal_h[S_NAN] == 0.0;
+    S->elem_ok = elem_form && S->sym_exact && hc[3] == 0 && hc[4] == 0 && S->scal_h[S_NAN] == 0.0;
     S->have_matrix = true;
     S->m32_ready = S->a32_ready = S->a16_ready = S->a64h_ready = false;
     S->a32_sym = S->a64_sym = false;

@@ -53,18 +53,29 @@ inline int elem_split(const Dims& d) {
 }
 inline int elem_parts(const Dims& d) { return elem_blocks(d) * ((d.nz + elem_split(d) - 1) / elem_split(d)); }
 
-// Counts the vertices whose x varies along j or whose y varies along i: the
-// element form needs none (x a function of i alone, y of j alone).
-__global__ void k_rectilinear(Dims d, const double* __restrict__ xV, const double* __restrict__ yV,
-                              unsigned long long* __restrict__ count) {
+// What the short cuts of the assembly rest on, counted: count[0] the vertices
+// whose x varies along j or whose y varies along i (the element form needs a
+// rectilinear vertex grid), count[1] the owned inactive vertices of active
+// cells.  The rows of those are zero (k_rows) while the element form would
+// give them their cells' part, and their neighbours' rows couple to them, so
+// the matrix is not symmetric off the rim either.
+__global__ void k_form_check(Dims d, AsmDev in, unsigned long long* __restrict__ count) {
     const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    unsigned long long bad = 0;
+    unsigned long long bent = 0, gap = 0;
     if (t < (long long)d.nvx * d.nvy) {
-        const long long i = t % d.nvx, j = t / d.nvx;
-        bad = (xV[t] != xV[i] || yV[t] != yV[j * d.nvx]) ? 1ull : 0ull;
+        const long long i0 = t % d.nvx, j0 = t / d.nvx;
+        bent = (in.xV[t] != in.xV[i0] || in.yV[t] != in.yV[j0 * d.nvx]) ? 1ull : 0ull;
+        const int i = 1 + (int)i0, j = 1 + (int)j0;
+        auto cell_on = [&](int ci, int cj) { return cell_in_range(d, in.nhalo, ci, cj) && in.acell[c2(d, ci, cj)]; };
+        if (!in.avert[t] && i >= d.ilo && i <= d.ihi && j >= d.jlo && j <= d.jhi)
+            gap = (cell_on(i, j) || cell_on(i + 1, j) || cell_on(i, j + 1) || cell_on(i + 1, j + 1)) ? 1ull : 0ull;
     }
-    for (int off = WAVE / 2; off > 0; off >>= 1) bad += __shfl_down(bad, off, WAVE);
-    if (threadIdx.x % WAVE == 0 && bad) atomicAdd(count, bad);
+    for (int off = WAVE / 2; off > 0; off >>= 1) {
+        bent += __shfl_down(bent, off, WAVE);
+        gap += __shfl_down(gap, off, WAVE);
+    }
+    if (threadIdx.x % WAVE == 0 && bent) atomicAdd(count, bent);
+    if (threadIdx.x % WAVE == 0 && gap) atomicAdd(count + 1, gap);
 }
 
 // Horizontal values of one component on one level: x derivative at the two s

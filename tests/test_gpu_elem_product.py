@@ -63,3 +63,39 @@ def test_bent_grid_keeps_the_rows(require_gpu):
     assert np.array_equal(x0, x1)
     assert not np.array_equal(_iterate(prob, False, pcg.ALGO_CHRONGEAR)[1],
                               _iterate(prob, True, pcg.ALGO_CHRONGEAR)[1])
+
+
+def _masked(env, drop):
+    """Assembled stream with inactive vertices inside the ice: nnz, pairs, two solves, residual."""
+    os.environ.update(env)
+    try:
+        prob = synthetic.ice_stream(40, nz=5, seed=9)
+        s = BPSolver(prob)
+        for i, j in drop:
+            assert s.active_vertex[i, j] == 1
+            s.active_vertex[i, j] = 0
+        info = s.assemble(prob.uvel, prob.vvel)
+        out = [info["nnz"], info["asym_pairs"], *s.residual()]
+        for kw in (dict(), dict(precision=pcg.MIXED_FP32, inner_tol=1e-4, max_outer=20)):
+            s.sys.zero_x()
+            r = s.sys.solve(precond=2, tolerance=1e-9, maxiters=1000, raise_on_error=False, **kw)
+            assert r["status"] == 0 and r["err"] < 1e-9, r
+            out.append(np.stack(s.sys.get_x()))
+        s.sys.close()
+        return out
+    finally:
+        for k in env:
+            os.environ.pop(k, None)
+
+
+def test_inactive_vertices_inside_the_ice(require_gpu):
+    """Their rows are zero and their neighbours' rows are not, so neither the
+    element form nor half storage stands for that matrix: the full rows do,
+    and every row is counted.  One vertex in a wavefront's middle, one at a
+    tile's edge, two neighbours."""
+    drop = [(12, 17), (20, 9), (21, 9), (33, 30)]
+    out = _masked({}, drop)
+    ref = _masked({"CISMGPU_SPMV_FULL": "1", "CISMGPU_SYMCHECK": "full"}, drop)
+    assert out[:2] == ref[:2] and out[1] > 0
+    assert out[2] == pytest.approx(ref[2], rel=1e-12) and out[3] == pytest.approx(ref[3], rel=1e-12)
+    assert all(np.array_equal(a, b) for a, b in zip(out[4:], ref[4:]))
