@@ -50,7 +50,6 @@ struct Dims {
     long long vlen;                 // doubles per padded vector: (nz+2)*nvy*px
     long long nrows;                // padded owned rows: nz*nyo*nxp
     long long plane;                // nvy*px
-    int zw;                         // > 0: a product stores zero in the columns of the zeroing halo rule
 };
 
 // Columns that a halo rule of width w (rows and columns per side) zeroes.

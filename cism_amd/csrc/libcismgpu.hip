@@ -78,7 +78,6 @@ struct cismgpu_system {
     double* scal_buf = nullptr;
     double* scal_h = nullptr;      // pinned copy of the scalars, then the three words of a check (k_scalars)
     unsigned long long scal_seq = 0;
-    int zw = 0;                    // halo width that the next products store as zero (Dims::zw)
     TriPC tri;
     // assembly inputs on the device
     void* asm_buf = nullptr;
@@ -267,28 +266,26 @@ template <typename TA, typename TV, int MODE>
 void spmv(cismgpu_system* S, const TA* A, const TV* xu, const TV* xv, TV* yu, TV* yv, const TV* bu, const TV* bv,
           double* part) {
     const bool t = S->timing && S->ev_used + 2 <= (int)S->ev.size();
-    Dims d = S->d;
-    d.zw = S->zw;
+    const Dims& d = S->d;
     if (t) hipEventRecord(S->ev[S->ev_used], S->s);
     if (S->two_d)   // one level: only the kA = 0 plane of the rows is read
-        k_spmv_plane<TA, TV, MODE><<<spmv_blocks(S->d), 256, 0, S->s>>>(d, A, xu, xv, yu, yv, bu, bv, part);
+        k_spmv_plane<TA, TV, MODE><<<spmv_blocks(d), 256, 0, S->s>>>(d, A, xu, xv, yu, yv, bu, bv, part);
     else if constexpr (std::is_same<TA, double>::value) {
-        if (S->elem_use && MODE != 0)   // an assembled system in element form
-            k_spmv_elem<MODE == 0 ? 1 : MODE>
-                <<<dim3(elem_blocks(S->d), elem_parts(S->d) / elem_blocks(S->d)), WAVE * EL_J, 0, S->s>>>(
-                    S->d, S->asm_in, S->elemq, S->elem_bd, xu, xv, yu, yv, bu, bv, part, elem_split(S->d));
+        if (S->elem_use && (MODE == 1 || MODE == 2))   // an assembled system in element form
+            k_spmv_elem<MODE == 2 ? 2 : 1>
+                <<<dim3(elem_blocks(d), elem_parts(d) / elem_blocks(d)), WAVE * EL_J, 0, S->s>>>(
+                    d, S->asm_in, S->elemq, S->elem_bd, xu, xv, yu, yv, bu, bv, part, elem_split(d));
         else if (S->a64_sym && (const double*)A == S->A64)   // FP64 half (symmetric) storage
-            k_spmv_sym64<MODE><<<spmv_grid(S->d), 256, 0, S->s>>>(d, S->A64h, xu, xv, yu, yv, bu, bv, part,
-                                                                  level_split(S->d));
+            k_spmv_sym64<MODE><<<spmv_grid(d), 256, 0, S->s>>>(d, S->A64h, xu, xv, yu, yv, bu, bv, part,
+                                                               level_split(d));
         else
-            k_spmv<TA, TV, MODE><<<spmv_grid(S->d), 256, 0, S->s>>>(d, A, xu, xv, yu, yv, bu, bv, part,
-                                                                    level_split(S->d));
+            k_spmv<TA, TV, MODE><<<spmv_grid(d), 256, 0, S->s>>>(d, A, xu, xv, yu, yv, bu, bv, part, level_split(d));
     }
     else if (std::is_same<TA, float>::value && S->a32_sym)   // FP32 half (symmetric) storage
         spmv_sym32<MODE>(S, (const float*)A, (const float*)xu, (const float*)xv, (float*)yu, (float*)yv,
                          (const float*)bu, (const float*)bv, part);
     else   // FP32 / BF16 copies in the quad layout
-        k_spmv_q<TA, MODE><<<spmv_grid(S->d), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part, level_split(S->d));
+        k_spmv_q<TA, MODE><<<spmv_grid(d), 256, 0, S->s>>>(d, A, xu, xv, yu, yv, bu, bv, part, level_split(d));
     if (t) { hipEventRecord(S->ev[S->ev_used + 1], S->s); S->ev_used += 2; }
 }
 
@@ -709,9 +706,12 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
     const bool fold = !noop && d.bc == 3 && !rs && std::is_same<TA, double>::value && !S->elem_use;
     for (int iter = 2; iter <= maxiters; ++iter) {
         if (!z_ready) apply_precond<TV>(S, precond, ru, rv, zu, zv);
-        S->zw = fold ? 2 : 0;
-        spmv<TA, TV, 1>(S, A, zu, zv, Azu, Azv, nullptr, nullptr, S->partB);
-        S->zw = 0;
+        if constexpr (std::is_same<TA, double>::value) {
+            if (fold) spmv<TA, TV, 3>(S, A, zu, zv, Azu, Azv, nullptr, nullptr, S->partB);
+            else spmv<TA, TV, 1>(S, A, zu, zv, Azu, Azv, nullptr, nullptr, S->partB);
+        } else {
+            spmv<TA, TV, 1>(S, A, zu, zv, Azu, Azv, nullptr, nullptr, S->partB);
+        }
         if (rs) {
             rs_dot<TV>(S, 1, ru, zu, rv, zv);
             rs_dot<TV>(S, 2, Azu, zu, Azv, zv);

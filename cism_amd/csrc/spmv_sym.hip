@@ -578,10 +578,10 @@ __global__ __launch_bounds__(256) void k_spmv_sym64(Dims d, const double* __rest
                 acc = dd_add_d(acc, ru * ru);
                 acc = dd_add_d(acc, rv * rv);
             } else {
-                const bool zr = MODE == 1 && zero_halo(d, d.ilo + io, d.jlo + jo, d.zw);
+                const bool zr = MODE == 3 && zero_halo(d, d.ilo + io, d.jlo + jo, 2);
                 yu[ck] = zr ? 0.0 : su;
                 yv[ck] = zr ? 0.0 : sv;
-                if (MODE == 1) {
+                if (MODE == 1 || MODE == 3) {
                     const int slot = (k + 1) % 3;
                     acc = dd_add_d(acc, su * xs[0][slot][w + 1][lane + 1]);
                     acc = dd_add_d(acc, sv * xs[1][slot][w + 1][lane + 1]);

@@ -10,6 +10,7 @@
 #define FN(name) static decltype(&name) p_##name
 FN(cismgpu_system_create);
 FN(cismgpu_system_destroy);
+FN(cismgpu_system_set_matrix);
 FN(cismgpu_system_assemble_3d);
 FN(cismgpu_system_solve);
 FN(cismgpu_system_residual);
@@ -30,12 +31,12 @@ struct Ice {
     std::vector<int32_t> acell, avert, ocean;
     cismgpu_assembly_in in{};
 
-    Ice(int n, int nz) {
+    Ice(int n, int nz, int bc = 3) {
         g.nx = g.ny = n + 4;
         g.nz = nz;
         g.ilo = g.jlo = 3;
         g.ihi = g.jhi = n + 2;
-        g.global_bc = 3;
+        g.global_bc = bc;
         const int nv = g.nx - 1;
         vert.assign((size_t)nv * nv, 1.0);
         levels.resize(nz + 1);
@@ -103,6 +104,22 @@ static void failed_reassembly(bool copy_fails) {
     EXPECT(p_cismgpu_system_internal_stress(s.S, tau.data(), nullptr, nullptr, nullptr, nullptr, nullptr) == 0);
 }
 
+// The products test for the no-ice halo rule only where it zeroes owned
+// columns (rows given by the caller; mode 3).
+static void zero_store(int bc, bool expected) {
+    Ice s(8, 3, bc);
+    const size_t n = s.vert.size() * 3;
+    const std::vector<double> A(27 * n), b(n);
+    EXPECT(p_cismgpu_system_set_matrix(s.S, s.avert.data(), A.data(), A.data(), A.data(), A.data(), b.data(), b.data(),
+                                       0) == 0);
+    s.solve();
+    EXPECT(onhost::count("k_spmv_sym64ILi3E") == (expected ? 5 : 0));
+    EXPECT(onhost::count("k_spmv_sym64ILi1E") == (expected ? 1 : 6));
+    EXPECT(s.assemble() == 0);
+    s.solve();
+    EXPECT(onhost::count("Li3E") == 0);
+}
+
 int main(int argc, char** argv) {
     if (argc != 3) return 2;
     void* lib = dlopen(argv[1], RTLD_NOW);
@@ -110,6 +127,7 @@ int main(int argc, char** argv) {
 #define LOAD(name) p_##name = (decltype(p_##name))dlsym(lib, #name)
     LOAD(cismgpu_system_create);
     LOAD(cismgpu_system_destroy);
+    LOAD(cismgpu_system_set_matrix);
     LOAD(cismgpu_system_assemble_3d);
     LOAD(cismgpu_system_solve);
     LOAD(cismgpu_system_residual);
@@ -117,6 +135,8 @@ int main(int argc, char** argv) {
     const std::map<std::string, std::function<void()>> checks = {
         {"reassembly_out_of_memory", [] { failed_reassembly(false); }},
         {"reassembly_failed_copy", [] { failed_reassembly(true); }},
+        {"zero_store_no_ice", [] { zero_store(3, true); }},
+        {"zero_store_outflow", [] { zero_store(1, false); }},
     };
     const auto c = checks.find(argv[2]);
     if (c == checks.end()) { printf("no check %s\n", argv[2]); return 2; }

@@ -21,7 +21,7 @@ def host_checks(tmp_path_factory):
     return exe
 
 
-CHECKS = ["reassembly_out_of_memory", "reassembly_failed_copy"]
+CHECKS = ["reassembly_out_of_memory", "reassembly_failed_copy", "zero_store_no_ice", "zero_store_outflow"]
 
 
 @pytest.mark.parametrize("check", CHECKS)
