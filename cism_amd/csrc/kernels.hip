@@ -162,15 +162,17 @@ __device__ __forceinline__ float2 node_sum(F term) {
     return y;
 }
 
-// FP32 rows at 5 wavefronts per SIMD; BF16 rows are half the bytes and want the
-// loads of 3 (149 registers: 0.52 ms at 1024^2 x 11 against 0.71 ms at 5), and
-// sum in the order of storage, since no other kernel has to give their bits.
+// At least 3 wavefronts per SIMD: the loads a wavefront has in flight count for
+// more than wavefronts.  FP32 rows then take 149 registers and 983 us at
+// 1024^2 x 11, 240 us at 512^2 x 11, 98 us at 320^2 x 11 without a split (at 5,
+// 86 registers: 1042, 245 and 164 us).  BF16 rows take 119 registers and 520,
+// 132 and 41 us (2 wavefronts and 176 registers: 512, 128 and 41 us, but up to
+// 14 % more below 448 columns a side); they sum in the order of storage, since
+// no other kernel has to give their bits.
 template <typename TA, int MODE>
-__global__ __launch_bounds__(256, sizeof(TA) == 4 ? 5 : 3) void k_spmv_q(Dims d, const TA* __restrict__ A, const float* __restrict__ xu,
-                                                const float* __restrict__ xv, float* __restrict__ yu,
-                                                float* __restrict__ yv, const float* __restrict__ bu,
-                                                const float* __restrict__ bv, double* __restrict__ partials,
-                                                int kper) {
+__global__ __launch_bounds__(256, 3) void k_spmv_q(Dims d, const TA* __restrict__ A, const float* __restrict__ xu, const float* __restrict__ xv,
+              float* __restrict__ yu, float* __restrict__ yv, const float* __restrict__ bu,
+              const float* __restrict__ bv, double* __restrict__ partials, int kper) {
     const int nbx = d.nxp / WAVE;
     const int bx = blockIdx.x % nbx, by = blockIdx.x / nbx;
     const int k0 = blockIdx.y * kper, k1 = min(d.nz, k0 + kper);
