@@ -27,7 +27,7 @@ __device__ __forceinline__ int xcd_remap(int lin, int nblk) {
 // SpMV: one thread per owned vertex column (io, jo); loop over the kper levels
 // of its share (blockIdx.y).  On small grids a workgroup that walks all the
 // levels leaves most CUs idle and pays a memory latency per level, so the
-// columns are split (level_split, libcismgpu.hip).
+// columns are split (row_cut, libcismgpu.hip).
 // MODE 0: y = A x
 // MODE 1: y = A x, partial (y, x) over owned            (delta, eta2)
 // MODE 2: r = b - A x, partial (r, r) over owned        (convergence check)

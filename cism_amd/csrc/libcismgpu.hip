@@ -176,21 +176,38 @@ Dims make_dims(const cismgpu_grid* g) {
 }
 
 inline int spmv_blocks(const Dims& d) { return (d.nxp / WAVE) * ((d.nyo + 3) / 4); }
-// Levels per workgroup of the row products.  A workgroup that walks all nz
-// levels pays the latency of a level nz times; below 512 tiles (two per CU)
-// the levels are dealt to as many workgroups as fill the chip four deep.
-inline int level_split(const Dims& d) {
+enum RowForm { FULL_ROWS, HALF32, HALF64, ROWS16 };
+// Workgroups of a row product: tiles, and shares of kper levels of each.
+struct RowCut {
+    int tiles, shares, kper;
+    dim3 grid() const { return dim3(tiles, shares); }
+    int parts() const { return tiles * shares; }         // partial sums
+};
+// A workgroup that walks all nz levels pays the latency of a level nz times;
+// below 512 tiles (two per CU) the levels are dealt to as many workgroups as
+// fill the chip four deep.  Where a share would be one or two levels on more
+// than a tile per CU, FP64 half rows stage x too often for what they gain
+// (us split / whole: 320^2 x 5 55.5 / 49.6, 288^2 x 6 60.0 / 55.1, 256^2 x 8
+// 57.7 / 53.8, but 240^2 x 8 46 / 49 and 288^2 x 8 84 / 95); BF16 rows are
+// through a column so fast that it takes more levels (320^2 x 8 31.5 / 30.1,
+// 320^2 x 11 42.6 / 40.3, 320^2 x 15 75 / 78).
+inline RowCut row_cut(const Dims& d, RowForm f) {
     const int b = spmv_blocks(d);
-    if (b >= 512) return d.nz;
-    const int split = std::min(d.nz, (1024 + b - 1) / b);
-    return (d.nz + split - 1) / split;
+    const int split = b >= 512 ? 1 : std::min(d.nz, (1024 + b - 1) / b);
+    int kper = (d.nz + split - 1) / split;
+    if (f == HALF64 && ((kper == 2 && b >= 256) || (kper == 1 && b > 256))) kper = d.nz;
+    if (f == ROWS16 && b > 256 && d.nz <= 12) kper = d.nz;
+    return {b, (d.nz + kper - 1) / kper, kper};
 }
-inline int level_shares(const Dims& d) { return (d.nz + level_split(d) - 1) / level_split(d); }
-inline dim3 spmv_grid(const Dims& d) { return dim3(spmv_blocks(d), level_shares(d)); }
-// workgroups, and so partial sums, of the products
-inline int spmv_parts(const Dims& d) { return spmv_blocks(d) * level_shares(d); }
+template <typename TA>
+constexpr RowForm full_form() { return sizeof(TA) == 2 ? ROWS16 : FULL_ROWS; }
+inline RowCut cut64(const cismgpu_system* S) { return row_cut(S->d, S->a64_sym ? HALF64 : FULL_ROWS); }
 inline int spmv64_parts(const cismgpu_system* S) {
-    return S->elem_use ? elem_parts(S->d) : S->two_d ? spmv_blocks(S->d) : spmv_parts(S->d);
+    return S->elem_use ? elem_parts(S->d) : S->two_d ? spmv_blocks(S->d) : cut64(S).parts();
+}
+// the most partial sums that a product of this grid can leave
+inline int most_parts(const Dims& d) {
+    return std::max(std::max(row_cut(d, FULL_ROWS).parts(), row_cut(d, HALF64).parts()), row_cut(d, ROWS16).parts());
 }
 inline int col_blocks(const Dims& d) { return (int)nblocks((long long)d.nvx * d.nvy, 256); }
 inline int upd_blocks(const Dims& d) { return (int)nblocks((long long)d.nvx * d.nvy, UPD_COLS); }
@@ -250,7 +267,8 @@ void spmv_sym32(cismgpu_system* S, const float* A, const float* xu, const float*
         k_spmv_symj<MODE><<<dim3((d.nxp / WAVE) * c.nj, c.nk), WAVE * c.waves, symj_lds(c), S->s>>>(
             d, A, xu, xv, yu, yv, bu, bv, part, c.jper, c.kper);
     } else {
-        k_spmv_sym<float, MODE><<<spmv_grid(d), 256, 0, S->s>>>(d, A, xu, xv, yu, yv, bu, bv, part, level_split(d));
+        const RowCut c = row_cut(d, HALF32);
+        k_spmv_sym<float, MODE><<<c.grid(), 256, 0, S->s>>>(d, A, xu, xv, yu, yv, bu, bv, part, c.kper);
     }
 }
 
@@ -259,7 +277,8 @@ template <typename TA>
 int spmv32_parts(const cismgpu_system* S) {
     const Dims& d = S->d;
     if (S->two_d) return spmv_blocks(d);
-    return std::is_same<TA, float>::value && S->a32_sym && use_symj(d) ? symj_blocks(d) : spmv_parts(d);
+    if (std::is_same<TA, float>::value && S->a32_sym) return use_symj(d) ? symj_blocks(d) : row_cut(d, HALF32).parts();
+    return row_cut(d, full_form<TA>()).parts();
 }
 
 template <typename TA, typename TV, int MODE>
@@ -276,16 +295,18 @@ void spmv(cismgpu_system* S, const TA* A, const TV* xu, const TV* xv, TV* yu, TV
                 <<<dim3(elem_blocks(d), elem_parts(d) / elem_blocks(d)), WAVE * EL_J, 0, S->s>>>(
                     d, S->asm_in, S->elemq, S->elem_bd, xu, xv, yu, yv, bu, bv, part, elem_split(d));
         else if (S->a64_sym && (const double*)A == S->A64)   // FP64 half (symmetric) storage
-            k_spmv_sym64<MODE><<<spmv_grid(d), 256, 0, S->s>>>(d, S->A64h, xu, xv, yu, yv, bu, bv, part,
-                                                               level_split(d));
+            k_spmv_sym64<MODE><<<cut64(S).grid(), 256, 0, S->s>>>(d, S->A64h, xu, xv, yu, yv, bu, bv, part,
+                                                                  cut64(S).kper);
         else
-            k_spmv<TA, TV, MODE><<<spmv_grid(d), 256, 0, S->s>>>(d, A, xu, xv, yu, yv, bu, bv, part, level_split(d));
+            k_spmv<TA, TV, MODE><<<cut64(S).grid(), 256, 0, S->s>>>(d, A, xu, xv, yu, yv, bu, bv, part, cut64(S).kper);
     }
     else if (std::is_same<TA, float>::value && S->a32_sym)   // FP32 half (symmetric) storage
         spmv_sym32<MODE>(S, (const float*)A, (const float*)xu, (const float*)xv, (float*)yu, (float*)yv,
                          (const float*)bu, (const float*)bv, part);
-    else   // FP32 / BF16 copies in the quad layout
-        k_spmv_q<TA, MODE><<<spmv_grid(d), 256, 0, S->s>>>(d, A, xu, xv, yu, yv, bu, bv, part, level_split(d));
+    else {   // FP32 / BF16 copies in the quad layout
+        const RowCut c = row_cut(d, full_form<TA>());
+        k_spmv_q<TA, MODE><<<c.grid(), 256, 0, S->s>>>(d, A, xu, xv, yu, yv, bu, bv, part, c.kper);
+    }
     if (t) { hipEventRecord(S->ev[S->ev_used + 1], S->s); S->ev_used += 2; }
 }
 
@@ -1042,7 +1063,7 @@ static int32_t system_create(const cismgpu_grid* grid, bool two_d, cismgpu_syste
     if ((e = hipStreamCreateWithFlags(&S->s, hipStreamNonBlocking)) != hipSuccess) return fail(e, "stream");
     const long long n2 = (long long)d.nvx * d.nvy;
     const long long na = d.nrows * NCOEF;
-    const int nparts = std::max(std::max(spmv_parts(d), std::max(elem_parts(d), symj_blocks(d))), std::max(std::max(upd_blocks(d), flat_blocks(d)), dot_blocks<double>(d))) + 8;
+    const int nparts = std::max(std::max(most_parts(d), std::max(elem_parts(d), symj_blocks(d))), std::max(std::max(upd_blocks(d), flat_blocks(d)), dot_blocks<double>(d))) + 8;
     if ((e = hipMalloc(&S->active, n2)) != hipSuccess) return fail(e, "active");
     if ((e = hipMalloc(&S->A64, na * sizeof(double))) != hipSuccess) return fail(e, "A64");
     if ((e = hipMalloc(&S->M64, 8 * d.vlen * sizeof(double))) != hipSuccess) return fail(e, "M64");
@@ -1390,15 +1411,15 @@ int32_t cismgpu_system_bench_spmv(cismgpu_system* S, int32_t kind, int32_t nrep,
             else
                 k_spmv_plane<__hip_bfloat16, float, 1><<<spmv_blocks(d), 256, 0, S->s>>>(d, S->A16, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB);
         } else if (kind == 0 && S->a64_sym)
-            k_spmv_sym64<1><<<spmv_grid(d), 256, 0, S->s>>>(d, S->A64h, S->V(0), S->V(1), S->V(12), S->V(13), nullptr, nullptr, S->partB, level_split(d));
+            k_spmv_sym64<1><<<cut64(S).grid(), 256, 0, S->s>>>(d, S->A64h, S->V(0), S->V(1), S->V(12), S->V(13), nullptr, nullptr, S->partB, cut64(S).kper);
         else if (kind == 0)
-            k_spmv<double, double, 1><<<spmv_grid(d), 256, 0, S->s>>>(d, S->A64, S->V(0), S->V(1), S->V(12), S->V(13), nullptr, nullptr, S->partB, level_split(d));
+            k_spmv<double, double, 1><<<cut64(S).grid(), 256, 0, S->s>>>(d, S->A64, S->V(0), S->V(1), S->V(12), S->V(13), nullptr, nullptr, S->partB, cut64(S).kper);
         else if (kind == 1 && S->a32_sym)
             spmv_sym32<1>(S, S->A32, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB);
         else if (kind == 1)
-            k_spmv_q<float, 1><<<spmv_grid(d), 256, 0, S->s>>>(d, S->A32, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB, level_split(d));
+            k_spmv_q<float, 1><<<row_cut(d, FULL_ROWS).grid(), 256, 0, S->s>>>(d, S->A32, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB, row_cut(d, FULL_ROWS).kper);
         else
-            k_spmv_q<__hip_bfloat16, 1><<<spmv_grid(d), 256, 0, S->s>>>(d, S->A16, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB, level_split(d));
+            k_spmv_q<__hip_bfloat16, 1><<<row_cut(d, ROWS16).grid(), 256, 0, S->s>>>(d, S->A16, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB, row_cut(d, ROWS16).kper);
     };
     launch();   // warm-up
     CG_CHECK(hipEventRecord(e0, S->s));
@@ -2538,12 +2559,13 @@ extern "C" int32_t cismgpu_system_residual(cismgpu_system* S, double* ru, double
     { const int st_ = reset_scal(S); if (st_) return st_; }
     // r = b - A x over owned rows with partial (r,r); resid = -r on owned active rows
     S->elem_use = S->elem_ok && elem_form_wanted();
-    const int nsp = spmv64_parts(S);
+    const RowCut c = row_cut(d, FULL_ROWS);
+    const int nsp = S->elem_use || S->two_d ? spmv64_parts(S) : c.parts();
     if (S->elem_use || S->two_d)
         spmv<double, double, 2>(S, S->A64, S->V(0), S->V(1), r0, r1, S->V(2), S->V(3), S->partB);
     else
-        k_spmv<double, double, 2><<<spmv_grid(d), 256, 0, S->s>>>(d, S->A64, S->V(0), S->V(1), r0, r1, S->V(2), S->V(3),
-                                                                  S->partB, level_split(d));
+        k_spmv<double, double, 2><<<c.grid(), 256, 0, S->s>>>(d, S->A64, S->V(0), S->V(1), r0, r1, S->V(2), S->V(3),
+                                                              S->partB, c.kper);
     S->elem_use = false;
     if (S->repro) {
         rs_dot<double>(S, 3, r0, r0, r1, r1);

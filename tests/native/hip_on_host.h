@@ -20,6 +20,7 @@ namespace onhost {
 
 inline std::map<const void*, std::string> kernels;
 inline std::vector<std::string> launched;
+inline dim3 grid;                         // of the last launch
 inline std::function<void(const std::string&, void**)> on_launch;
 inline bool fail_malloc = false;          // hipMalloc fails
 inline bool fail_pinned = false;          // hipHostMalloc fails
@@ -67,9 +68,10 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t*
     *g = onhost::config.grid; *b = onhost::config.block; *lds = onhost::config.lds; *s = onhost::config.s;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t) {
+hipError_t hipLaunchKernel(const void* f, dim3 g, dim3, void** args, size_t, hipStream_t) {
     const std::string& name = onhost::kernels[f];
     onhost::launched.push_back(name);
+    onhost::grid = g;
     if (onhost::on_launch) onhost::on_launch(name, args);
     return hipSuccess;
 }

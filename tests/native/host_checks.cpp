@@ -76,6 +76,20 @@ struct Ice {
     }
 };
 
+// Scalars that keep a solve going: norms of one, a residual of a half.
+static void converging(const std::string& name, void** args) {
+    if (name.find("k_scalars") == std::string::npos) return;
+    double* scal = *(double**)args[7];
+    scal[6] = 1.0;      // L2 norm of the rhs
+    scal[8] = 0.5;      // relative residual of a check
+    scal[12] = 1.0;     // plain dot product
+    if (auto* mirror = *(unsigned long long**)args[9]) {
+        memcpy(mirror, &scal[8], 8);
+        mirror[1] = 4 * *(unsigned long long*)args[10];
+        mirror[2] = mirror[0] ^ mirror[1];
+    }
+}
+
 // A re-assembly that fails once its inputs are being replaced: the element
 // form of the products reads those inputs, so what follows keeps to the rows
 // of the old matrix, and the diagnostics, which have nothing else, refuse.
@@ -120,6 +134,34 @@ static void zero_store(int bc, bool expected) {
     EXPECT(onhost::count("Li3E") == 0);
 }
 
+// Levels that a workgroup of a product takes: whole columns where a share would
+// be too thin to pay, shares elsewhere; and every partial sum is summed.
+static void level_shares(int n, int nz, int half64, int rows16) {
+    Ice s(n, nz, 1);
+    const size_t m = s.vert.size() * nz;
+    std::vector<double> A(27 * m), b(m);
+    EXPECT(p_cismgpu_system_set_matrix(s.S, s.avert.data(), A.data(), A.data(), A.data(), A.data(), b.data(), b.data(),
+                                       0) == 0);
+    const int tiles = (n + 63) / 64 * ((n + 3) / 4);
+    int kper = 0, blocks = 0;
+    onhost::on_launch = [&](const std::string& name, void** args) {
+        if (name.find("k_spmv_sym64") != std::string::npos || name.find("k_spmv_q") != std::string::npos) {
+            kper = *(int*)args[9];
+            blocks = onhost::grid.x * onhost::grid.y;
+            EXPECT((int)onhost::grid.x == tiles && (int)onhost::grid.y == (nz + kper - 1) / kper);
+        }
+        // the stage of the first iteration takes the product's sums as its second
+        if (name.find("k_scalars") != std::string::npos && *(int*)args[0] == 2) EXPECT(*(int*)args[5] == blocks);
+        converging(name, args);
+    };
+    s.solve();
+    EXPECT(kper == half64);
+    kper = 0;
+    s.solve(CISMGPU_MIXED_BF16);
+    EXPECT(kper == rows16);
+    onhost::on_launch = nullptr;
+}
+
 int main(int argc, char** argv) {
     if (argc != 3) return 2;
     void* lib = dlopen(argv[1], RTLD_NOW);
@@ -135,6 +177,9 @@ int main(int argc, char** argv) {
     const std::map<std::string, std::function<void()>> checks = {
         {"reassembly_out_of_memory", [] { failed_reassembly(false); }},
         {"reassembly_failed_copy", [] { failed_reassembly(true); }},
+        {"level_shares_thin", [] { level_shares(320, 5, 5, 5); }},
+        {"level_shares_deep", [] { level_shares(270, 15, 4, 4); }},
+        {"level_shares_small", [] { level_shares(100, 4, 1, 1); }},
         {"zero_store_no_ice", [] { zero_store(3, true); }},
         {"zero_store_outflow", [] { zero_store(1, false); }},
     };
