@@ -259,6 +259,21 @@ static bool use_symj(const Dims& d) {
 }
 
 template <int MODE>
+void spmv_sym64(cismgpu_system* S, const double* xu, const double* xv, double* yu, double* yv, const double* bu,
+                const double* bv, double* part) {
+    const RowCut c = row_cut(S->d, HALF64);
+    const auto k = c.shares > 1 ? k_spmv_sym64<MODE, true> : k_spmv_sym64<MODE, false>;
+    k<<<c.grid(), 256, 0, S->s>>>(S->d, S->A64h, xu, xv, yu, yv, bu, bv, part, c.kper);
+}
+
+template <int MODE, typename TA>
+void spmv_q(cismgpu_system* S, const TA* A, const float* xu, const float* xv, float* yu, float* yv, const float* bu,
+            const float* bv, double* part) {
+    const RowCut c = row_cut(S->d, full_form<TA>());
+    k_spmv_q<TA, MODE><<<c.grid(), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part, c.kper);
+}
+
+template <int MODE>
 void spmv_sym32(cismgpu_system* S, const float* A, const float* xu, const float* xv, float* yu, float* yv,
                 const float* bu, const float* bv, double* part) {
     const Dims& d = S->d;
@@ -295,18 +310,15 @@ void spmv(cismgpu_system* S, const TA* A, const TV* xu, const TV* xv, TV* yu, TV
                 <<<dim3(elem_blocks(d), elem_parts(d) / elem_blocks(d)), WAVE * EL_J, 0, S->s>>>(
                     d, S->asm_in, S->elemq, S->elem_bd, xu, xv, yu, yv, bu, bv, part, elem_split(d));
         else if (S->a64_sym && (const double*)A == S->A64)   // FP64 half (symmetric) storage
-            k_spmv_sym64<MODE><<<cut64(S).grid(), 256, 0, S->s>>>(d, S->A64h, xu, xv, yu, yv, bu, bv, part,
-                                                                  cut64(S).kper);
+            spmv_sym64<MODE>(S, xu, xv, yu, yv, bu, bv, part);
         else
             k_spmv<TA, TV, MODE><<<cut64(S).grid(), 256, 0, S->s>>>(d, A, xu, xv, yu, yv, bu, bv, part, cut64(S).kper);
     }
     else if (std::is_same<TA, float>::value && S->a32_sym)   // FP32 half (symmetric) storage
         spmv_sym32<MODE>(S, (const float*)A, (const float*)xu, (const float*)xv, (float*)yu, (float*)yv,
                          (const float*)bu, (const float*)bv, part);
-    else {   // FP32 / BF16 copies in the quad layout
-        const RowCut c = row_cut(d, full_form<TA>());
-        k_spmv_q<TA, MODE><<<c.grid(), 256, 0, S->s>>>(d, A, xu, xv, yu, yv, bu, bv, part, c.kper);
-    }
+    else   // FP32 / BF16 copies in the quad layout
+        spmv_q<MODE, TA>(S, A, xu, xv, yu, yv, bu, bv, part);
     if (t) { hipEventRecord(S->ev[S->ev_used + 1], S->s); S->ev_used += 2; }
 }
 
@@ -1411,15 +1423,15 @@ int32_t cismgpu_system_bench_spmv(cismgpu_system* S, int32_t kind, int32_t nrep,
             else
                 k_spmv_plane<__hip_bfloat16, float, 1><<<spmv_blocks(d), 256, 0, S->s>>>(d, S->A16, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB);
         } else if (kind == 0 && S->a64_sym)
-            k_spmv_sym64<1><<<cut64(S).grid(), 256, 0, S->s>>>(d, S->A64h, S->V(0), S->V(1), S->V(12), S->V(13), nullptr, nullptr, S->partB, cut64(S).kper);
+            spmv_sym64<1>(S, S->V(0), S->V(1), S->V(12), S->V(13), nullptr, nullptr, S->partB);
         else if (kind == 0)
             k_spmv<double, double, 1><<<cut64(S).grid(), 256, 0, S->s>>>(d, S->A64, S->V(0), S->V(1), S->V(12), S->V(13), nullptr, nullptr, S->partB, cut64(S).kper);
         else if (kind == 1 && S->a32_sym)
             spmv_sym32<1>(S, S->A32, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB);
         else if (kind == 1)
-            k_spmv_q<float, 1><<<row_cut(d, FULL_ROWS).grid(), 256, 0, S->s>>>(d, S->A32, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB, row_cut(d, FULL_ROWS).kper);
+            spmv_q<1>(S, (const float*)S->A32, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB);
         else
-            k_spmv_q<__hip_bfloat16, 1><<<row_cut(d, ROWS16).grid(), 256, 0, S->s>>>(d, S->A16, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB, row_cut(d, ROWS16).kper);
+            spmv_q<1>(S, (const __hip_bfloat16*)S->A16, S->W(10), S->W(11), S->W(12), S->W(13), nullptr, nullptr, S->partB);
     };
     launch();   // warm-up
     CG_CHECK(hipEventRecord(e0, S->s));
