@@ -88,6 +88,9 @@ struct cismgpu_system {
     double* elem_bd = nullptr;   // basal friction term of the diagonal per vertex (element-form product)
     bool elem_ok = false;        // A64 equals the element form of asm_in, elemq and elem_bd
     bool elem_use = false;       // the running FP64 solve takes its products in element form
+    int elem_kper = 1;           // levels per workgroup of the element-form products (elem_split)
+    SjCut sj{};                  // shares of the marching FP32 product (symj_cut)
+    bool use_sj = false;         // the running solve takes it for half-stored FP32 rows
     bool raw_ready = false;      // stage holds the raw Auu/Avv of the current matrix
     bool saved_raw_ready = false;
     bool sym_exact = false;      // the assembled FP64 matrix is known to be exactly symmetric
@@ -203,7 +206,7 @@ template <typename TA>
 constexpr RowForm full_form() { return sizeof(TA) == 2 ? ROWS16 : FULL_ROWS; }
 inline RowCut cut64(const cismgpu_system* S) { return row_cut(S->d, S->a64_sym ? HALF64 : FULL_ROWS); }
 inline int spmv64_parts(const cismgpu_system* S) {
-    return S->elem_use ? elem_parts(S->d) : S->two_d ? spmv_blocks(S->d) : cut64(S).parts();
+    return S->elem_use ? elem_parts(S->d, S->elem_kper) : S->two_d ? spmv_blocks(S->d) : cut64(S).parts();
 }
 // the most partial sums that a product of this grid can leave
 inline int most_parts(const Dims& d) {
@@ -250,8 +253,9 @@ static bool elem_form_wanted() {
 // its ghost rows and its serial march from about 160 tiles on (193^2 x 11, 196
 // tiles: 24.8 against 31.1 us; 128^2 x 7, 64 tiles: 15.3 against 9.3 us).
 // CISMGPU_SPMV_SYMX=0: the re-reading kernel always; 1: the marching one
-// wherever it can run.
-static bool use_symj(const Dims& d) {
+// wherever it can run.  Read once per solve: its products and the counts of
+// their partial sums have to be those of one kernel.
+static bool symj_wanted(const Dims& d) {
     const char* e = getenv("CISMGPU_SPMV_SYMX");
     if (!symj_fits(d)) return false;
     if (e && (e[0] == '0' || e[0] == '1')) return e[0] == '1';
@@ -277,8 +281,8 @@ template <int MODE>
 void spmv_sym32(cismgpu_system* S, const float* A, const float* xu, const float* xv, float* yu, float* yv,
                 const float* bu, const float* bv, double* part) {
     const Dims& d = S->d;
-    if (use_symj(d)) {
-        const SjCut c = symj_cut(d);
+    if (S->use_sj) {
+        const SjCut& c = S->sj;
         k_spmv_symj<MODE><<<dim3((d.nxp / WAVE) * c.nj, c.nk), WAVE * c.waves, symj_lds(c), S->s>>>(
             d, A, xu, xv, yu, yv, bu, bv, part, c.jper, c.kper);
     } else {
@@ -292,7 +296,7 @@ template <typename TA>
 int spmv32_parts(const cismgpu_system* S) {
     const Dims& d = S->d;
     if (S->two_d) return spmv_blocks(d);
-    if (std::is_same<TA, float>::value && S->a32_sym) return use_symj(d) ? symj_blocks(d) : row_cut(d, HALF32).parts();
+    if (std::is_same<TA, float>::value && S->a32_sym) return S->use_sj ? symj_blocks(d, S->sj) : row_cut(d, HALF32).parts();
     return row_cut(d, full_form<TA>()).parts();
 }
 
@@ -307,8 +311,8 @@ void spmv(cismgpu_system* S, const TA* A, const TV* xu, const TV* xv, TV* yu, TV
     else if constexpr (std::is_same<TA, double>::value) {
         if (S->elem_use && (MODE == 1 || MODE == 2))   // an assembled system in element form
             k_spmv_elem<MODE == 2 ? 2 : 1>
-                <<<dim3(elem_blocks(d), elem_parts(d) / elem_blocks(d)), WAVE * EL_J, 0, S->s>>>(
-                    d, S->asm_in, S->elemq, S->elem_bd, xu, xv, yu, yv, bu, bv, part, elem_split(d));
+                <<<dim3(elem_blocks(d), elem_parts(d, S->elem_kper) / elem_blocks(d)), WAVE * EL_J, 0, S->s>>>(
+                    d, S->asm_in, S->elemq, S->elem_bd, xu, xv, yu, yv, bu, bv, part, S->elem_kper);
         else if (S->a64_sym && (const double*)A == S->A64)   // FP64 half (symmetric) storage
             spmv_sym64<MODE>(S, xu, xv, yu, yv, bu, bv, part);
         else
@@ -1075,7 +1079,9 @@ static int32_t system_create(const cismgpu_grid* grid, bool two_d, cismgpu_syste
     if ((e = hipStreamCreateWithFlags(&S->s, hipStreamNonBlocking)) != hipSuccess) return fail(e, "stream");
     const long long n2 = (long long)d.nvx * d.nvy;
     const long long na = d.nrows * NCOEF;
-    const int nparts = std::max(std::max(most_parts(d), std::max(elem_parts(d), symj_blocks(d))), std::max(std::max(upd_blocks(d), flat_blocks(d)), dot_blocks<double>(d))) + 8;
+    S->elem_kper = elem_split(d);
+    S->sj = symj_cut(d);
+    const int nparts = std::max(std::max(most_parts(d), std::max(elem_parts(d, S->elem_kper), symj_blocks(d, S->sj))), std::max(std::max(upd_blocks(d), flat_blocks(d)), dot_blocks<double>(d))) + 8;
     if ((e = hipMalloc(&S->active, n2)) != hipSuccess) return fail(e, "active");
     if ((e = hipMalloc(&S->A64, na * sizeof(double))) != hipSuccess) return fail(e, "A64");
     if ((e = hipMalloc(&S->M64, 8 * d.vlen * sizeof(double))) != hipSuccess) return fail(e, "M64");
@@ -1306,6 +1312,7 @@ int32_t cismgpu_system_solve(cismgpu_system* S, const cismgpu_solve_opts* o, cis
     o = &eff;
     memset(info, 0, sizeof(*info));
     info->err = NAN;
+    S->use_sj = symj_wanted(S->d);
     // per-assembly set-up, done by the first solve after an assembly or a
     // new matrix and cached until the next: the line-solve factors, the
     // exact-symmetry checks and the half-storage / low-precision copies
@@ -1402,6 +1409,7 @@ int32_t cismgpu_system_bench_spmv(cismgpu_system* S, int32_t kind, int32_t nrep,
     const Dims& d = S->d;
     const long long nodes = (long long)d.nz * d.nxo * d.nyo;
     int st = CISMGPU_OK;
+    S->use_sj = symj_wanted(d);
     if (kind > 0) {
         st = ensure_lowp(S, kind);
         if (st) return st;

@@ -51,7 +51,7 @@ inline int elem_split(const Dims& d) {
     }
     return best;
 }
-inline int elem_parts(const Dims& d) { return elem_blocks(d) * ((d.nz + elem_split(d) - 1) / elem_split(d)); }
+inline int elem_parts(const Dims& d, int kper) { return elem_blocks(d) * ((d.nz + kper - 1) / kper); }
 
 // What the short cuts of the assembly rest on, counted: count[0] the vertices
 // whose x varies along j or whose y varies along i (the element form needs a

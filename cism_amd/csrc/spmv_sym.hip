@@ -257,7 +257,7 @@ inline SjCut symj_cut(const Dims& d) {
     return c;
 }
 inline bool symj_fits(const Dims& d) { return (long long)d.nyo * d.nxp * NSLOT * 16 < (1LL << 31); }
-inline int symj_blocks(const Dims& d) { const SjCut c = symj_cut(d); return (d.nxp / WAVE) * c.nj * c.nk; }
+inline int symj_blocks(const Dims& d, const SjCut& c) { return (d.nxp / WAVE) * c.nj * c.nk; }
 inline size_t symj_lds(const SjCut& c) {
     return sizeof(float2) * (4 * (c.waves + 1) * (WAVE + 2) + 2 * 3 * c.waves * WAVE);
 }

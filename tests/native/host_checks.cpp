@@ -162,6 +162,26 @@ static void level_shares(int n, int nz, int half64, int rows16) {
     onhost::on_launch = nullptr;
 }
 
+// A solve keeps to the FP32 product it began with, whatever happens to the
+// environment meanwhile: the counts of the partial sums belong to it.
+static void one_product() {
+    Ice s(64, 3);
+    EXPECT(s.assemble() == 0);
+    for (const char* first : {"1", "0"}) {
+        int n = 0;
+        setenv("CISMGPU_SPMV_SYMX", first, 1);
+        onhost::on_launch = [&](const std::string& name, void** args) {
+            setenv("CISMGPU_SPMV_SYMX", ++n % 2 ? "0" : "1", 1);
+            converging(name, args);
+        };
+        s.solve(CISMGPU_MIXED_FP32, 12);
+        const int marching = onhost::count("k_spmv_symj"), rereading = onhost::count("k_spmv_symI");
+        EXPECT(first[0] == '1' ? marching > 4 && rereading == 0 : marching == 0 && rereading > 4);
+    }
+    unsetenv("CISMGPU_SPMV_SYMX");
+    onhost::on_launch = nullptr;
+}
+
 int main(int argc, char** argv) {
     if (argc != 3) return 2;
     void* lib = dlopen(argv[1], RTLD_NOW);
@@ -180,6 +200,7 @@ int main(int argc, char** argv) {
         {"level_shares_thin", [] { level_shares(320, 5, 5, 5); }},
         {"level_shares_deep", [] { level_shares(270, 15, 4, 4); }},
         {"level_shares_small", [] { level_shares(100, 4, 1, 1); }},
+        {"one_product_per_solve", one_product},
         {"zero_store_no_ice", [] { zero_store(3, true); }},
         {"zero_store_outflow", [] { zero_store(1, false); }},
     };
