@@ -10,11 +10,10 @@
 // 185 MB of velocities: down 18.7 -> 5.7 ms (33 GB/s), up 6.6 -> 4.9 ms; 9.6
 // and 8.9 ms with 512 KiB chunks and eight threads, which wait on the runtime's
 // locks; 4 MiB or eight threads of 2 MiB gain nothing.
+#include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <system_error>
 #include <thread>
-#include <vector>
 
 #include "cismgpu_internal.h"
 
@@ -24,7 +23,7 @@ constexpr size_t HC_CHUNK = 2 << 20;
 constexpr size_t HC_MIN = 6 << 20;
 constexpr int HC_THREADS = 4;
 
-struct HostSeg { void* host; const void* dev; size_t n; };   // dev is written to on the way up
+struct HostSeg { void* host; void* dev; size_t n; };
 
 // The pinned slots of one system (16 MiB), made by its first large copy.
 struct HostPipe {
@@ -47,24 +46,30 @@ struct HostPipe {
 };
 
 // Copies the segments down to host memory (or up from it), ordered on stream
-// s; returns when they are complete.
-int host_copy(HostPipe& P, hipStream_t s, const std::vector<HostSeg>& segs, bool down = true) {
-    size_t total = 0;
-    for (const HostSeg& g : segs) total += g.n;
-    if (total < HC_MIN) {
-        for (const HostSeg& g : segs)
-            CG_CHECK(down ? hipMemcpyAsync(g.host, g.dev, g.n, hipMemcpyDeviceToHost, s)
-                          : hipMemcpyAsync((void*)g.dev, g.host, g.n, hipMemcpyHostToDevice, s));
+// s; returns when they are complete.  Takes no memory from the heap, and does
+// with the runtime's copy where there is no pinned memory and with fewer
+// threads where one cannot be started, so it fails only if a copy does.
+int host_copy(HostPipe& P, hipStream_t s, const HostSeg* segs, int nseg, bool down = true) {
+    size_t total = 0, nchunk = 0;
+    for (int g = 0; g < nseg; ++g) {
+        total += segs[g].n;
+        nchunk += (segs[g].n + HC_CHUNK - 1) / HC_CHUNK;
+    }
+    if (total < HC_MIN || P.open() != CISMGPU_OK) {
+        (void)hipGetLastError();                  // the copy below is what counts
+        for (int g = 0; g < nseg; ++g)
+            CG_CHECK(down ? hipMemcpyAsync(segs[g].host, segs[g].dev, segs[g].n, hipMemcpyDeviceToHost, s)
+                          : hipMemcpyAsync(segs[g].dev, segs[g].host, segs[g].n, hipMemcpyHostToDevice, s));
         CG_CHECK(hipStreamSynchronize(s));
         return CISMGPU_OK;
     }
-    const int st = P.open();
-    if (st) return st;
     struct Chunk { char* host; char* dev; size_t n; };
-    std::vector<Chunk> chunks;
-    for (const HostSeg& g : segs)
-        for (size_t o = 0; o < g.n; o += HC_CHUNK)
-            chunks.push_back({(char*)g.host + o, (char*)g.dev + o, std::min(HC_CHUNK, g.n - o)});
+    auto chunk = [&](size_t c) {                  // the c-th of all segments
+        int g = 0;
+        for (size_t m; c >= (m = (segs[g].n + HC_CHUNK - 1) / HC_CHUNK); ++g) c -= m;
+        const size_t o = c * HC_CHUNK;
+        return Chunk{(char*)segs[g].host + o, (char*)segs[g].dev + o, std::min(HC_CHUNK, segs[g].n - o)};
+    };
     int dev = 0;
     CG_CHECK(hipGetDevice(&dev));
     std::atomic<int> err{hipSuccess};
@@ -79,17 +84,18 @@ int host_copy(HostPipe& P, hipStream_t s, const std::vector<HostSeg>& segs, bool
         hipEvent_t* ev = P.ev + 2 * t;
         // the link's part of this thread's c-th chunk
         auto link = [&](size_t c, int b) {
-            const Chunk& k = chunks[c];
+            const Chunk k = chunk(c);
             return keep(down ? hipMemcpyAsync(slot[b], k.dev, k.n, hipMemcpyDeviceToHost, s)
                              : hipMemcpyAsync(k.dev, slot[b], k.n, hipMemcpyHostToDevice, s)) &&
                    keep(hipEventRecord(ev[b], s));
         };
-        const size_t n = chunks.size();
+        const size_t n = nchunk;
         int b = 0;
         if (!down) {
             for (size_t c = t, m = 0; c < n; c += HC_THREADS, b ^= 1, ++m) {
                 if (m >= 2 && !keep(hipEventSynchronize(ev[b]))) return;
-                memcpy(slot[b], chunks[c].host, chunks[c].n);
+                const Chunk k = chunk(c);
+                memcpy(slot[b], k.host, k.n);
                 if (!link(c, b)) return;
             }
             return;
@@ -98,7 +104,8 @@ int host_copy(HostPipe& P, hipStream_t s, const std::vector<HostSeg>& segs, bool
         for (size_t c = t; c < n; c += HC_THREADS, b ^= 1) {
             if (c + HC_THREADS < n && !link(c + HC_THREADS, b ^ 1)) return;
             if (!keep(hipEventSynchronize(ev[b]))) return;
-            memcpy(chunks[c].host, slot[b], chunks[c].n);
+            const Chunk k = chunk(c);
+            memcpy(k.host, slot[b], k.n);
         }
     };
     std::thread th[HC_THREADS];
@@ -107,7 +114,7 @@ int host_copy(HostPipe& P, hipStream_t s, const std::vector<HostSeg>& segs, bool
         try {
             th[t] = std::thread(work, t);
             started[t] = true;
-        } catch (const std::system_error&) {      // no thread: its share is done below
+        } catch (...) {                           // no thread, or no memory for one: its share is done below
         }
     }
     work(0);

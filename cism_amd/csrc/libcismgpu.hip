@@ -1170,7 +1170,10 @@ static int set_matrix_impl(cismgpu_system* S, const int32_t* active_vertex, int 
     // Auv, Avu first through the staging pair, then Auu/Avv which stay staged
     auto stage2 = [&](const double* a, const double* b) -> int {
         const size_t n = nraw * sizeof(double);
-        if (!where_A) return host_copy(S->pipe, S->s, {{(void*)a, s0, n}, {(void*)b, s1, n}}, false);
+        if (!where_A) {
+            const HostSeg segs[2] = {{(void*)a, s0, n}, {(void*)b, s1, n}};
+            return host_copy(S->pipe, S->s, segs, 2, false);
+        }
         CG_CHECK(hipMemcpyAsync(s0, a, n, kind, S->s));
         CG_CHECK(hipMemcpyAsync(s1, b, n, kind, S->s));
         return CISMGPU_OK;
@@ -1278,7 +1281,8 @@ int32_t cismgpu_system_set_x(cismgpu_system* S, const double* xu, const double* 
     CG_CHECK(hipMemsetAsync(S->V(0), 0, 2 * d.vlen * sizeof(double), S->s));
     double* tmp2 = S->V(13);
     const size_t nb = nvec * sizeof(double);
-    const int st = host_copy(S->pipe, S->s, {{(void*)xu, tmp, nb}, {(void*)xv, tmp2, nb}}, false);
+    const HostSeg segs[2] = {{(void*)xu, tmp, nb}, {(void*)xv, tmp2, nb}};
+    const int st = host_copy(S->pipe, S->s, segs, 2, false);
     if (st) return st;
     k_vec_in<double, double><<<nblocks(nvec, 256), 256, 0, S->s>>>(d, tmp, S->V(0));
     k_vec_in<double, double><<<nblocks(nvec, 256), 256, 0, S->s>>>(d, tmp2, S->V(1));
@@ -1295,7 +1299,8 @@ int32_t cismgpu_system_get_x(cismgpu_system* S, double* xu, double* xv) {
     k_vec_out<double, double><<<nblocks(nvec, 256), 256, 0, S->s>>>(d, S->V(0), tmp);
     k_vec_out<double, double><<<nblocks(nvec, 256), 256, 0, S->s>>>(d, S->V(1), tmp2);
     const size_t nb = nvec * sizeof(double);
-    const int st = host_copy(S->pipe, S->s, {{xu, tmp, nb}, {xv, tmp2, nb}});
+    const HostSeg segs[2] = {{xu, tmp, nb}, {xv, tmp2, nb}};
+    const int st = host_copy(S->pipe, S->s, segs, 2);
     if (st) return st;
     CG_CHECK(hipMemsetAsync(tmp, 0, 2 * d.vlen * sizeof(double), S->s));
     return CISMGPU_OK;
@@ -2418,11 +2423,12 @@ extern "C" int32_t cismgpu_system_internal_stress(cismgpu_system* S, double* tau
     k_internal_stress<<<nblocks(nfl, 128), 128, 0, S->s>>>(d, S->asm_in, 2, 0, S->V(0), S->V(1), nullptr, tau);
     double* out[6] = {tau_xz, tau_yz, tau_xx, tau_yy, tau_xy, tau_eff};
     hipError_t e = hipGetLastError();
-    std::vector<HostSeg> segs;
+    HostSeg segs[6];
+    int ns = 0;
     for (int q = 0; q < 6; ++q)
-        if (out[q]) segs.push_back({out[q], tau + q * nfl, nfl * sizeof(double)});
+        if (out[q]) segs[ns++] = {out[q], tau + q * nfl, nfl * sizeof(double)};
     int st = CISMGPU_OK;
-    if (e == hipSuccess) st = host_copy(S->pipe, S->s, segs);
+    if (e == hipSuccess) st = host_copy(S->pipe, S->s, segs, ns);
     hipFree(tau);
     if (e != hipSuccess) {
         cismgpu_set_error("internal_stress: %s", hipGetErrorString(e));
@@ -2472,11 +2478,12 @@ extern "C" int32_t cismgpu_system_internal_stress_2d(cismgpu_system* S, const do
         e = hipGetLastError();
     }
     double* out[6] = {tau_xz, tau_yz, tau_xx, tau_yy, tau_xy, tau_eff};
-    std::vector<HostSeg> segs;
+    HostSeg segs[6];
+    int ns = 0;
     for (int q = 0; q < 6; ++q)
-        if (out[q]) segs.push_back({out[q], tau + q * nfl, nfl * sizeof(double)});
+        if (out[q]) segs[ns++] = {out[q], tau + q * nfl, nfl * sizeof(double)};
     int st = CISMGPU_OK;
-    if (e == hipSuccess) st = host_copy(S->pipe, S->s, segs);
+    if (e == hipSuccess) st = host_copy(S->pipe, S->s, segs, ns);
     hipFree(buf);
     if (e != hipSuccess) {
         cismgpu_set_error("internal_stress_2d: %s", hipGetErrorString(e));
@@ -2568,7 +2575,8 @@ extern "C" int32_t cismgpu_system_get_efvs(cismgpu_system* S, double* efvs) {
     if (!S || !S->efvs || !efvs) return CISMGPU_ERR_ARG;
     const int nzl = S->two_d ? S->nz_levels : S->d.nz;
     const long long nfl = (long long)(nzl - 1) * S->d.nx * S->d.ny;
-    return host_copy(S->pipe, S->s, {{efvs, S->efvs, nfl * sizeof(double)}});
+    const HostSeg seg{efvs, S->efvs, nfl * sizeof(double)};
+    return host_copy(S->pipe, S->s, &seg, 1);
 }
 
 extern "C" int32_t cismgpu_system_residual(cismgpu_system* S, double* ru, double* rv, double* L2, double* L2rel) {

@@ -7,12 +7,14 @@
 #pragma once
 #include <hip/hip_runtime_api.h>
 
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <functional>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -22,6 +24,7 @@ inline std::map<const void*, std::string> kernels;
 inline std::vector<std::string> launched;
 inline dim3 grid;                         // of the last launch
 inline std::function<void(const std::string&, void**)> on_launch;
+inline std::atomic<bool> heap_fails{false};   // operator new throws
 inline bool fail_malloc = false;          // hipMalloc fails
 inline bool fail_pinned = false;          // hipHostMalloc fails
 inline long long copies_to_failure = -1;  // >= 0: so many more copies succeed
@@ -50,6 +53,14 @@ inline thread_local Config config;
 
 }  // namespace onhost
 
+void* operator new(size_t n) {
+    void* p = onhost::heap_fails ? nullptr : malloc(n ? n : 1);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
+
 extern "C" {
 void** __hipRegisterFatBinary(const void*) {
     static void* h = nullptr;
@@ -70,7 +81,7 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t*
 }
 hipError_t hipLaunchKernel(const void* f, dim3 g, dim3, void** args, size_t, hipStream_t) {
     const std::string& name = onhost::kernels[f];
-    onhost::launched.push_back(name);
+    if (!onhost::heap_fails) onhost::launched.push_back(name);
     onhost::grid = g;
     if (onhost::on_launch) onhost::on_launch(name, args);
     return hipSuccess;

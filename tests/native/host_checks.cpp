@@ -14,6 +14,8 @@ FN(cismgpu_system_set_matrix);
 FN(cismgpu_system_assemble_3d);
 FN(cismgpu_system_solve);
 FN(cismgpu_system_residual);
+FN(cismgpu_system_set_x);
+FN(cismgpu_system_get_x);
 FN(cismgpu_system_internal_stress);
 
 static int bad = 0;
@@ -182,6 +184,34 @@ static void one_product() {
     onhost::on_launch = nullptr;
 }
 
+// Large copies in and out, in chunks by several threads: every value arrives,
+// also without heap or pinned memory, and a failing copy is reported.
+static void large_copies(bool no_heap, bool no_pinned) {
+    Ice s(210, 10);
+    const size_t n = s.vert.size() * 10;          // 3.6 MB each: a partial last chunk
+    std::vector<double> u(n), v(n), a(n), b(n);
+    for (size_t i = 0; i < n; ++i) { u[i] = (double)i; v[i] = -(double)i - 0.5; }
+    int in = 0, out = 0;
+    auto hook = [&](const std::string& name, void** args) {
+        if (name.find("k_vec_in") != std::string::npos)
+            EXPECT(memcmp(*(double**)args[1], in++ % 2 ? v.data() : u.data(), n * sizeof(double)) == 0);
+        if (name.find("k_vec_out") != std::string::npos)
+            memcpy(*(double**)args[2], out++ % 2 ? u.data() : v.data(), n * sizeof(double));
+    };
+    onhost::on_launch = hook;
+    onhost::fail_pinned = no_pinned;
+    onhost::heap_fails = no_heap;
+    const int st_in = p_cismgpu_system_set_x(s.S, u.data(), v.data());
+    const int st_out = p_cismgpu_system_get_x(s.S, a.data(), b.data());
+    onhost::heap_fails = false;
+    EXPECT(st_in == 0 && in == 2 && st_out == 0 && out == 2);
+    EXPECT(a == v && b == u);
+    onhost::copies_to_failure = 2;
+    EXPECT((p_cismgpu_system_get_x(s.S, a.data(), b.data()) != 0) == !no_pinned);   // two whole copies, or many chunks
+    onhost::copies_to_failure = -1;
+    onhost::on_launch = nullptr;
+}
+
 int main(int argc, char** argv) {
     if (argc != 3) return 2;
     void* lib = dlopen(argv[1], RTLD_NOW);
@@ -193,6 +223,8 @@ int main(int argc, char** argv) {
     LOAD(cismgpu_system_assemble_3d);
     LOAD(cismgpu_system_solve);
     LOAD(cismgpu_system_residual);
+    LOAD(cismgpu_system_set_x);
+    LOAD(cismgpu_system_get_x);
     LOAD(cismgpu_system_internal_stress);
     const std::map<std::string, std::function<void()>> checks = {
         {"reassembly_out_of_memory", [] { failed_reassembly(false); }},
@@ -201,6 +233,9 @@ int main(int argc, char** argv) {
         {"level_shares_deep", [] { level_shares(270, 15, 4, 4); }},
         {"level_shares_small", [] { level_shares(100, 4, 1, 1); }},
         {"one_product_per_solve", one_product},
+        {"large_copies", [] { large_copies(false, false); }},
+        {"large_copies_no_heap", [] { large_copies(true, false); }},
+        {"large_copies_no_pinned", [] { large_copies(false, true); }},
         {"zero_store_no_ice", [] { zero_store(3, true); }},
         {"zero_store_outflow", [] { zero_store(1, false); }},
     };

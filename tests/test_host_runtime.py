@@ -22,7 +22,8 @@ def host_checks(tmp_path_factory):
 
 
 CHECKS = ["reassembly_out_of_memory", "reassembly_failed_copy", "zero_store_no_ice", "zero_store_outflow",
-          "one_product_per_solve", "level_shares_thin", "level_shares_deep", "level_shares_small"]
+          "one_product_per_solve", "level_shares_thin", "level_shares_deep", "level_shares_small",
+          "large_copies", "large_copies_no_heap", "large_copies_no_pinned"]
 
 
 @pytest.mark.parametrize("check", CHECKS)
