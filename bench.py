@@ -31,6 +31,10 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBPS = 8000.0   # MI355X HBM3E, 8 TB/s
+# FP64 products: matrix values read per node (4 blocks of 27; 14 slots of 4; f at 8 points per element), and kernel
+COEF64 = {"full rows": 108, "half rows": 56, "element form": 8}
+KERNEL64 = {"full rows": "cg::k_spmv<double, double, 1>", "half rows": "cg::k_spmv_sym64<1, false>",
+            "element form": "cg::k_spmv_elem<1>"}
 
 
 def log(msg):
@@ -129,7 +133,7 @@ def main():
         t64.append(time.perf_counter() - tw)
         it64.append(r["niters"])
         sp64.append((r["spmv_ms"], r["spmv_count"]))
-        r64_kind = r["spmv_kind"]
+        form64 = s.fp64_product
         log(f"fp64 step {k}: {r['niters']} it, device {r['solve_ms']:.1f} ms, wall {t64[-1] * 1e3:.1f} ms")
     x64 = np.stack(s.get_x())
 
@@ -166,7 +170,7 @@ def main():
         with open(pmc_path) as f:
             traffic = json.load(f)["kernels"].get(kname, {}).get("traffic_bytes")
     sp64_ms = sum(a for a, _ in sp64) / max(sum(b for _, b in sp64), 1)
-    coef64 = 8 * 8 if r64_kind == 4 else 108 * 8       # FP64 element form (8 factors) or full rows
+    coef64 = COEF64[form64] * 8
     ach64 = nodes * (coef64 + 4 * 8) / (sp64_ms * 1e-3) / 1e9
 
     # ---- BF16-storage variant of the mixed solve (same system, same tolerance)
@@ -303,7 +307,7 @@ def main():
                  "iterations": it64, "rel_err_vs_oracle": errs.get("fp64"),
                  "spmv_avg_ms": round(sp64_ms, 4), "spmv_gbps": round(ach64, 1),
                  "spmv_frac": round(ach64 / HBM_PEAK_GBPS, 4),
-                 "spmv_storage": "half (symmetric)" if r64_kind == 4 else "full rows"},
+                 "spmv_storage": form64},
         "mixed": {"inner_iterations": itm, "outer_iterations": outm, "rel_err_vs_oracle": errs.get("mixed"),
                   "meets_1e-6": None if errs.get("mixed") is None else bool(errs["mixed"] <= 1e-6)},
         "speedup_mixed_vs_fp64": round(ms_fp64 / ms_mixed, 3),
@@ -543,15 +547,13 @@ def run_config2(args):
             its.append(r["niters"])
             sp.append((r["spmv_ms"], r["spmv_count"]))
         spavg = sum(a for a, _ in sp) / max(sum(b for _, b in sp), 1)
-        # element form of the assembled system: f at 8 points per element; full rows: 4 blocks of 27
-        coef = 8 * 8 if r["spmv_kind"] == 4 else 108 * 8
-        by = nodes * (coef + 4 * 8)
+        form64 = s.fp64_product
+        by = nodes * (COEF64[form64] * 8 + 4 * 8)
         out = dict(workload=f"synthetic ice stream {n}x{n}x{args.nz} seed 5, FP64 C-G, SIA preconditioner, tol 1e-8",
                    owned_nodes=nodes, ms_per_solve=round(1e3 * float(np.mean(ts)), 2),
                    solves_per_s=round(1.0 / float(np.mean(ts)), 4), iterations=its, err=r["err"],
                    setup_ms=round(setup_ms, 3),
-                   spmv_kernel=("cg::k_spmv_elem<1> (element form)" if r["spmv_kind"] == 4 else
-                                "cg::k_spmv<double, double, 1> (full rows)"),
+                   spmv_kernel=f"{KERNEL64[form64]} ({form64})",
                    spmv_avg_ms=round(spavg, 4), spmv_algorithmic_bytes=by,
                    spmv_gbps=round(by / (spavg * 1e-3) / 1e9, 1),
                    spmv_frac=round(by / (spavg * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4))

@@ -43,7 +43,7 @@ EXPORTS = (
     "cismgpu_residual_vector_3d_noalloc", "cismgpu_reprosum_calc",
     "cismgpu_system_calcbeta_setup", "cismgpu_system_calcbeta", "cismgpu_dropin_release",
     "cismgpu_system_internal_stress", "cismgpu_system_internal_stress_2d",
-    "cismgpu_system_basal_friction",
+    "cismgpu_system_basal_friction", "cismgpu_system_fp64_product",
 )
 
 
@@ -104,6 +104,8 @@ def _declare(L):
     L.cismgpu_system_matvec.argtypes = [vp, _D, _D]
     L.cismgpu_system_bench_spmv.argtypes = [vp, ctypes.c_int32, ctypes.c_int32, _D, _D]
     L.cismgpu_system_zero_x.argtypes = [vp]
+    L.cismgpu_system_fp64_product.argtypes = [vp]
+    L.cismgpu_system_fp64_product.restype = ctypes.c_int32
     L.cismgpu_residual_vector_3d_noalloc.argtypes = [_G] + [ctypes.c_void_p] * 13
     L.cismgpu_residual_vector_3d_noalloc.restype = ctypes.c_int32
     L.cismgpu_reprosum_calc.argtypes = [_D, ctypes.c_int64, ctypes.c_int32, _D]

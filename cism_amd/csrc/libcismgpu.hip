@@ -88,6 +88,7 @@ struct cismgpu_system {
     double* elem_bd = nullptr;   // basal friction term of the diagonal per vertex (element-form product)
     bool elem_ok = false;        // A64 equals the element form of asm_in, elemq and elem_bd
     bool elem_use = false;       // the running FP64 solve takes its products in element form
+    int form64 = -1;             // form of the products of the last FP64 solve (cismgpu_system_fp64_product)
     int elem_kper = 1;           // levels per workgroup of the element-form products (elem_split)
     SjCut sj{};                  // shares of the marching FP32 product (symj_cut)
     bool use_sj = false;         // the running solve takes it for half-stored FP32 rows
@@ -1372,7 +1373,8 @@ int32_t cismgpu_system_solve(cismgpu_system* S, const cismgpu_solve_opts* o, cis
         }
         info->err = err;
         info->niters = nit;
-        info->spmv_kind = (S->elem_use || S->a64_sym) ? 4 : 0;
+        S->form64 = S->elem_use ? 2 : S->a64_sym ? 1 : 0;
+        info->spmv_kind = S->form64 ? 4 : 0;
         S->elem_use = false;
     } else {
         st = mixed_solve(S, o, info);
@@ -1388,6 +1390,8 @@ int32_t cismgpu_system_solve(cismgpu_system* S, const cismgpu_solve_opts* o, cis
     S->timing = false;
     return st ? st : st2;
 }
+
+int32_t cismgpu_system_fp64_product(const cismgpu_system* S) { return S ? S->form64 : -1; }
 
 int32_t cismgpu_system_matvec(cismgpu_system* S, double* yu, double* yv) {
     if (!S || !S->have_matrix || !yu || !yv) return CISMGPU_ERR_ARG;

@@ -223,6 +223,11 @@ class System:
             raise _lib.CismGpuError(st, "system_solve")
         return res
 
+    @property
+    def fp64_product(self):
+        """Products of the last FP64 solve: "full rows", "half rows", "element form", or None before one."""
+        return {0: "full rows", 1: "half rows", 2: "element form"}.get(self._L.cismgpu_system_fp64_product(self._h))
+
     def bench_spmv(self, kind=0, nrep=20):
         ms = ctypes.c_double()
         by = ctypes.c_double()

@@ -204,6 +204,12 @@ int32_t cismgpu_system_get_x(cismgpu_system* sys, double* xu, double* xv);
 int32_t cismgpu_system_solve(cismgpu_system* sys, const cismgpu_solve_opts* opts,
                              cismgpu_solve_info* info);
 
+/* Form of the products of the last FP64 solve of this system (what
+ * info.spmv_kind 4 leaves open): 0 full rows, 1 half (symmetric) rows,
+ * 2 element form of an assembled system; -1 when there was none.  No
+ * reference counterpart. */
+int32_t cismgpu_system_fp64_product(const cismgpu_system* sys);
+
 /* y = A x with the resident matrix (FP64) on the resident x; host result. */
 int32_t cismgpu_system_matvec(cismgpu_system* sys, double* yu, double* yv);
 

@@ -1,6 +1,9 @@
 """FP64 solves of an assembled system take their products in element form; the
 rows (CISMGPU_SPMV_FULL=1) are the reference.  Sides around the 63 x 7 vertex
-tile, two to seventeen levels, periodic and ice-free rims, floating ice.
+tile, two to seventeen levels, an ice-free rim, floating ice.  Systems that
+the element form does not stand for keep the rows: prescribed velocities,
+periodic grids (the images of an element have other coordinates, and so other
+last bits), a bent grid, inactive vertices inside the ice, a restored matrix.
 
 Bar: the iterates after 7 Chronopoulos-Gear (6 standard) iterations.  Each
 product of either form sums a few hundred terms, so it is off by some 1e-14 of
@@ -25,6 +28,8 @@ PROBLEMS = {
     "yield_stream": lambda: synthetic.yield_stress_stream("raymond"),
     "marine": lambda: synthetic.marine_sheet(70, nz=7, seed=6),
 }
+# what a problem's FP64 products are read from when nothing forces the full rows
+ROWS = {"yield_stream": "half rows", "ismip_c": "half rows"}
 
 
 def _iterate(prob, full, algo, bend=False):
@@ -38,6 +43,8 @@ def _iterate(prob, full, algo, bend=False):
         r = s.sys.solve(algo=algo, precond=2, tolerance=0.0, maxiters=7 if algo == pcg.ALGO_CHRONGEAR else 6,
                         raise_on_error=False)
         x = np.stack(s.sys.get_x())
+        r["form"] = s.sys.fp64_product
+        r["L2"] = s.residual()[0]
         s.sys.close()
         return r, x
     finally:
@@ -50,11 +57,14 @@ def test_element_form_matches_rows(require_gpu, name, algo):
     prob = PROBLEMS[name]()
     r1, x1 = _iterate(prob, True, algo)
     r0, x0 = _iterate(prob, False, algo)
-    assert r1["spmv_kind"] == 0
+    assert r1["spmv_kind"] == 0 and r1["form"] == "full rows"
+    assert r0["form"] == ROWS.get(name, "element form")
     rel = np.linalg.norm(x0 - x1) / np.linalg.norm(x1)
     print(name, algo, f"rel {rel:.2e}, err {r0['err']:.6e} / {r1['err']:.6e}, same bits {np.array_equal(x0, x1)}")
     assert np.linalg.norm(x1) > 0 and rel < 1e-12
     assert r0["err"] == pytest.approx(r1["err"], rel=1e-10)
+    # one product each on iterates that differ by rel: |A dx| <= |A| |dx|, and |A||x| is within 1e4 of the residual here
+    assert r0["L2"] == pytest.approx(r1["L2"], rel=1e-8)
 
 
 def test_bent_grid_keeps_the_rows(require_gpu):
@@ -63,6 +73,57 @@ def test_bent_grid_keeps_the_rows(require_gpu):
     assert np.array_equal(x0, x1)
     assert not np.array_equal(_iterate(prob, False, pcg.ALGO_CHRONGEAR)[1],
                               _iterate(prob, True, pcg.ALGO_CHRONGEAR)[1])
+
+
+def test_restored_assembly_keeps_the_rows(require_gpu):
+    """The element form belongs to the last assembly: after a restore the
+    products are the rows of the restored matrix, with the bits of a run that
+    had no other form, until the next assembly."""
+    prob = PROBLEMS["stream20"]()
+    out = []
+    for full in (True, False):
+        os.environ["CISMGPU_SPMV_FULL"] = "1" if full else "0"
+        try:
+            s = BPSolver(prob)
+            s.assemble(prob.uvel, prob.vvel)
+            s.save_assembly()
+            s.assemble(2.0 * prob.uvel, 2.0 * prob.vvel)
+            s.restore_assembly()
+            s.sys.zero_x()
+            s.sys.solve(precond=2, tolerance=0.0, maxiters=7, raise_on_error=False)
+            assert s.sys.fp64_product == ("full rows" if full else "half rows")
+            out.append((np.stack(s.sys.get_x()), *s.residual()))
+            s.assemble(prob.uvel, prob.vvel)
+            s.sys.solve(precond=2, tolerance=0.0, maxiters=7, raise_on_error=False)
+            assert s.sys.fp64_product == ("full rows" if full else "element form")
+            s.sys.close()
+        finally:
+            os.environ.pop("CISMGPU_SPMV_FULL", None)
+    assert np.array_equal(out[0][0], out[1][0]) and out[0][1:] == out[1][1:]
+
+
+def test_accelerated_picard_matches_the_rows(require_gpu):
+    """Accelerated iterations that reject an extension solve a restored
+    matrix: the same decisions and iteration counts as on full rows, and the
+    same velocity to what the linear tolerance leaves (1e-8 relative residual,
+    condition number below 1e2 after the column preconditioner)."""
+    prob = PROBLEMS["stream63"]()
+    out = []
+    for full in (True, False):
+        os.environ["CISMGPU_SPMV_FULL"] = "1" if full else "0"
+        try:
+            s = BPSolver(prob)
+            out.append(s.picard(maxiter=8, resid_target=1e-12, linear_maxiters=2000, accelerate=True))
+            s.sys.close()
+        finally:
+            os.environ.pop("CISMGPU_SPMV_FULL", None)
+    a, b = out
+    assert a.alpha == b.alpha and a.linear_iters == b.linear_iters
+    rejected = sum(1 for q in range(1, len(a.alpha)) if a.alpha[q] == 1.0 and a.alpha[q - 1] > 1.0 and
+                   a.L2_norm[q + 1] >= a.L2_norm[q])
+    assert rejected > 0
+    u, v = np.stack([a.uvel, a.vvel]), np.stack([b.uvel, b.vvel])
+    assert np.linalg.norm(u - v) < 1e-6 * np.linalg.norm(u)
 
 
 def _masked(env, drop):
