@@ -1219,35 +1219,6 @@ __global__ void k_ir_update(Dims d, double* __restrict__ xu, double* __restrict_
 // ---------------------------------------------------------------------------
 // explicit instantiations used by the host drivers
 // ---------------------------------------------------------------------------
-#define INST_SPMV(TA, TV)                                                                                   \
-    template __global__ void k_spmv<TA, TV, 0>(Dims, const TA*, const TV*, const TV*, TV*, TV*, const TV*,   \
-                                               const TV*, double*, int);                                   \
-    template __global__ void k_spmv<TA, TV, 1>(Dims, const TA*, const TV*, const TV*, TV*, TV*, const TV*,   \
-                                               const TV*, double*, int);                                   \
-    template __global__ void k_spmv<TA, TV, 2>(Dims, const TA*, const TV*, const TV*, TV*, TV*, const TV*,   \
-                                               const TV*, double*, int);
-INST_SPMV(double, double)
-INST_SPMV(float, float)
-INST_SPMV(__hip_bfloat16, float)
-#define INST_SPMV_Q(TA)                                                                                      \
-    template __global__ void k_spmv_q<TA, 0>(Dims, const TA*, const float*, const float*, float*, float*,     \
-                                             const float*, const float*, double*, int);                     \
-    template __global__ void k_spmv_q<TA, 1>(Dims, const TA*, const float*, const float*, float*, float*,     \
-                                             const float*, const float*, double*, int);                     \
-    template __global__ void k_spmv_q<TA, 2>(Dims, const TA*, const float*, const float*, float*, float*,     \
-                                             const float*, const float*, double*, int);
-INST_SPMV_Q(float)
-INST_SPMV_Q(__hip_bfloat16)
-#define INST_SPMV_PLANE(TA, TV)                                                                              \
-    template __global__ void k_spmv_plane<TA, TV, 0>(Dims, const TA*, const TV*, const TV*, TV*, TV*,       \
-                                                     const TV*, const TV*, double*);                        \
-    template __global__ void k_spmv_plane<TA, TV, 1>(Dims, const TA*, const TV*, const TV*, TV*, TV*,       \
-                                                     const TV*, const TV*, double*);                        \
-    template __global__ void k_spmv_plane<TA, TV, 2>(Dims, const TA*, const TV*, const TV*, TV*, TV*,       \
-                                                     const TV*, const TV*, double*);
-INST_SPMV_PLANE(double, double)
-INST_SPMV_PLANE(float, float)
-INST_SPMV_PLANE(__hip_bfloat16, float)
 template __global__ void k_convert_quad<float>(long long, const double*, float*);
 template __global__ void k_convert_quad<__hip_bfloat16>(long long, const double*, __hip_bfloat16*);
 

@@ -678,12 +678,13 @@ int finish_timing(cismgpu_system* S, cismgpu_solve_info* info) {
 
 // Chronopoulos-Gear solve, reference semantics (pcg.F90:2632-3594), on
 // vectors of type TV with matrix storage TA.  x, r etc. point into the
-// system's vector pools.  With `given_r` the initial residual is supplied in
-// r (x = 0), as in the inner solve of iterative refinement, and the
+// system's vector pools.  FP32 vectors are the inner solve of iterative
+// refinement: the initial residual is supplied in r (given_r, x = 0), and the
 // convergence test uses the recurrence residual relative to ||r0||.
 template <typename TA, typename TV>
 int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const TV* bv, int precond, int ncheck,
-             double tol, int maxiters, bool given_r, double* err, int* niters, bool fuse_ok) {
+             double tol, int maxiters, double* err, int* niters, bool fuse_ok) {
+    constexpr bool given_r = !std::is_same<TV, double>::value;
     const Dims& d = S->d;
     TV *xu = v[0], *xv = v[1], *ru = v[2], *rv = v[3], *du = v[4], *dv = v[5], *qu = v[6], *qv = v[7];
     TV *zu = v[8], *zv = v[9], *Azu = v[10], *Azv = v[11];
@@ -693,7 +694,7 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
     const long long nv = d.vlen * sizeof(TV);
     // reprosum: the global sums of the FP64 solve are exact integer-vector
     // sums (the fused compensated partials are then not used)
-    const bool rs = S->repro && std::is_same<TV, double>::value && !given_r;
+    const bool rs = S->repro && !given_r;
     int st = reset_scal(S);
     if (st) return st;
     for (TV* p : {du, dv, zu, zv, qu, qv, Azu, Azv}) CG_CHECK(hipMemsetAsync(p, 0, nv, S->s));
@@ -707,7 +708,7 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
                                                        given_r ? rv : bv, S->partB);
         scalars(S, ST_BB, S->partB, dot_blocks<TV>(d), 2, nullptr, 0, 0);
     }
-    if (!given_r) {
+    if constexpr (!given_r) {
         CG_CHECK(hipMemsetAsync(ru, 0, nv, S->s));
         CG_CHECK(hipMemsetAsync(rv, 0, nv, S->s));
         halo<TV>(S, xu, xv, d.nz);
@@ -735,7 +736,7 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
     // themselves (their (A z, z) sums still take the values before it).
     const bool noop = zero_halo_is_noop(S);
     const bool fuse_scal = !rs && nub + nsp <= FUSE_MAX;   // the update sums the partials itself
-    const bool defer_x = given_r && fuse_ok && precond == 2 && std::is_same<TV, float>::value;
+    const bool defer_x = given_r && fuse_ok && precond == 2;
     bool late_x = false;
     auto finish_x = [&]() {
         if (late_x)
@@ -767,7 +768,7 @@ int cg_solve(cismgpu_system* S, const TA* A, TV* const* v, const TV* bu, const T
         late_x = xm == 1;
         z_ready = fuse;
         if (check) {
-            if (given_r) {
+            if constexpr (given_r) {
                 // recurrence residual (r,r) from the fused update's partials
                 if (!fuse) {
                     apply_precond<TV>(S, precond, ru, rv, zu, zv);
@@ -1017,10 +1018,10 @@ int mixed_solve(cismgpu_system* S, const cismgpu_solve_opts* o, cismgpu_solve_in
         const int budget = o->maxiters - inner_total;
         if (o->precision == CISMGPU_MIXED_BF16)
             st = cg_solve<__hip_bfloat16, float>(S, S->A16, w, nullptr, nullptr, o->precond, o->ncheck, inner_tol,
-                                                 budget, true, &ierr, &nit, true);
+                                                 budget, &ierr, &nit, true);
         else
             st = cg_solve<float, float>(S, S->A32, w, nullptr, nullptr, o->precond, o->ncheck, inner_tol,
-                                        budget, true, &ierr, &nit, true);
+                                        budget, &ierr, &nit, true);
         if (st) return st;
         inner_total += nit;
         k_ir_update<<<nblocks(d.nz * d.plane, 256), 256, 0, S->s>>>(d, xu, xv, w[0], w[1]);
@@ -1367,7 +1368,7 @@ int32_t cismgpu_system_solve(cismgpu_system* S, const cismgpu_solve_opts* o, cis
         if (o->algo == CISMGPU_ALGO_CHRONGEAR) {
             double* v[12] = {S->V(0), S->V(1), S->V(4), S->V(5), S->V(6), S->V(7), S->V(8), S->V(9), S->V(10), S->V(11), S->V(12), S->V(13)};
             st = cg_solve<double, double>(S, S->A64, v, S->V(2), S->V(3), o->precond, o->ncheck, o->tolerance,
-                                          o->maxiters, false, &err, &nit, true);
+                                          o->maxiters, &err, &nit, true);
         } else {
             st = std_solve(S, o->precond, o->ncheck, o->tolerance, o->maxiters, &err, &nit);
         }

@@ -115,8 +115,10 @@ __device__ __forceinline__ void plane_corners(const PlaneQ& p, double hx2, doubl
 
 // MODE 1: y = A x with the (y, x) partials; MODE 2: r = b - A x with the
 // (r, r) partials, as the row kernels.  bd: the basal friction term of the
-// diagonal at the bed, per vertex.  With the no-ice rule the rows of the last
-// two vertex rows and columns are zero, as k_matrix_noice_edge leaves them.
+// diagonal at the bed, per vertex.  The rows that the no-ice rule zeroes
+// (k_matrix_noice_edge) need no case of their own: where one was not zero
+// before, its neighbours still couple to it, the matrix is not symmetric and
+// its rows are the only form.
 template <int MODE>
 __global__ __launch_bounds__(WAVE * EL_J) void k_spmv_elem(Dims d, AsmDev in, const double* __restrict__ E,
                                                            const double* __restrict__ bd,
@@ -133,7 +135,6 @@ __global__ __launch_bounds__(WAVE * EL_J) void k_spmv_elem(Dims d, AsmDev in, co
     const int ci = d.ilo + bx * (WAVE - 1) + lane, cj = d.jlo + by * (EL_J - 1) + w;   // cell; its NE vertex is (ci, cj)
     const bool on = ci <= d.ihi + 1 && cj <= d.jhi + 1 && cell_in_range(d, in.nhalo, ci, cj) && in.acell[c2(d, ci, cj)];
     const bool out = lane < WAVE - 1 && w < EL_J - 1 && ci <= d.ihi && cj <= d.jhi;
-    const bool zero_row = d.bc == 3 && (ci >= d.nvx - 1 || cj >= d.nvy - 1);
     const double g = 0.57735026918962576451;
     double kq[4], zx[2], zy[2], tx[2], ty[2], hx2 = 0.0, hy2 = 0.0;
 #pragma unroll
@@ -188,7 +189,6 @@ __global__ __launch_bounds__(WAVE * EL_J) void k_spmv_elem(Dims d, AsmDev in, co
                 au = au + s * x0;
                 av = av + s * x1;
             }
-            if (zero_row) au = av = 0.0;
             if (MODE == 2) {
                 const double r0 = bu[c] - au, r1 = bv[c] - av;
                 yu[c] = r0;
