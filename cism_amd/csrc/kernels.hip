@@ -168,14 +168,16 @@ __device__ __forceinline__ float2 node_sum(F term) {
 // 86 registers: 1042, 245 and 164 us).  BF16 rows take 119 registers and 520,
 // 132 and 41 us (2 wavefronts and 176 registers: 512, 128 and 41 us, but up to
 // 14 % more below 448 columns a side); they sum in the order of storage, since
-// no other kernel has to give their bits.
-template <typename TA, int MODE>
+// no other kernel has to give their bits.  SPLIT false: whole columns, with
+// the first level and the share constants (BF16 111 registers, 288^2 x 11 34.2
+// for 35.4 us, 512^2 x 11 130.8 for 133.5).
+template <typename TA, int MODE, bool SPLIT>
 __global__ __launch_bounds__(256, 3) void k_spmv_q(Dims d, const TA* __restrict__ A, const float* __restrict__ xu, const float* __restrict__ xv,
               float* __restrict__ yu, float* __restrict__ yv, const float* __restrict__ bu,
               const float* __restrict__ bv, double* __restrict__ partials, int kper) {
     const int nbx = d.nxp / WAVE;
     const int bx = blockIdx.x % nbx, by = blockIdx.x / nbx;
-    const int k0 = blockIdx.y * kper, k1 = min(d.nz, k0 + kper);
+    const int k0 = SPLIT ? blockIdx.y * kper : 0, k1 = SPLIT ? min(d.nz, k0 + kper) : d.nz;
     const int lane = threadIdx.x % WAVE;
     const int io = bx * WAVE + lane;
     const int jo = by * 4 + threadIdx.x / WAVE;
@@ -247,7 +249,7 @@ __global__ __launch_bounds__(256, 3) void k_spmv_q(Dims d, const TA* __restrict_
         dd v[1] = {acc};
         block_reduce_dd<1, 256>(v);
         if (threadIdx.x == 0) {
-            const int lin = blockIdx.y * gridDim.x + blockIdx.x;
+            const int lin = SPLIT ? blockIdx.y * gridDim.x + blockIdx.x : blockIdx.x;
             partials[2 * lin + 0] = v[0].hi;
             partials[2 * lin + 1] = v[0].lo;
         }

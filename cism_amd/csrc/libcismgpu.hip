@@ -193,8 +193,8 @@ struct RowCut {
 // than a tile per CU, FP64 half rows stage x too often for what they gain
 // (us split / whole: 320^2 x 5 55.5 / 49.6, 288^2 x 6 60.0 / 55.1, 256^2 x 8
 // 57.7 / 53.8, but 240^2 x 8 46 / 49 and 288^2 x 8 84 / 95); BF16 rows are
-// through a column so fast that it takes more levels (320^2 x 8 31.5 / 30.1,
-// 320^2 x 11 42.6 / 40.3, 320^2 x 15 75 / 78).
+// through a column so fast that it takes more levels (320^2 x 8 31.5 / 29.6,
+// 320^2 x 11 42.6 / 40.8, 320^2 x 15 75 / 78).
 inline RowCut row_cut(const Dims& d, RowForm f) {
     const int b = spmv_blocks(d);
     const int split = b >= 512 ? 1 : std::min(d.nz, (1024 + b - 1) / b);
@@ -275,7 +275,15 @@ template <int MODE, typename TA>
 void spmv_q(cismgpu_system* S, const TA* A, const float* xu, const float* xv, float* yu, float* yv, const float* bu,
             const float* bv, double* part) {
     const RowCut c = row_cut(S->d, full_form<TA>());
-    k_spmv_q<TA, MODE><<<c.grid(), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part, c.kper);
+    // BF16 columns taken whole have their own instance, except on two to three
+    // tiles per CU (352^2 x 8 39.2 us as a single share, 42.0 whole; 448^2 x 8 83.5 and 81.6)
+    if constexpr (sizeof(TA) == 2) {
+        if (c.shares == 1 && (c.tiles < 512 || c.tiles >= 700)) {
+            k_spmv_q<TA, MODE, false><<<c.grid(), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part, c.kper);
+            return;
+        }
+    }
+    k_spmv_q<TA, MODE, true><<<c.grid(), 256, 0, S->s>>>(S->d, A, xu, xv, yu, yv, bu, bv, part, c.kper);
 }
 
 template <int MODE>
