@@ -122,7 +122,7 @@ def main():
         log(f"warmup mixed {w}: {r['niters']} inner it, {r['outer_iters']} outer, {r['solve_ms']:.1f} ms "
             f"(set-up {r['setup_ms']:.2f} ms)")
     setup["note"] = ("host wall time of the per-assembly set-up done by the first solve after an assembly "
-                     "(FP64: none, element form; mixed: symmetry check, FP64 half-storage and FP32 copies, preconditioner cast); "
+                     "(FP64: none, element form; mixed: FP32 copy and preconditioner cast); "
                      "cached and outside the timed solves below, paid once per Picard assembly")
 
     # ---- timed FP64 solves
@@ -164,7 +164,7 @@ def main():
     # HBM bytes per launch of the same kernel from the rocprofv3 FETCH_SIZE / WRITE_SIZE
     # passes of this workload, scaled by the counters' reading of a copy kernel of known size
     traffic = None
-    kname = {1: "cg::k_spmv_q<float, 1>", 2: "cg::k_spmv_q<__hip_bfloat16, 1>", 3: "cg::k_spmv_symj<1>"}[spmv_kind]
+    kname = {1: "cg::k_spmv_q<float, 1, true>", 2: "cg::k_spmv_q<__hip_bfloat16, 1, false>", 3: "cg::k_spmv_symj<1>"}[spmv_kind]
     pmc_path = os.path.join(ROOT, "profiles", "spmv_pmc_icestream1024.json")
     if args.n == 1024 and args.nz == 11 and os.path.exists(pmc_path):
         with open(pmc_path) as f:
@@ -192,7 +192,7 @@ def main():
         bf16 = dict(ms_per_solve=round(1e3 * float(np.mean(tb)), 2), solves_per_s=round(1.0 / float(np.mean(tb)), 4),
                     inner_iterations=itb, outer_iterations=r["outer_iters"], err=r["err"],
                     speedup_vs_fp64=round(ms_fp64 / (1e3 * float(np.mean(tb))), 3), setup_ms=round(bsetup, 3),
-                    spmv_kernel="cg::k_spmv_q<__hip_bfloat16, 1> (quad rows)", spmv_avg_ms=round(sbm, 4),
+                    spmv_kernel="cg::k_spmv_q<__hip_bfloat16, 1, false> (quad rows)", spmv_avg_ms=round(sbm, 4),
                     spmv_algorithmic_bytes=byb, spmv_gbps=round(byb / (sbm * 1e-3) / 1e9, 1),
                     spmv_frac=round(byb / (sbm * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4))
         log(f"bf16 storage: {bf16}")
